@@ -30,21 +30,46 @@
 
 namespace att {
 
-// Energy and its position gradient at one point: pot as pot_bead computes it
-// (bit-identical energy), plus d(E channel)/dp of the same voxel.
+// Energy and its position gradient at one point: the energy as pot_bead
+// computes it (trilin's weights and order of summation: the same bits), plus
+// d(E channel)/dp of the same voxel.  Bound by the L1's address processing:
+// the lanes of a wave read unrelated voxels, so every load instruction is 64
+// accesses.  From the energy octets a lookup is two 16 B loads of one 32 B
+// sector instead of eight 4 B loads strided over the 128 B line of all four
+// channels, and the grid a quarter of the footprint (100,000 poses: 1000/300
+// rigid 3.88 -> 3.53 ms, 3000/800 with 5 + 5 modes and parameter gradients 20.3 -> 19.3 ms).
+// energyOct is uniform: both levels of a grid have energy octets, or neither
+// (memory too short for them, or att_set_energy_octets).
 __device__ __forceinline__ void trilin_grad(const DGrid& g, float px, float py, float pz,
                                             unsigned ix, unsigned iy, unsigned iz, unsigned type,
-                                            float4& V, float3& dE) {
+                                            bool energyOct, float& E, float3& dE) {
     const float mnx = (float)(int)ix * g.dVox + g.lox;
     const float mny = (float)(int)iy * g.dVox + g.loy;
     const float mnz = (float)(int)iz * g.dVox + g.loz;
     const float ax = px - mnx, ay = py - mny, az = pz - mnz;
     const float bx = (mnx + g.dVox) - px, by = (mny + g.dVox) - py, bz = (mnz + g.dVox) - pz;
-    V = trilin(g, px, py, pz, ix, iy, iz, type);
     const size_t o = (((size_t)type * (g.nz - 1) + iz) * (g.ny - 1) + iy) * (g.nx - 1) + ix;
-    const float4* d = g.oct + 8 * o;  // same lines as trilin: cache hits
-    const float E0 = d[0].w, E1 = d[1].w, E2 = d[2].w, E3 = d[3].w;
-    const float E4 = d[4].w, E5 = d[5].w, E6 = d[6].w, E7 = d[7].w;
+    float4 lo, hi;
+    if (energyOct) {
+        lo = g.octE[2 * o];
+        hi = g.octE[2 * o + 1];
+    } else {
+        const float4* d = g.oct + 8 * o;
+        lo = make_float4(d[0].w, d[1].w, d[2].w, d[3].w);
+        hi = make_float4(d[4].w, d[5].w, d[6].w, d[7].w);
+    }
+    const float E0 = lo.x, E1 = lo.y, E2 = lo.z, E3 = lo.w;
+    const float E4 = hi.x, E5 = hi.y, E6 = hi.z, E7 = hi.w;
+    const float tmpMax_xy = bx * by, tmpMin_xy = ax * ay;
+    E = E0 * (tmpMax_xy * bz);
+    E = E + E1 * ((ax * by) * bz);
+    E = E + E2 * ((bx * ay) * bz);
+    E = E + E3 * (tmpMax_xy * az);
+    E = E + E4 * ((ax * by) * az);
+    E = E + E5 * ((bx * ay) * az);
+    E = E + E6 * (tmpMin_xy * bz);
+    E = E + E7 * (tmpMin_xy * az);
+    E = E * g.vol_inv;
     // corners: 0 (000) 1 (100) 2 (010) 3 (001) 4 (101) 5 (011) 6 (110) 7 (111)
     dE.x = ((E1 - E0) * (by * bz) + (E4 - E3) * (by * az) + (E6 - E2) * (ay * bz) +
             (E7 - E5) * (ay * az)) * g.vol_inv;
@@ -80,20 +105,20 @@ template <int PG>
 __device__ __forceinline__ float grid_adj_one(const DGrid& g, const DBasis& b, float px, float py,
                                               float pz, unsigned mtype, unsigned type, float charge,
                                               float3& G, const PGrad& pg, unsigned cellBase,
-                                              size_t rec) {
+                                              size_t rec, bool energyOct) {
     const unsigned ix = grid_index(px, g.lox, g.dVox_inv, g.nx);
     const unsigned iy = grid_index(py, g.loy, g.dVox_inv, g.ny);
     const unsigned iz = grid_index(pz, g.loz, g.dVox_inv, g.nz);
-    float4 pot;
+    float pot;
     float3 dE;
-    trilin_grad(g, px, py, pz, ix, iy, iz, mtype, pot, dE);
+    trilin_grad(g, px, py, pz, ix, iy, iz, mtype, energyOct, pot, dE);
     G = dE;
     if (fabsf(charge) > 0.001f) {
-        float4 el;
+        float el;
         float3 dEl;
-        trilin_grad(g, px, py, pz, ix, iy, iz, 0, el, dEl);
-        el.w = el.w * charge;
-        pot.w = pot.w + el.w;
+        trilin_grad(g, px, py, pz, ix, iy, iz, 0, energyOct, el, dEl);
+        el = el * charge;
+        pot = pot + el;
         G.x += charge * dEl.x; G.y += charge * dEl.y; G.z += charge * dEl.z;
     }
     // The grid of mapped type mtype holds the bead type's column of the pair
@@ -146,7 +171,7 @@ __device__ __forceinline__ float grid_adj_one(const DGrid& g, const DBasis& b, f
             }
         }
     }
-    return pot.w;
+    return pot;
 }
 
 // Grid term of one ligand bead: inner grid, else outer grid, else nothing
@@ -171,6 +196,7 @@ __device__ __forceinline__ float grid_adj(const DGrid& inner, const DGrid& outer
     }
     DGrid g{};
     g.oct = in ? inner.oct : outer.oct;
+    g.octE = in ? inner.octE : outer.octE;
     g.nx = in ? inner.nx : outer.nx;
     g.ny = in ? inner.ny : outer.ny;
     g.nz = in ? inner.nz : outer.nz;
@@ -183,7 +209,8 @@ __device__ __forceinline__ float grid_adj(const DGrid& inner, const DGrid& outer
     DBasis b{};
     b.oct = in ? bin.oct : bout.oct;
     b.nb = in ? bin.nb : bout.nb;
-    return grid_adj_one<PG>(g, b, px, py, pz, mtype, type, charge, G, pg, in ? 0u : pg.cellsIn, rec);
+    return grid_adj_one<PG>(g, b, px, py, pz, mtype, type, charge, G, pg, in ? 0u : pg.cellsIn,
+                            rec, inner.octE != nullptr);
 }
 
 // LJ derivatives with respect to (rc, ac, emin) at squared distance dr2.

@@ -22,8 +22,12 @@ constexpr unsigned kMaxTypesLDS = 32;  // pair table staged in LDS up to 32x32 t
 // for every (grid, iz, iy, ix) with i < n-1 the eight corner float4 values, in
 // the order trilinearInterpolation sums them (000, 100, 010, 001, 101, 011,
 // 110, 111), contiguous and 128-byte aligned — one cache line per lookup.
+// octE holds the energy channel of the same octets (8 floats, 32 bytes per
+// voxel) for the adjoint, which reads no other channel; null for grids without
+// a neighbour list (the adjoint never reads those) and where memory is short.
 struct DGrid {
     const float4* oct;
+    const float4* octE;
     unsigned nx, ny, nz, nxy, nvox, ngrids;
     float lox, loy, loz, hix, hiy, hiz;
     float dVox, dVox_inv, vol_inv;

@@ -87,6 +87,7 @@ struct att_ctx {
     void* d_ord = nullptr;  // spatial pose order: permutation + sort scratch
     size_t d_ord_cap = 0;
     bool poseOrder = true;
+    bool energyOctets = true;
     int modesWaves = 0;  // waves per pose of the flexible forward kernel, 0: by ligand size
     uint2* pairCounts = nullptr;  // att_debug_pair_counts: per-pose counts, capacity in poses
     size_t pairCountsCap = 0;
@@ -170,10 +171,16 @@ att_handle store(att_ctx* c, std::unique_ptr<Obj> o) {
     return h;
 }
 
+// Both levels of a grid have energy octets, or neither.
+void pair_octets(float4** inner, float4** outer) {
+    if (!*inner || !*outer) *inner = *outer = nullptr;
+}
+
 // Grid constants as IntrplGrid's constructor computes them (float arithmetic).
-DGrid make_dgrid(const att_grid_desc& g, const float4* oct) {
+DGrid make_dgrid(const att_grid_desc& g, const float4* oct, const float4* octE) {
     DGrid d{};
     d.oct = oct;
+    d.octE = octE;
     d.nx = g.nx; d.ny = g.ny; d.nz = g.nz;
     d.nxy = g.nx * g.ny;
     d.nvox = g.nx * g.ny * g.nz;
@@ -189,41 +196,48 @@ DGrid make_dgrid(const att_grid_desc& g, const float4* oct) {
     return d;
 }
 
-// Upload a [grid][z][y][x] float4 grid and expand it on the device into voxel
-// octets (8x the memory, one 128-byte line per lookup); the compact copy is
-// freed once expanded.
-att_status upload_octets(att_ctx* c, Obj* o, const att_grid_desc& g, float4** out) {
-    const size_t n = (size_t)g.nx * g.ny * g.nz * g.numGrids;
-    const size_t noct = (size_t)(g.nx - 1) * (g.ny - 1) * (g.nz - 1) * g.numGrids * 8;
-    void* tmp = nullptr;
+// Expands a device-resident point grid into voxel octets (owned by o) on the
+// context's stream; *octE (the energy octets) stays null unless `energy`, and
+// where memory is too short for them.
+att_status expand_octets(att_ctx* c, Obj* o, const att_grid_desc& g, const float4* d_points,
+                         bool energy, float4** out, float4** octE) {
+    const size_t cells = (size_t)(g.nx - 1) * (g.ny - 1) * (g.nz - 1) * g.numGrids;
     void* oct = nullptr;
-    ATT_HIP(c, hipMalloc(&oct, sizeof(float4) * noct));
+    void* e = nullptr;
+    ATT_HIP(c, hipMalloc(&oct, sizeof(float4) * 8 * cells));
     o->allocs.push_back(oct);
-    hipError_t e = hipMalloc(&tmp, sizeof(float4) * n);
-    if (e == hipSuccess) e = hipMemcpy(tmp, g.data, sizeof(float4) * n, hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = launch_octets(static_cast<const float4*>(tmp), static_cast<float4*>(oct), g.nx, g.ny,
-                          g.nz, g.numGrids, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (tmp) (void)hipFree(tmp);
-    if (e != hipSuccess)
-        return fail(c, e == hipErrorOutOfMemory ? ATT_ERR_NOMEM : ATT_ERR_HIP,
-                    std::string("grid upload: ") + hipGetErrorString(e));
+    if (energy && c->energyOctets) {
+        if (hipMalloc(&e, sizeof(float4) * 2 * cells) == hipSuccess) {
+            o->allocs.push_back(e);
+        } else {
+            (void)hipGetLastError();  // done without
+            e = nullptr;
+        }
+    }
+    ATT_HIP(c, launch_octets(d_points, static_cast<float4*>(oct), static_cast<float4*>(e), g.nx, g.ny,
+                             g.nz, g.numGrids, c->stream));
     *out = static_cast<float4*>(oct);
+    *octE = static_cast<float4*>(e);
     return ATT_OK;
 }
 
-// Expands a device-resident point grid into voxel octets (owned by o).
-att_status expand_octets(att_ctx* c, Obj* o, const att_grid_desc& g, const float4* d_points,
-                         float4** out) {
-    const size_t noct = (size_t)(g.nx - 1) * (g.ny - 1) * (g.nz - 1) * g.numGrids * 8;
-    void* oct = nullptr;
-    ATT_HIP(c, hipMalloc(&oct, sizeof(float4) * noct));
-    o->allocs.push_back(oct);
-    ATT_HIP(c, launch_octets(d_points, static_cast<float4*>(oct), g.nx, g.ny, g.nz, g.numGrids,
-                             c->stream));
-    *out = static_cast<float4*>(oct);
-    return ATT_OK;
+// Upload a [grid][z][y][x] float4 grid and expand it on the device into voxel
+// octets (8x the memory, one 128-byte line per lookup; 10x with the energy
+// octets); the compact copy is freed once expanded.
+att_status upload_octets(att_ctx* c, Obj* o, const att_grid_desc& g, bool energy, float4** out,
+                         float4** octE) {
+    const size_t n = (size_t)g.nx * g.ny * g.nz * g.numGrids;
+    void* tmp = nullptr;
+    ATT_HIP(c, hipMalloc(&tmp, sizeof(float4) * n));
+    hipError_t e = hipMemcpy(tmp, g.data, sizeof(float4) * n, hipMemcpyHostToDevice);
+    att_status st = ATT_OK;
+    if (e == hipSuccess) st = expand_octets(c, o, g, static_cast<const float4*>(tmp), energy, out, octE);
+    if (e == hipSuccess && st == ATT_OK) e = hipStreamSynchronize(c->stream);
+    (void)hipFree(tmp);
+    if (e != hipSuccess)
+        return fail(c, e == hipErrorOutOfMemory ? ATT_ERR_NOMEM : ATT_ERR_HIP,
+                    std::string("grid upload: ") + hipGetErrorString(e));
+    return st;
 }
 
 // Neighbour-list constants of a grid whose desc/list are already on the
@@ -322,6 +336,12 @@ const char* att_build_info(void) {
 att_status att_set_pose_order(att_ctx* c, int enabled) {
     if (!c) return ATT_ERR_INVALID;
     c->poseOrder = enabled != 0;
+    return ATT_OK;
+}
+
+att_status att_set_energy_octets(att_ctx* c, int enabled) {
+    if (!c) return ATT_ERR_INVALID;
+    c->energyOctets = enabled != 0;
     return ATT_OK;
 }
 
@@ -463,11 +483,12 @@ att_status att_upload_grid(att_ctx* c, const att_grid_desc* inner, const att_gri
     if (inner->numGrids != outer->numGrids)
         return fail(c, ATT_ERR_INVALID, "inner and outer grids differ in the number of types");
     auto o = std::make_unique<GridObj>();
-    float4 *din, *dout;
-    if ((st = upload_octets(c, o.get(), *inner, &din)) != ATT_OK) return st;
-    if ((st = upload_octets(c, o.get(), *outer, &dout)) != ATT_OK) return st;
-    o->inner = make_dgrid(*inner, din);
-    o->outer = make_dgrid(*outer, dout);
+    float4 *din, *dout, *ein, *eout;
+    if ((st = upload_octets(c, o.get(), *inner, nl != nullptr, &din, &ein)) != ATT_OK) return st;
+    if ((st = upload_octets(c, o.get(), *outer, nl != nullptr, &dout, &eout)) != ATT_OK) return st;
+    pair_octets(&ein, &eout);
+    o->inner = make_dgrid(*inner, din, ein);
+    o->outer = make_dgrid(*outer, dout, eout);
     if (nl) {
         if (!nl->desc) return fail(c, ATT_ERR_INVALID, "neighbour grid descriptors missing");
         if (nl->nx < 1 || nl->ny < 1 || nl->nz < 1) return fail(c, ATT_ERR_INVALID, "empty neighbour grid");
@@ -2007,18 +2028,19 @@ att_status att_build_grid(att_ctx* c, const att_protein_desc* body, const att_pa
     if ((st = gen_prepare(c, body, table, numTypes, srcIsLigand, plateau, in)) != ATT_OK) return st;
     auto o = std::make_unique<GridObj>();
     const att_grid_geom* geoms[2] = {inner, outer};
-    float4* oct[2];
+    float4 *oct[2], *octE[2];
     for (int k = 0; k < 2; ++k) {
         const att_grid_desc gd = grid_of(*geoms[k], numTypes + 1);
         Tmp tmp;
         float4* d;
         ATT_HIP(c, tmp.alloc(&d, (size_t)gd.nx * gd.ny * gd.nz * gd.numGrids));
         if ((st = gen_grid(c, in, *geoms[k], numTypes, potShape, dielec, ffelec, d)) != ATT_OK) return st;
-        if ((st = expand_octets(c, o.get(), gd, d, &oct[k])) != ATT_OK) return st;
+        if ((st = expand_octets(c, o.get(), gd, d, neighbourdis > 0.f, &oct[k], &octE[k])) != ATT_OK) return st;
         ATT_HIP(c, hipStreamSynchronize(c->stream));
     }
-    o->inner = make_dgrid(grid_of(*inner, numTypes + 1), oct[0]);
-    o->outer = make_dgrid(grid_of(*outer, numTypes + 1), oct[1]);
+    pair_octets(&octE[0], &octE[1]);
+    o->inner = make_dgrid(grid_of(*inner, numTypes + 1), oct[0], octE[0]);
+    o->outer = make_dgrid(grid_of(*outer, numTypes + 1), oct[1], octE[1]);
     if (neighbourdis > 0.f) {
         Obj* owner = o.get();
         auto alloc = [&](void** p, size_t bytes) {

@@ -486,9 +486,11 @@ __global__ void k_debug_plateau_ratio(float P2, unsigned n, float* ratio) {
     if (i < n) ratio[i] = plateau_ratio(i, P2);
 }
 
-// Expands a [grid][z][y][x] float4 grid into voxel octets (see DGrid).
+// Expands a [grid][z][y][x] float4 grid into voxel octets and, with octE, their
+// energy channel (see DGrid).
 __global__ __launch_bounds__(256) void k_octets(const float4* __restrict__ g,
-                                                float4* __restrict__ oct, unsigned nx,
+                                                float4* __restrict__ oct,
+                                                float4* __restrict__ octE, unsigned nx,
                                                 unsigned ny, unsigned nz, unsigned ngrids) {
     const size_t nvo = (size_t)(nx - 1) * (ny - 1) * (nz - 1);
     const size_t total = nvo * ngrids;
@@ -510,6 +512,10 @@ __global__ __launch_bounds__(256) void k_octets(const float4* __restrict__ g,
         d[5] = b[nxy + nx];
         d[6] = b[nx + 1];
         d[7] = b[nxy + nx + 1];
+        if (octE) {
+            octE[2 * o] = make_float4(b[0].w, b[1].w, b[nx].w, b[nxy].w);
+            octE[2 * o + 1] = make_float4(b[nxy + 1].w, b[nxy + nx].w, b[nx + 1].w, b[nxy + nx + 1].w);
+        }
     }
 }
 
@@ -522,12 +528,12 @@ __global__ __launch_bounds__(256) void k_copy(float4* __restrict__ dst,
 
 // ------------------------------------------------------------------ launchers
 
-hipError_t launch_octets(const float4* grid, float4* oct, unsigned nx, unsigned ny, unsigned nz,
-                         unsigned ngrids, hipStream_t s) {
+hipError_t launch_octets(const float4* grid, float4* oct, float4* octE, unsigned nx, unsigned ny,
+                         unsigned nz, unsigned ngrids, hipStream_t s) {
     const size_t total = (size_t)(nx - 1) * (ny - 1) * (nz - 1) * ngrids;
     const size_t blocks = std::min<size_t>((total + 255) / 256, 256 * 256);
-    hipLaunchKernelGGL(k_octets, dim3((unsigned)blocks), dim3(256), 0, s, grid, oct, nx, ny, nz,
-                       ngrids);
+    hipLaunchKernelGGL(k_octets, dim3((unsigned)blocks), dim3(256), 0, s, grid, oct, octE, nx, ny,
+                       nz, ngrids);
     return hipGetLastError();
 }
 

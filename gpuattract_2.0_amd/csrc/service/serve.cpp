@@ -58,6 +58,8 @@ struct Receptor {
     att_grid_geom inner{}, outer{};
     float plateau = 0.f, nd = 0.f;
     size_t bytes = 0;
+    size_t energyBytes = 0;  // of the grids' energy octets: held when memory allows
+    bool energy = false;     // and held now
     att_handle hProt = 0, hGrid = 0;
     bool resident = false;
     int refs = 0;
@@ -113,6 +115,11 @@ size_t grid_bytes(const as::GridUnionData::Grid& g) {
     const size_t points = (size_t)g.nx * g.ny * g.nz;
     // voxel octets plus the point grid they are expanded from
     return g.numGrids * (cells * 128 + points * 16);
+}
+
+// The energy octets of one level of a grid.
+size_t energy_bytes(size_t nx, size_t ny, size_t nz, size_t numGrids) {
+    return 32 * numGrids * (nx - 1) * (ny - 1) * (nz - 1);
 }
 
 size_t protein_bytes(const as::ProteinData& p) {
@@ -259,7 +266,7 @@ bool att_server::evict_for(size_t need, const Job* j) {
             att_release(ctx, r.hProt);
             r.hGrid = r.hProt = 0;
             r.resident = false;
-            used -= r.bytes;
+            used -= r.bytes + (r.energy ? r.energyBytes : 0);
         } else {
             Ligand& l = *ligands[best];
             att_release(ctx, l.h);
@@ -301,6 +308,9 @@ bool att_server::admit(Job* j) {
         }
         queue.erase(std::find(queue.begin(), queue.end(), j));
         j->admitSeq = ++admitted;
+        // The energy octets only make the scoring faster: no job waits, and
+        // nothing is evicted, for their memory.
+        if (!r->resident) r->energy = used + need + r->energyBytes <= budget;
         used += j->bytes;  // receptor and ligand bytes are added on upload
         r->refs++;
         l->refs++;
@@ -317,6 +327,7 @@ bool att_server::admit(Job* j) {
         const att_protein_desc pd = r->prot.desc();
         if (att_upload_protein(ctx, &pd, &r->hProt) != ATT_OK) return bad("receptor upload");
         att_status gs;
+        att_set_energy_octets(ctx, r->energy ? 1 : 0);
         if (r->fromBody) {
             gs = att_build_grid(ctx, &pd, p->table.data(), p->T, p->shape, p->dielec, p->ffelec,
                                 r->plateau, 0, &r->inner, &r->outer, r->nd, &r->hGrid);
@@ -332,7 +343,7 @@ bool att_server::admit(Job* j) {
         }
         r->resident = true;
         std::lock_guard<std::mutex> g(m);
-        used += r->bytes;
+        used += r->bytes + (r->energy ? r->energyBytes : 0);
     }
     if (!l->resident) {
         const att_protein_desc pd = l->prot.desc();
@@ -556,6 +567,8 @@ att_status att_server_add_receptor(att_server* s, const att_protein_desc* rec,
     g.desc.assign(nl->desc, nl->desc + 2 * (size_t)nl->nx * nl->ny * nl->nz);
     if (nl->numEl) g.list.assign(nl->list, nl->list + nl->numEl);
     r->bytes = receptor_bytes(*r);
+    for (const auto* g : {&r->grid.inner, &r->grid.outer})
+        r->energyBytes += energy_bytes(g->nx, g->ny, g->nz, g->numGrids);
     std::lock_guard<std::mutex> lk(s->m);
     *id = s->nextId++;
     s->receptors[*id] = std::move(r);
@@ -581,6 +594,8 @@ att_status att_server_add_receptor_body(att_server* s, const att_protein_desc* r
     auto pit = s->params.find(params);
     if (pit == s->params.end()) return set_err(ATT_ERR_HANDLE, "unknown table id");
     r->bytes = body_receptor_bytes(*r, pit->second->T);
+    for (const auto* g : {&r->inner, &r->outer})
+        r->energyBytes += energy_bytes(g->nx, g->ny, g->nz, pit->second->T + 1);
     *id = s->nextId++;
     s->receptors[*id] = std::move(r);
     return ATT_OK;

@@ -121,6 +121,7 @@ def lib():
         L = C.CDLL(LIBPATH)
         L.att_ctx_create.argtypes = [C.c_int, C.POINTER(P)]
         L.att_set_pose_order.argtypes = [P, C.c_int]
+        L.att_set_energy_octets.argtypes = [P, C.c_int]
         L.att_set_modes_waves.argtypes = [P, C.c_int]
         L.att_debug_pair_counts.argtypes = [P, P, C.c_size_t]
         L.att_ctx_destroy.argtypes = [P]
@@ -284,6 +285,10 @@ class Context:
     def set_pose_order(self, enabled):
         """Spatial pose order of the single-pair adjoint (default on)."""
         self._chk(self.L.att_set_pose_order(self.h, 1 if enabled else 0))
+
+    def set_energy_octets(self, enabled):
+        """Energy octets for the grids uploaded or built from now on (default on)."""
+        self._chk(self.L.att_set_energy_octets(self.h, 1 if enabled else 0))
 
     def pair_counts(self, fn, n):
         """Per-pose {listed neighbours walked, pairs inside the plateau} of the
