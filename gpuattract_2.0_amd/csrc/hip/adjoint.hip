@@ -225,7 +225,9 @@ __device__ __forceinline__ void lj_dparam(float dr2, float dr2_inv, const att_pa
 }
 
 // The neighbour-list pairs of one ligand bead at p (charge q, type lt) over
-// its list d = {numEl, idx}, in list order:
+// its list d = {numEl, idx} (numEl > 0), by the four lanes of a quad (s = lane
+// in the quad): each step takes four consecutive list entries, one per lane,
+// and the four pairs' terms are then added in list order on every lane:
 //  eAcc  the pair energies folded as NLPotForce folds them (+LJ(r), -LJ(P),
 //        +C(r), -C(P), model/neighborlist.h:66-158): the reference's bits;
 //  gAcc  the sum of the pair forces (LJ and Coulomb at r; the plateau terms
@@ -233,78 +235,105 @@ __device__ __forceinline__ void lj_dparam(float dr2, float dr2_inv, const att_pa
 //  gR    += force . (receptor mode vector) per pair (dE/d receptor amplitude
 //        through the receptor's deformation);
 //  the parameter derivatives into this wave's LDS slice.
-// Receptor beads are deformed from their padded mode row (one cache line).
+// A pair outside the plateau, or past the list's end, adds zeros (an
+// accumulator that starts at +0 never becomes -0, so that changes no bit).
+// Receptor beads are deformed from their padded mode row (one cache line),
+// which also holds the type.
+// Bound by the L1's address processing of the receptor gathers and by VALU
+// issue.  Four lanes per bead rather than one: a wave's step ends after the
+// longest of 16 lists over four instead of the longest of 64, so 73 % of the
+// lanes hold a pair instead of 50 % (3000/800 beads; 61 against 30 % for
+// 1000/300), the pose's serial chain is half as long, and the four list
+// entries are one access; the fold in list order costs 4 adds per sum and
+// step instead of 1.  100,000 poses: 1000/300 rigid 3.53 -> 2.36 ms, 3000/800
+// with 5 + 5 modes and parameter gradients 18.8 -> 17.1 ms; 10,007 poses 3989/997 with
+// 10 + 10 modes 2.42 -> 1.76 ms.
 template <int MM, int PG>
 __device__ __forceinline__ void adj_walk(const PairDesc& P, const PairTab& tab,
                                          const PGrad& pg, float px, float py, float pz, float q,
-                                         unsigned lt, uint2 d, const float* ampR, float* gR,
-                                         float& eAcc, float3& gAcc, unsigned& inside) {
+                                         unsigned lt, uint2 d, unsigned s, const float* ampR,
+                                         float* gR, float& eAcc, float3& gAcc, unsigned& inside) {
     constexpr int MA = MM > 0 ? MM : 1;
     const DNL& nl = P.nl;
     const DPar& par = P.par;
     const float4* __restrict__ rpos = P.rec.pos;
-    const float4* __restrict__ rmodesT = P.rec.modesT;
-    const unsigned Mr = MM > 0 ? P.rec.M : 0, rowT = P.rec.rowT;
-    const unsigned lt1 = lt - 1;
+    const unsigned lt1 = lt - 1, last = d.x - 1;
     const uint32_t* lst = nl.list + d.y;
+    const float rrdP = par.shape == 8 ? nl.P2_inv : nl.P6_inv;
+    const float ddP = nl.ddP[par.dielec];
     eAcc = 0.f;
     gAcc = make_float3(0.f, 0.f, 0.f);
-    unsigned nxt = d.x ? lst[0] : 0u;
-    for (unsigned jj = 0; jj < d.x; ++jj) {
+    unsigned nxt = lst[min(s, last)];
+    for (unsigned jj = 0; jj < d.x; jj += 4) {
         const unsigned j = nxt;
-        if (jj + 1 < d.x) nxt = lst[jj + 1];  // next entry in flight
+        nxt = lst[min(jj + 4 + s, last)];  // next step's entry in flight
         const float4 rx = rpos[j];
-        const unsigned rt = P.rec.type[j];
-        float mt[MM > 0 ? 4 * ((3 * MA + 3) / 4) : 4];
+        float row[MM > 0 ? 4 * ((3 * MA + 4) / 4) : 4];
         float yx = rx.x, yy = rx.y, yz = rx.z;
+        unsigned rt;
         if (MM > 0) {
-            constexpr unsigned Q = (3 * MA + 3) / 4;
-            const float4* row = rmodesT + (size_t)j * rowT;
+            load_row<MA>(P.rec, j, row);
+            rt = __float_as_uint(row[0]);
+            // the deformation of deform(), same order of operations; amplitudes
+            // and modes beyond the receptor's are zero
 #pragma unroll
-            for (unsigned qq = 0; qq < Q; ++qq) {
-                const float4 v = qq < rowT ? row[qq] : make_float4(0.f, 0.f, 0.f, 0.f);
-                mt[4 * qq] = v.x; mt[4 * qq + 1] = v.y; mt[4 * qq + 2] = v.z; mt[4 * qq + 3] = v.w;
+            for (unsigned m = 0; m < (unsigned)MA; ++m) {
+                const float a = ampR[m];
+                yx = yx + a * row[3 * m + 1];
+                yy = yy + a * row[3 * m + 2];
+                yz = yz + a * row[3 * m + 3];
             }
-            // the deformation of deform(), same order of operations
-#pragma unroll
-            for (unsigned m = 0; m < (unsigned)MA; ++m)
-                if (m < Mr) {
-                    const float a = ampR[m];
-                    yx = yx + a * mt[3 * m];
-                    yy = yy + a * mt[3 * m + 1];
-                    yz = yz + a * mt[3 * m + 2];
-                }
+        } else {
+            rt = P.rec.type[j];
         }
         const float ddx = px - yx, ddy = py - yy, ddz = pz - yz;
         const float dr2 = ddx * ddx + ddy * ddy + ddz * ddz;
-        if (!(dr2 <= nl.P2) || rt - 1u >= par.T) continue;
-        ++inside;
+        const bool in = jj + s < d.x && dr2 <= nl.P2 && rt - 1u < par.T;
+        inside += in ? 1u : 0u;
         const float dr2_inv = (float)(1.0 / (double)dr2);
         const float dx = ddx * dr2_inv, dy = ddy * dr2_inv, dz = ddz * dr2_inv;
-        const unsigned kk = par.T * (rt - 1) + lt1;
+        const unsigned kk = in ? par.T * (rt - 1) + lt1 : 0u;
         const att_pair_params pp = tab[kk];
-        float Fx, Fy, Fz, ve, vx, vy, vz;
+        float Fx, Fy, Fz, ve;
         lj(dr2, dr2_inv, dx, dy, dz, pp, par.shape, Fx, Fy, Fz, ve);
-        eAcc += ve;
-        lj(nl.P2, nl.P2_inv, 0.f, 0.f, 0.f, pp, par.shape, vx, vy, vz, ve);
-        eAcc -= ve;
-        if (q != 0.f) {
-            const float qlr = q * rx.w * par.ffelec;
-            if (fabsf(qlr) > 0.001f) {
-                coulomb(dr2_inv, dx, dy, dz, qlr, par.dielec, vx, vy, vz, ve);
-                eAcc += ve;
-                Fx += vx; Fy += vy; Fz += vz;
-                coulomb(nl.P2_inv, 0.f, 0.f, 0.f, qlr, par.dielec, vx, vy, vz, ve);
-                eAcc -= ve;
+        // lj()'s energy at the plateau
+        const float ivor = (float)pp.ipon;
+        const float vljP = (pp.rc * rrdP - pp.ac) * nl.P6_inv;
+        float veP = nl.P2 < pp.rmin2 ? vljP + (ivor - 1.f) * pp.emin : ivor * vljP;
+        const float qlr = q * rx.w * par.ffelec;
+        const bool charged = in && fabsf(qlr) > 0.001f;
+        float vc = 0.f, vcP = 0.f;
+        const bool anyCharged = __any(charged);
+        if (anyCharged) {
+            float cx, cy, cz, ce;
+            coulomb(dr2_inv, dx, dy, dz, qlr, par.dielec, cx, cy, cz, ce);
+            if (charged) {
+                Fx += cx; Fy += cy; Fz += cz;
+                vc = ce;
+                vcP = qlr * ddP;
             }
         }
-        gAcc.x += Fx; gAcc.y += Fy; gAcc.z += Fz;
+        if (!in) { Fx = 0.f; Fy = 0.f; Fz = 0.f; ve = 0.f; veP = 0.f; }
+        if (anyCharged) {
+            eAcc += quad_lane<0>(ve); eAcc -= quad_lane<0>(veP); eAcc += quad_lane<0>(vc); eAcc -= quad_lane<0>(vcP);
+            eAcc += quad_lane<1>(ve); eAcc -= quad_lane<1>(veP); eAcc += quad_lane<1>(vc); eAcc -= quad_lane<1>(vcP);
+            eAcc += quad_lane<2>(ve); eAcc -= quad_lane<2>(veP); eAcc += quad_lane<2>(vc); eAcc -= quad_lane<2>(vcP);
+            eAcc += quad_lane<3>(ve); eAcc -= quad_lane<3>(veP); eAcc += quad_lane<3>(vc); eAcc -= quad_lane<3>(vcP);
+        } else {
+            eAcc += quad_lane<0>(ve); eAcc -= quad_lane<0>(veP);
+            eAcc += quad_lane<1>(ve); eAcc -= quad_lane<1>(veP);
+            eAcc += quad_lane<2>(ve); eAcc -= quad_lane<2>(veP);
+            eAcc += quad_lane<3>(ve); eAcc -= quad_lane<3>(veP);
+        }
+        gAcc.x = quad_fold(gAcc.x, Fx);
+        gAcc.y = quad_fold(gAcc.y, Fy);
+        gAcc.z = quad_fold(gAcc.z, Fz);
         if (MM > 0) {
 #pragma unroll
             for (unsigned m = 0; m < (unsigned)MA; ++m)
-                if (m < Mr) gR[m] += Fx * mt[3 * m] + Fy * mt[3 * m + 1] + Fz * mt[3 * m + 2];
+                gR[m] = quad_fold(gR[m], Fx * row[3 * m + 1] + Fy * row[3 * m + 2] + Fz * row[3 * m + 3]);
         }
-        if (PG != kPgNone) {
+        if (PG != kPgNone && in) {
             float drc, dac, dem, drcP, dacP, demP;
             lj_dparam(dr2, dr2_inv, pp, par.shape, drc, dac, dem);
             lj_dparam(nl.P2, nl.P2_inv, pp, par.shape, drcP, dacP, demP);
@@ -330,13 +359,21 @@ struct PoseLDS {
     float e;
 };
 
+// The group (of nthr / 4) whose queue item this thread's quad takes in
+// sub-round `sub`.
+template <int WAVES>
+__device__ __forceinline__ unsigned quad_group(unsigned tid, unsigned sub) {
+    const unsigned wave = tid / kWave, quad = (tid & (kWave - 1)) >> 2;
+    return (sub & 1u ? WAVES - 1u - wave : wave) * 16u + quad;
+}
+
 // Adjoint of one pose by one workgroup of WAVES waves, the ligand in
 // super-chunks of equal size, at most PoseLDS<WAVES>::kSuper beads (super_chunk):
 //  P1  every bead: transform, grid term with its exact gradient (and the
 //      basis-grid parameter derivatives), neighbour-list cell;
 //  P2  beads with a list, longest lists first (class_queue);
-//  P3  one bead per lane walks its list (adj_walk); the bead's energy becomes
-//      grid + pair fold, the reference's per-bead value;
+//  P3  one bead per quad of lanes walks its list (adj_walk); the bead's energy
+//      becomes grid + pair fold, the reference's per-bead value;
 //  P4  the energy summed in bead order (reducePotForce's order, so the pose
 //      energy is the reference's bits), and the chain rule through p = R x~ + t
 //      by wave 0, bead k on lane k % 64, lane sums reduced by a butterfly.
@@ -361,7 +398,7 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
     float ampR[MA], ampL[MA];
 #pragma unroll
     for (int m = 0; m < MA; ++m) {
-        ampR[m] = MM > 0 ? d[6 + m] : 0.f;
+        ampR[m] = MM > 0 && m < (int)Mr ? d[6 + m] : 0.f;
         ampL[m] = MM > 0 ? d[16 + m] : 0.f;
     }
     float t[6];
@@ -390,6 +427,30 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
         return p;
     };
 
+    // the same from the bead's row (one lane in four needs a bead of its own:
+    // five loads of one address per quad instead of 1 + 3 M)
+    auto place_row = [&](unsigned i, float4& x, unsigned& lt) __attribute__((always_inline)) {
+        x = lig.pos[i];
+        V3 xt{x.x, x.y, x.z};
+        if (MM > 0) {
+            float row[4 * ((3 * MA + 4) / 4)];
+            load_row<MA>(lig, i, row);
+            lt = __float_as_uint(row[0]);
+#pragma unroll
+            for (unsigned m = 0; m < (unsigned)MA; ++m)
+                if (m < Ml) {
+                    xt.x = xt.x + ampL[m] * row[3 * m + 1];
+                    xt.y = xt.y + ampL[m] * row[3 * m + 2];
+                    xt.z = xt.z + ampL[m] * row[3 * m + 3];
+                }
+        } else {
+            lt = lig.type[i];
+        }
+        V3 p = matvec(R, xt.x, xt.y, xt.z);
+        p.x = p.x + tx; p.y = p.y + ty; p.z = p.z + tz;
+        return p;
+    };
+
     const unsigned span = super_chunk(lig.n, PoseLDS<WAVES>::kSuper);
     for (unsigned sc = 0; sc < lig.n; sc += span) {
         const unsigned m = min(span, lig.n - sc);
@@ -410,19 +471,35 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
                                         nthr, [] { __syncthreads(); });
         // P3
         for (unsigned q0 = 0; q0 < qn; q0 += nthr) {
-            if (q0 + tid < qn) {
-                const unsigned k = S.q[q0 + tid];
-                float4 x;
-                const V3 p = place(sc + k, x);
-                float eAcc;
-                float3 gAcc;
-                adj_walk<MM, PG>(P, tab, pg, p.x, p.y, p.z, x.w, lig.type[sc + k], S.nlc[k], ampR, gR,
-                                 eAcc, gAcc, inside);
-                listed += S.nlc[k].x;
-                float4 g = S.g[k];
-                g.x = g.x - gAcc.x; g.y = g.y - gAcc.y; g.z = g.z - gAcc.z;
-                g.w = g.w + eAcc;  // outLig_E[i] += eAcc
-                S.g[k] = g;
+            for (unsigned sub = 0; sub < 4; ++sub) {
+                // Quad sums of queue item i belong to thread i % nthr: item
+                // q0 + sub * nthr / 4 + group, kept by the quad's lane `sub`.
+                // Odd sub-rounds give the waves the groups in reverse order
+                // (the queue is sorted: a later group's lists are shorter).
+                const unsigned item = q0 + sub * (nthr / 4) + quad_group<WAVES>(tid, sub);
+                if (item < qn) {
+                    const unsigned k = S.q[item];
+                    float4 x;
+                    unsigned lt;
+                    const V3 p = place_row(sc + k, x, lt);
+                    float eAcc, g4[MA];
+                    float3 gAcc;
+#pragma unroll
+                    for (int m = 0; m < MA; ++m) g4[m] = MM > 0 ? __shfl(gR[m], (lane & ~3u) | sub) : 0.f;
+                    const uint2 nlc = S.nlc[k];
+                    adj_walk<MM, PG>(P, tab, pg, p.x, p.y, p.z, x.w, lt, nlc, lane & 3u, ampR, g4,
+                                     eAcc, gAcc, inside);
+#pragma unroll
+                    for (int m = 0; m < MA; ++m)
+                        if (MM > 0 && (lane & 3u) == sub) gR[m] = g4[m];
+                    if ((lane & 3u) == 0) {
+                        listed += nlc.x;
+                        float4 g = S.g[k];
+                        g.x = g.x - gAcc.x; g.y = g.y - gAcc.y; g.z = g.z - gAcc.z;
+                        g.w = g.w + eAcc;  // outLig_E[i] += eAcc
+                        S.g[k] = g;
+                    }
+                }
             }
         }
         __syncthreads();
@@ -468,8 +545,17 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
 #pragma unroll
         for (int m = 0; m < MA; ++m) gL[m] = wave_sum(gL[m]);
     }
+    if (MM > 0) {
+        // the quads' receptor-mode sums to the threads they belong to (the
+        // beads' array is free), then the wave butterflies
+        float* t = reinterpret_cast<float*>(S.g);
+        const unsigned owner = (lane & 3u) * (nthr / 4) + quad_group<WAVES>(tid, lane & 3u);
 #pragma unroll
-    for (int m = 0; m < MA; ++m) gR[m] = wave_sum(gR[m]);
+        for (int m = 0; m < MA; ++m) t[m * nthr + owner] = gR[m];
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < MA; ++m) gR[m] = wave_sum(t[m * nthr + tid]);
+    }
     if (lane == 0) {
 #pragma unroll
         for (int m = 0; m < ATT_MODES_MAX; ++m) S.red[wave][m] = m < MA ? gR[m < MA ? m : 0] : 0.f;

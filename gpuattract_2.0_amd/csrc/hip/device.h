@@ -40,6 +40,8 @@ struct DNL {
     unsigned nx, ny, nz;
     float lox, loy, loz, hix, hiy, hiz;
     float dVox_inv, P2, P2_inv;
+    float P6_inv;  // P2_inv^3, as lj() forms it
+    float ddP[2];  // coulomb()'s distance factor at the plateau, by dielec
 };
 
 // Protein (model/Protein.h:38-167): pos = {x, y, z, charge}.
@@ -48,7 +50,7 @@ struct DProt {
     const unsigned* type;
     const unsigned* mtype;
     const float* modes;   // [c][m][n]: coalesced over beads
-    const float4* modesT; // per bead one row of 3*M floats [m][c], padded to a float4 multiple
+    const float4* modesT; // per bead one row {type bits, 3*M floats [m][c]}, padded to a float4 multiple
     const float* modeForce;
     unsigned n, M, rowT;  // rowT = float4 per modesT row
 };
@@ -553,6 +555,21 @@ __device__ __forceinline__ unsigned class_queue(Cnt cnt, unsigned m, unsigned sh
     return total;
 }
 
+// The value of lane K of this lane's quad (four consecutive lanes, all active).
+template <int K>
+__device__ __forceinline__ float quad_lane(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), K * 0x55, 0xf, 0xf, true));
+}
+
+// acc + the quad's four values, added one after the other in lane order.
+__device__ __forceinline__ float quad_fold(float acc, float v) {
+    acc += quad_lane<0>(v);
+    acc += quad_lane<1>(v);
+    acc += quad_lane<2>(v);
+    acc += quad_lane<3>(v);
+    return acc;
+}
+
 // Butterfly sum over the 64 lanes of a wave (same value on every lane).
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
@@ -674,6 +691,26 @@ __device__ __forceinline__ void load_modes(const DProt& b, unsigned i, BeadModes
         md.x[m] = m < b.M ? b.modes[(size_t)m * b.n + i] : 0.f;
         md.y[m] = m < b.M ? b.modes[nM + (size_t)m * b.n + i] : 0.f;
         md.z[m] = m < b.M ? b.modes[2 * nM + (size_t)m * b.n + i] : 0.f;
+    }
+}
+
+// The row of bead i, f = {type bits, m0x, m0y, m0z, m1x, ...}, zero beyond the
+// body's modes up to the capacity MM (4 * ceil((3 MM + 1) / 4) floats).
+template <int MM>
+__device__ __forceinline__ void load_row(const DProt& b, unsigned i, float* f) {
+    constexpr unsigned Q = (3 * MM + 4) / 4;
+    const float4* row = b.modesT + (size_t)i * b.rowT;
+    float4 v[Q];
+    if (b.rowT >= Q) {  // uniform; the loads issue together
+#pragma unroll
+        for (unsigned q = 0; q < Q; ++q) v[q] = row[q];
+    } else {
+#pragma unroll
+        for (unsigned q = 0; q < Q; ++q) v[q] = q < b.rowT ? row[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (unsigned q = 0; q < Q; ++q) {
+        f[4 * q] = v[q].x; f[4 * q + 1] = v[q].y; f[4 * q + 2] = v[q].z; f[4 * q + 3] = v[q].w;
     }
 }
 

@@ -259,6 +259,9 @@ att_status attach_nl(att_ctx* c, GridObj* o, unsigned nx, unsigned ny, unsigned 
     d.dVox_inv = 1.f / dv;
     d.P2 = P2;
     d.P2_inv = 1.f / P2;
+    d.P6_inv = d.P2_inv * d.P2_inv * d.P2_inv;
+    d.ddP[0] = std::max((float)((double)std::sqrt(d.P2_inv) - 1.0 / 50.0), 0.f);
+    d.ddP[1] = std::max((float)((double)d.P2_inv - 1.0 / (50.0 * 50.0)), 0.f);
     o->hasNL = true;
     return ATT_OK;
 }
@@ -446,29 +449,35 @@ att_status att_upload_protein(att_ctx* c, const att_protein_desc* d, att_handle*
     o->d.mtype = dmtype;
     o->d.n = n;
     o->d.M = M;
-    if (M > 0) {
-        const size_t nM = (size_t)n * M;
-        const unsigned rowT = (3 * M + 3) / 4;  // float4 per padded row
-        std::vector<float> soa(3 * nM), aos((size_t)n * rowT * 4, 0.f);
-        for (unsigned cc = 0; cc < 3; ++cc)
-            for (unsigned i = 0; i < n; ++i)
-                for (unsigned m = 0; m < M; ++m) {
-                    const float v = d->modes[cc * nM + (size_t)i * M + m];
-                    soa[(cc * M + m) * (size_t)n + i] = v;
-                    aos[(size_t)i * rowT * 4 + 3 * m + cc] = v;
-                }
-        float *dsoa, *dmf;
-        float4* daos;
-        if ((st = dev_copy(c, o.get(), soa.data(), soa.size(), &dsoa)) != ATT_OK) return st;
-        if ((st = dev_copy(c, o.get(), reinterpret_cast<const float4*>(aos.data()),
-                           (size_t)n * rowT, &daos)) != ATT_OK)
-            return st;
-        if ((st = dev_copy(c, o.get(), d->modeForce, M, &dmf)) != ATT_OK) return st;
-        o->d.modes = dsoa;
-        o->d.modesT = daos;
-        o->d.modeForce = dmf;
-        o->d.rowT = rowT;
-    }
+    // rows {type, modes} for the neighbour-list gathers; without modes too, for
+    // a rigid body scored with a flexible one.  A bead with a non-finite mode
+    // has no finite distance to anything, so none of its pairs counts: its row
+    // is zero (type 0), so that the walks' masked sums stay finite.
+    const size_t nM = (size_t)n * M;
+    const unsigned rowT = (3 * M + 4) / 4;  // float4 per padded row
+    std::vector<float> soa(3 * nM), rows((size_t)n * rowT * 4, 0.f);
+    for (unsigned i = 0; i < n; ++i) std::memcpy(&rows[(size_t)i * rowT * 4], &d->type[i], 4);
+    std::vector<unsigned> bad;
+    for (unsigned cc = 0; cc < 3; ++cc)
+        for (unsigned i = 0; i < n; ++i)
+            for (unsigned m = 0; m < M; ++m) {
+                const float v = d->modes[cc * nM + (size_t)i * M + m];
+                soa[(cc * M + m) * (size_t)n + i] = v;
+                rows[(size_t)i * rowT * 4 + 1 + 3 * m + cc] = v;
+                if (!std::isfinite(v)) bad.push_back(i);
+            }
+    for (unsigned i : bad) std::fill_n(&rows[(size_t)i * rowT * 4], (size_t)rowT * 4, 0.f);
+    float *dsoa, *dmf;
+    float4* drows;
+    if ((st = dev_copy(c, o.get(), soa.data(), soa.size(), &dsoa)) != ATT_OK) return st;
+    if ((st = dev_copy(c, o.get(), reinterpret_cast<const float4*>(rows.data()), (size_t)n * rowT,
+                       &drows)) != ATT_OK)
+        return st;
+    if ((st = dev_copy(c, o.get(), d->modeForce, M, &dmf)) != ATT_OK) return st;
+    o->d.modes = dsoa;
+    o->d.modesT = drows;
+    o->d.modeForce = dmf;
+    o->d.rowT = rowT;
     *out = store(c, std::move(o));
     return ATT_OK;
 }

@@ -121,8 +121,8 @@ __global__ __launch_bounds__(256) void k_rigid(DProt rec, DProt lig, DGrid inner
 
 // The deformed receptor position of bead j from its padded mode row (one or
 // two 16-byte loads), in the order of deform(): bit-identical coordinates.
-// The row is also left in `rowOut` (4 * ceil(3M / 4) floats) for the pair's
-// reaction, which then does not load it again.
+// The row {type, modes} is also left in `rowOut` (4 * ceil((3M + 1) / 4)
+// floats) for the pair's reaction, which then does not load it again.
 template <int MM>
 struct RecPosDeform {
     const float4* pos;
@@ -135,7 +135,7 @@ struct RecPosDeform {
         float yx = x.x, yy = x.y, yz = x.z;
         if (MM > 0) {
             constexpr int MA = MM > 0 ? MM : 1;
-            constexpr unsigned Q = (3 * MA + 3) / 4;
+            constexpr unsigned Q = (3 * MA + 4) / 4;
             float mt[4 * Q];
             const float4* row = modesT + (size_t)j * rowT;
 #pragma unroll
@@ -149,9 +149,9 @@ struct RecPosDeform {
             for (unsigned m = 0; m < (unsigned)MA; ++m)
                 if (m < M) {
                     const float a = amp[m];
-                    yx = yx + a * mt[3 * m];
-                    yy = yy + a * mt[3 * m + 1];
-                    yz = yz + a * mt[3 * m + 2];
+                    yx = yx + a * mt[3 * m + 1];
+                    yy = yy + a * mt[3 * m + 2];
+                    yz = yz + a * mt[3 * m + 3];
                 }
         }
         return make_float3(yx, yy, yz);
@@ -272,12 +272,12 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
     // one RecPosDeform left in rowBuf.
     constexpr int kWalkBatch = 1;
     static_assert(kWalkBatch == 1, "the reaction reads the row of the last deformed bead");
-    float rowBuf[4 * ((3 * MA + 3) / 4)];
+    float rowBuf[4 * ((3 * MA + 4) / 4)];
     auto reaction = [&](unsigned, float fx, float fy, float fz) {
         const float* mt = rowBuf;
 #pragma unroll
         for (unsigned m = 0; m < (unsigned)MM; ++m)
-            if (m < Mr) mR[m] -= fx * mt[3 * m] + fy * mt[3 * m + 1] + fz * mt[3 * m + 2];
+            if (m < Mr) mR[m] -= fx * mt[3 * m + 1] + fy * mt[3 * m + 2] + fz * mt[3 * m + 3];
     };
     auto place = [&](unsigned i, float4& x) {
         x = lig.pos[i];

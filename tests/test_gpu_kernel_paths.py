@@ -29,3 +29,31 @@ def test_energy_octets_same_bits(ctx, W, nl, mr, ml, n):
     finally:
         ctx.set_energy_octets(True)
     assert np.array_equal(got.view(np.uint32), full.view(np.uint32))
+
+
+@pytest.mark.parametrize("nl, mr, ml", [(1, 0, 0), (64, 0, 0), (257, 0, 0), (384, 0, 0), (67, 0, 7),
+                                        (130, 1, 0), (300, 5, 5), (383, 10, 4), (513, 4, 9),
+                                        (520, 10, 10)])
+def test_list_walk_by_quads_is_the_kernel_order(ctx, W, O, nl, mr, ml):
+    """Lists of every length (poses from contact to out of reach), queues that
+    are no multiple of the 16 beads a wave walks at once, one to three
+    super-chunks, every mode capacity: the oracle's kernel-order bits."""
+    wl = W.make_workload("quads", 400 + nl, 250, nl, 24, mr, ml, shell=(8.0, 45.0),
+                         with_lig_grid=False)
+    hs = ctx.upload_workload(wl)
+    w = np.linspace(-1.0, 2.0, 24).astype(np.float32)
+    got = ctx.adjoint(hs, wl.dofs, w=w)
+    ref = O.adjoint_kernel_order(wl, w=w)[:, :got.shape[1]].astype(np.float32)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
+def test_receptor_bead_with_a_non_finite_mode_is_skipped(ctx, W, O):
+    """Its pairs have no finite distance: they add nothing to any sum."""
+    wl = W.make_workload("nan mode", 420, 250, 90, 30, 3, 2, shell=(8.0, 30.0), with_lig_grid=False)
+    m = wl.rec.modes.reshape(3, wl.rec.n, 3)
+    m[0, ::7, 1] = np.nan
+    m[2, ::11, 2] = np.inf
+    got = ctx.adjoint(ctx.upload_workload(wl), wl.dofs)
+    ref = O.adjoint_kernel_order(wl)[:, :got.shape[1]].astype(np.float32)
+    assert np.isfinite(got).all()
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
