@@ -256,7 +256,6 @@ __device__ __forceinline__ void adj_walk(const PairDesc& P, const PairTab& tab,
     constexpr int MA = MM > 0 ? MM : 1;
     const DNL& nl = P.nl;
     const DPar& par = P.par;
-    const float4* __restrict__ rpos = P.rec.pos;
     const unsigned lt1 = lt - 1, last = d.x - 1;
     const uint32_t* lst = nl.list + d.y;
     const float rrdP = par.shape == 8 ? nl.P2_inv : nl.P6_inv;
@@ -267,26 +266,10 @@ __device__ __forceinline__ void adj_walk(const PairDesc& P, const PairTab& tab,
     for (unsigned jj = 0; jj < d.x; jj += 4) {
         const unsigned j = nxt;
         nxt = lst[min(jj + 4 + s, last)];  // next step's entry in flight
-        const float4 rx = rpos[j];
-        float row[MM > 0 ? 4 * ((3 * MA + 4) / 4) : 4];
-        float yx = rx.x, yy = rx.y, yz = rx.z;
-        unsigned rt;
-        if (MM > 0) {
-            load_row<MA>(P.rec, j, row);
-            rt = __float_as_uint(row[0]);
-            // the deformation of deform(), same order of operations; amplitudes
-            // and modes beyond the receptor's are zero
-#pragma unroll
-            for (unsigned m = 0; m < (unsigned)MA; ++m) {
-                const float a = ampR[m];
-                yx = yx + a * row[3 * m + 1];
-                yy = yy + a * row[3 * m + 2];
-                yz = yz + a * row[3 * m + 3];
-            }
-        } else {
-            rt = P.rec.type[j];
-        }
-        const float ddx = px - yx, ddy = py - yy, ddz = pz - yz;
+        RecBead<MM> rb;
+        rb.load(P.rec, j, ampR);
+        const unsigned rt = rb.type;
+        const float ddx = px - rb.x, ddy = py - rb.y, ddz = pz - rb.z;
         const float dr2 = ddx * ddx + ddy * ddy + ddz * ddz;
         const bool in = jj + s < d.x && dr2 <= nl.P2 && rt - 1u < par.T;
         inside += in ? 1u : 0u;
@@ -300,7 +283,7 @@ __device__ __forceinline__ void adj_walk(const PairDesc& P, const PairTab& tab,
         const float ivor = (float)pp.ipon;
         const float vljP = (pp.rc * rrdP - pp.ac) * nl.P6_inv;
         float veP = nl.P2 < pp.rmin2 ? vljP + (ivor - 1.f) * pp.emin : ivor * vljP;
-        const float qlr = q * rx.w * par.ffelec;
+        const float qlr = q * rb.q * par.ffelec;
         const bool charged = in && fabsf(qlr) > 0.001f;
         float vc = 0.f, vcP = 0.f;
         const bool anyCharged = __any(charged);
@@ -331,7 +314,7 @@ __device__ __forceinline__ void adj_walk(const PairDesc& P, const PairTab& tab,
         if (MM > 0) {
 #pragma unroll
             for (unsigned m = 0; m < (unsigned)MA; ++m)
-                gR[m] = quad_fold(gR[m], Fx * row[3 * m + 1] + Fy * row[3 * m + 2] + Fz * row[3 * m + 3]);
+                gR[m] = quad_fold(gR[m], Fx * rb.row[3 * m + 1] + Fy * rb.row[3 * m + 2] + Fz * rb.row[3 * m + 3]);
         }
         if (PG != kPgNone && in) {
             float drc, dac, dem, drcP, dacP, demP;
@@ -358,14 +341,6 @@ struct PoseLDS {
     unsigned cnt[WAVES][2];
     float e;
 };
-
-// The group (of nthr / 4) whose queue item this thread's quad takes in
-// sub-round `sub`.
-template <int WAVES>
-__device__ __forceinline__ unsigned quad_group(unsigned tid, unsigned sub) {
-    const unsigned wave = tid / kWave, quad = (tid & (kWave - 1)) >> 2;
-    return (sub & 1u ? WAVES - 1u - wave : wave) * 16u + quad;
-}
 
 // Adjoint of one pose by one workgroup of WAVES waves, the ligand in
 // super-chunks of equal size, at most PoseLDS<WAVES>::kSuper beads (super_chunk):
@@ -399,7 +374,7 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
 #pragma unroll
     for (int m = 0; m < MA; ++m) {
         ampR[m] = MM > 0 && m < (int)Mr ? d[6 + m] : 0.f;
-        ampL[m] = MM > 0 ? d[16 + m] : 0.f;
+        ampL[m] = MM > 0 && m < (int)Ml ? d[16 + m] : 0.f;
     }
     float t[6];
     pose_trig(d[3], d[4], d[5], lane, t);
@@ -427,28 +402,8 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
         return p;
     };
 
-    // the same from the bead's row (one lane in four needs a bead of its own:
-    // five loads of one address per quad instead of 1 + 3 M)
     auto place_row = [&](unsigned i, float4& x, unsigned& lt) __attribute__((always_inline)) {
-        x = lig.pos[i];
-        V3 xt{x.x, x.y, x.z};
-        if (MM > 0) {
-            float row[4 * ((3 * MA + 4) / 4)];
-            load_row<MA>(lig, i, row);
-            lt = __float_as_uint(row[0]);
-#pragma unroll
-            for (unsigned m = 0; m < (unsigned)MA; ++m)
-                if (m < Ml) {
-                    xt.x = xt.x + ampL[m] * row[3 * m + 1];
-                    xt.y = xt.y + ampL[m] * row[3 * m + 2];
-                    xt.z = xt.z + ampL[m] * row[3 * m + 3];
-                }
-        } else {
-            lt = lig.type[i];
-        }
-        V3 p = matvec(R, xt.x, xt.y, xt.z);
-        p.x = p.x + tx; p.y = p.y + ty; p.z = p.z + tz;
-        return p;
+        return place_from_row<MM>(lig, i, ampL, R, tx, ty, tz, x, lt);
     };
 
     const unsigned span = super_chunk(lig.n, PoseLDS<WAVES>::kSuper);

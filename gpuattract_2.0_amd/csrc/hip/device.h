@@ -42,6 +42,7 @@ struct DNL {
     float dVox_inv, P2, P2_inv;
     float P6_inv;  // P2_inv^3, as lj() forms it
     float ddP[2];  // coulomb()'s distance factor at the plateau, by dielec
+    double ratioC; // 1 / (10000 P2), for plateau_ratio_fast
 };
 
 // Protein (model/Protein.h:38-167): pos = {x, y, z, charge}.
@@ -283,7 +284,8 @@ __device__ __forceinline__ void lj(float dr2, float dr2_inv, float dx, float dy,
     const float shapedelta = shape == 8 ? 2.f : 6.f;
     const float rep = p.rc * rrd;
     const float vlj = (rep - p.ac) * rr23;
-    const double s = 6.0 * (double)vlj + (double)(shapedelta * (rep * rr23));
+    // 6 vlj is exact in double: fma rounds as the product and the sum would
+    const double s = __builtin_fma(6.0, (double)vlj, (double)(shapedelta * (rep * rr23)));
     float fb;
     if (dr2 < p.rmin2) {
         e = vlj + (ivor - 1.f) * p.emin;
@@ -373,6 +375,22 @@ __device__ __forceinline__ PairTab stage_table(const DPar& par, att_pair_params*
 // over every entry), and the walk waits on no load after the distance.
 __device__ __forceinline__ float plateau_ratio(unsigned n, float P2) {
     return (float)__builtin_sqrt((((double)n + 0.5) / 10000.0) / (double)P2);
+}
+
+// plateau_ratio from one square-root estimate: the entry to a relative error
+// below 2^-42 in double (the estimate's 2^-22 squared by one Newton step; c =
+// 1 / (10000 P2)), which rounds to the entry's float unless a rounding boundary
+// lies that close (one entry in 2^17): those take plateau_ratio.  The same
+// bits in 16 instructions instead of about 50.
+__device__ __forceinline__ float plateau_ratio_fast(unsigned n, float P2, double c) {
+    const double u = __builtin_fma((double)n, c, 0.5 * c);
+    const float uf = (float)u;
+    const float rs = __builtin_amdgcn_rsqf(uf);
+    const double s0 = (double)(uf * rs), h = (double)(0.5f * rs);
+    const double s = __builtin_fma(__builtin_fma(-s0, s0, u), h, s0);
+    constexpr double eps = 0x1p-42;
+    const float lo = (float)__builtin_fma(s, -eps, s), hi = (float)__builtin_fma(s, eps, s);
+    return lo == hi ? lo : plateau_ratio(n, P2);  // NaN takes the exact path too
 }
 
 // The pair loop of NLPotForce for one ligand bead (model/neighborlist.h:66-158
@@ -494,9 +512,9 @@ __device__ __forceinline__ bool nl_bead(const DNL& nl, const DPar& par,
     return true;
 }
 
-// Beads whose neighbour lists are walked one per lane are ordered by list
+// Beads whose neighbour lists are walked one per quad are ordered by list
 // length: nine classes, longest first (>= 64, 48, 36, 28, 22, 16, 11, 6, 1
-// pairs), bead order inside a class, so that the lanes of a wave walk lists of
+// pairs), bead order inside a class, so that the quads of a wave walk lists of
 // similar length.  The class of a bead with cnt > 0 listed neighbours:
 constexpr unsigned kQueueClasses = 9;
 __device__ __forceinline__ unsigned queue_class(unsigned cnt) {
@@ -656,7 +674,8 @@ struct BatchTile {
 constexpr unsigned kBatchQueues = 8;
 
 struct NoReaction {
-    __device__ void operator()(unsigned, float, float, float) const {}
+    template <class Rec>
+    __device__ void operator()(const Rec&, float, float, float) const {}
 };
 
 // Receptor accessors reading the protein arrays in global memory.
@@ -714,6 +733,109 @@ __device__ __forceinline__ void load_row(const DProt& b, unsigned i, float* f) {
     }
 }
 
+// A receptor bead as the list walks need it: position (deformed by the
+// amplitudes amp, zero beyond the receptor's modes; the order of deform()),
+// charge, type, and its row for the projections on the modes.
+template <int MM>
+struct RecBead {
+    float x, y, z, q;
+    unsigned type;
+    float row[MM > 0 ? 4 * ((3 * MM + 4) / 4) : 1];
+
+    __device__ __forceinline__ void load(const DProt& rec, unsigned j, const float* amp) {
+        const float4 p = rec.pos[j];
+        x = p.x; y = p.y; z = p.z; q = p.w;
+        if constexpr (MM > 0) {
+            load_row<MM>(rec, j, row);
+            type = __float_as_uint(row[0]);
+#pragma unroll
+            for (unsigned m = 0; m < (unsigned)MM; ++m) {
+                x = x + amp[m] * row[3 * m + 1];
+                y = y + amp[m] * row[3 * m + 2];
+                z = z + amp[m] * row[3 * m + 3];
+            }
+        } else {
+            type = rec.type[j];
+        }
+    }
+};
+
+// The pair loop of NLPotForce for one ligand bead as nl_walk below, by the four
+// lanes of a quad (s = lane in the quad) over the list d = {numEl, idx}
+// (numEl > 0): each step takes four consecutive list entries, one per lane, and
+// the four pairs' terms are then added in list order on every lane, so every
+// lane returns the reference's bits.  A pair outside the plateau, or past the
+// list's end, adds zeros (an accumulator that starts at +0 never becomes -0,
+// so that changes no bit).  reaction(rec, fx, fy, fz) receives each lane's
+// pair's reaction force (zero for those).  Bound like the adjoint's adj_walk;
+// 100,000 rigid poses (1000/300): 4.43 -> 3.42 ms against one lane per bead,
+// 20,011 flexible ones (3000/800, 5 + 5 modes) 6.22 -> 5.08 ms.
+template <int MM, class Reaction>
+__device__ __forceinline__ float4 nl_walk_quad(const DNL& nl, const DPar& par, const PairTab& tab,
+                                               const DProt& rec, const float* ampR,
+                                               Reaction reaction, float px, float py, float pz,
+                                               unsigned ligType, float ligCharge, uint2 d,
+                                               unsigned s, unsigned& inside) {
+    float fx = 0.f, fy = 0.f, fz = 0.f, e = 0.f;
+    const unsigned lt1 = ligType - 1, last = d.x - 1;
+    const uint32_t* lst = nl.list + d.y;
+    unsigned nxt = lst[min(s, last)];
+    for (unsigned jj = 0; jj < d.x; jj += 4) {
+        const unsigned j = nxt;
+        nxt = lst[min(jj + 4 + s, last)];  // next step's entry in flight
+        RecBead<MM> rb;
+        rb.load(rec, j, ampR);
+        const float ddx = px - rb.x, ddy = py - rb.y, ddz = pz - rb.z;
+        const float dr2 = ddx * ddx + ddy * ddy + ddz * ddz;
+        const bool in = jj + s < d.x && dr2 <= nl.P2 && rb.type - 1u < par.T;
+        inside += in ? 1u : 0u;
+        const float ratio = in ? plateau_ratio_fast((unsigned)(int)(dr2 * 10000.f), nl.P2, nl.ratioC) : 0.f;
+        const float dr2_inv = (float)(1.0 / (double)dr2);
+        const float dx = ddx * dr2_inv, dy = ddy * dr2_inv, dz = ddz * dr2_inv;
+        const att_pair_params p = tab[in ? par.T * (rb.type - 1) + lt1 : 0u];
+        float vx, vy, vz, ve, wx, wy, wz, we;  // at r, at the plateau
+        lj(dr2, dr2_inv, dx, dy, dz, p, par.shape, vx, vy, vz, ve);
+        const float rdx = ratio * dx, rdy = ratio * dy, rdz = ratio * dz;
+        lj(nl.P2, nl.P2_inv, rdx, rdy, rdz, p, par.shape, wx, wy, wz, we);
+        if (!in) { vx = vy = vz = ve = 0.f; wx = wy = wz = we = 0.f; }
+        float rfx = wx - vx, rfy = wy - vy, rfz = wz - vz;  // -v + w: (0 - v) + w exactly
+        const float qlr = ligCharge * rb.q * par.ffelec;
+        const bool charged = in && fabsf(qlr) > 0.001f;
+        if (__any(charged)) {
+            float cx, cy, cz, ce, ex, ey, ez, ee;
+            coulomb(dr2_inv, dx, dy, dz, qlr, par.dielec, cx, cy, cz, ce);
+            coulomb(nl.P2_inv, rdx, rdy, rdz, qlr, par.dielec, ex, ey, ez, ee);
+            if (!charged) { cx = cy = cz = ce = 0.f; ex = ey = ez = ee = 0.f; }
+            rfx = (rfx - cx) + ex; rfy = (rfy - cy) + ey; rfz = (rfz - cz) + ez;
+            auto fold = [](float acc, float a, float b, float c, float g) __attribute__((always_inline)) {
+                acc += quad_lane<0>(a); acc -= quad_lane<0>(b); acc += quad_lane<0>(c); acc -= quad_lane<0>(g);
+                acc += quad_lane<1>(a); acc -= quad_lane<1>(b); acc += quad_lane<1>(c); acc -= quad_lane<1>(g);
+                acc += quad_lane<2>(a); acc -= quad_lane<2>(b); acc += quad_lane<2>(c); acc -= quad_lane<2>(g);
+                acc += quad_lane<3>(a); acc -= quad_lane<3>(b); acc += quad_lane<3>(c); acc -= quad_lane<3>(g);
+                return acc;
+            };
+            fx = fold(fx, vx, wx, cx, ex);
+            fy = fold(fy, vy, wy, cy, ey);
+            fz = fold(fz, vz, wz, cz, ez);
+            e = fold(e, ve, we, ce, ee);
+        } else {
+            auto fold = [](float acc, float a, float b) __attribute__((always_inline)) {
+                acc += quad_lane<0>(a); acc -= quad_lane<0>(b);
+                acc += quad_lane<1>(a); acc -= quad_lane<1>(b);
+                acc += quad_lane<2>(a); acc -= quad_lane<2>(b);
+                acc += quad_lane<3>(a); acc -= quad_lane<3>(b);
+                return acc;
+            };
+            fx = fold(fx, vx, wx);
+            fy = fold(fy, vy, wy);
+            fz = fold(fz, vz, wz);
+            e = fold(e, ve, we);
+        }
+        reaction(rb, rfx, rfy, rfz);
+    }
+    return make_float4(fx, fy, fz, e);
+}
+
 // Mode deformation x + sum_m a_m * mode_m, sequential over modes
 // (model/transform.h:69-73).
 template <int MM>
@@ -729,6 +851,42 @@ __device__ __forceinline__ V3 deform(const BeadModes<MM>& md, unsigned M, float 
             p.z = p.z + a * md.z[m];
         }
     }
+    return p;
+}
+
+// The group (of nthr / 4) whose queue item this thread's quad takes in
+// sub-round `sub`.
+template <int WAVES>
+__device__ __forceinline__ unsigned quad_group(unsigned tid, unsigned sub) {
+    const unsigned wave = tid / kWave, quad = (tid & (kWave - 1)) >> 2;
+    return (sub & 1u ? WAVES - 1u - wave : wave) * 16u + quad;
+}
+
+// A ligand bead's position from its row (one bead per quad: a few loads of one
+// address per quad instead of 1 + 3 M), deformed as deform() does and moved by
+// (R, t); amp is zero beyond the ligand's modes.
+template <int MM>
+__device__ __forceinline__ V3 place_from_row(const DProt& lig, unsigned i, const float* amp,
+                                             const float* R, float tx, float ty, float tz, float4& x,
+                                             unsigned& type) {
+    x = lig.pos[i];
+    V3 xt{x.x, x.y, x.z};
+    if constexpr (MM > 0) {
+        float row[4 * ((3 * MM + 4) / 4)];
+        load_row<MM>(lig, i, row);
+        type = __float_as_uint(row[0]);
+#pragma unroll
+        for (unsigned m = 0; m < (unsigned)MM; ++m)
+            if (m < lig.M) {
+                xt.x = xt.x + amp[m] * row[3 * m + 1];
+                xt.y = xt.y + amp[m] * row[3 * m + 2];
+                xt.z = xt.z + amp[m] * row[3 * m + 3];
+            }
+    } else {
+        type = lig.type[i];
+    }
+    V3 p = matvec(R, xt.x, xt.y, xt.z);
+    p.x = p.x + tx; p.y = p.y + ty; p.z = p.z + tz;
     return p;
 }
 

@@ -259,6 +259,7 @@ att_status attach_nl(att_ctx* c, GridObj* o, unsigned nx, unsigned ny, unsigned 
     d.dVox_inv = 1.f / dv;
     d.P2 = P2;
     d.P2_inv = 1.f / P2;
+    d.ratioC = 1.0 / (10000.0 * (double)P2);
     d.P6_inv = d.P2_inv * d.P2_inv * d.P2_inv;
     d.ddP[0] = std::max((float)((double)std::sqrt(d.P2_inv) - 1.0 / 50.0), 0.f);
     d.ddP[1] = std::max((float)((double)d.P2_inv - 1.0 / (50.0 * 50.0)), 0.f);

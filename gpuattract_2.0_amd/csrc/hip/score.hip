@@ -1,21 +1,19 @@
 // Scoring kernels for gfx950 and their launchers.
 //
 //  k_rigid  one 64-lane wavefront per pose, four poses per 256-thread workgroup.
-//           Lanes stride over ligand beads (transform, grid interpolation),
-//           then walk the neighbour-list pairs of each chunk of 64 beads one
-//           pair per lane; per-lane partial sums of E, F and the torque
-//           tensor; a butterfly reduction and a one-lane epilogue (force
-//           clamp, torque matrix) write the 28-byte result.  Replaces
+//           Lanes stride over ligand beads (transform, grid interpolation,
+//           neighbour-list cell), quads of lanes walk the beads' lists, and
+//           the reference's bead-order reductions and a one-lane epilogue
+//           (force clamp, torque matrix) write the 28-byte result.  Replaces
 //           d_DOF2Pos, d_potForce, d_NLPotForce, d_reduce and h_finalReduce
 //           (model/*.cu, model/reduction.h:159-207) with one launch and no
 //           intermediate buffers.
-//  k_modes  one 256-thread workgroup per pose.  Phase A moves the deformed
-//           receptor into the ligand frame, scores it on the ligand grid and
-//           keeps its deformed coordinates in LDS; phase B scores the ligand on
-//           the receptor grid and runs the neighbour-list pairs, one pair per
-//           lane, against those LDS coordinates, folding the receptor reaction
-//           straight into the receptor mode gradients.  Semantics of
-//           service/CPUEnergyService6DModes.tpp:121-327.
+//  k_modes  one workgroup per pose.  Phase A moves the deformed receptor into
+//           the ligand frame and scores it on the ligand grid; phase B scores
+//           the ligand on the receptor grid and walks the lists against the
+//           receptor beads, deformed per pair from their mode rows, folding
+//           the receptor reaction straight into the receptor mode gradients.
+//           Semantics of service/CPUEnergyService6DModes.tpp:121-327.
 #include <algorithm>
 
 #include "device.h"
@@ -81,23 +79,22 @@ __global__ __launch_bounds__(256) void k_rigid(DProt rec, DProt lig, DGrid inner
         // P2: beads with a list, longest lists first.
         const unsigned qn = class_queue([&](unsigned k) { return s_n[k].x; }, m, s_q, s_cc, lane,
                                         kWave, wave_sync);
-        // P3: one bead per lane walks its list in the reference's order
-        // (NLPotForce); its sums are added to the bead's grid values as
+        // P3: one bead per quad of lanes walks its list in the reference's
+        // order (NLPotForce); its sums are added to the bead's grid values as
         // outLig[i] += fAcc.
-        for (unsigned q0 = 0; q0 < qn; q0 += kWave) {
-            if (q0 + lane < qn) {
-                const unsigned k = s_q[q0 + lane];
+        for (unsigned q0 = 0; q0 < qn; q0 += kWave / 4) {
+            if (q0 + (lane >> 2) < qn) {
+                const unsigned k = s_q[q0 + (lane >> 2)];
                 float4 x;
                 const V3 p = place(sc + k, x);
-                unsigned np = 0;
-                const float4 a = nl_walk(nl, par, tab, RecPosG{rec.pos}, RecTypeG{rec.type},
-                                         RecChargeG{rec.pos}, NoReaction{}, p.x, p.y, p.z,
-                                         lig.type[sc + k], x.w, s_n[k], &np);
-                listed += s_n[k].x;
-                inside += np;
-                float4 f = s_f[k];
-                f.x = f.x + a.x; f.y = f.y + a.y; f.z = f.z + a.z; f.w = f.w + a.w;
-                s_f[k] = f;
+                const float4 a = nl_walk_quad<0>(nl, par, tab, rec, nullptr, NoReaction{}, p.x, p.y,
+                                                 p.z, lig.type[sc + k], x.w, s_n[k], lane & 3u, inside);
+                if ((lane & 3u) == 0) {
+                    listed += s_n[k].x;
+                    float4 f = s_f[k];
+                    f.x = f.x + a.x; f.y = f.y + a.y; f.z = f.z + a.z; f.w = f.w + a.w;
+                    s_f[k] = f;
+                }
             }
         }
         wave_sync();
@@ -118,45 +115,6 @@ __global__ __launch_bounds__(256) void k_rigid(DProt rec, DProt lig, DGrid inner
         if (lane == 0) counts[pose] = make_uint2(listed, inside);
     }
 }
-
-// The deformed receptor position of bead j from its padded mode row (one or
-// two 16-byte loads), in the order of deform(): bit-identical coordinates.
-// The row {type, modes} is also left in `rowOut` (4 * ceil((3M + 1) / 4)
-// floats) for the pair's reaction, which then does not load it again.
-template <int MM>
-struct RecPosDeform {
-    const float4* pos;
-    const float4* modesT;
-    unsigned rowT, M;
-    const float* amp;
-    float* rowOut;
-    __device__ float3 operator()(unsigned j) const {
-        const float4 x = pos[j];
-        float yx = x.x, yy = x.y, yz = x.z;
-        if (MM > 0) {
-            constexpr int MA = MM > 0 ? MM : 1;
-            constexpr unsigned Q = (3 * MA + 4) / 4;
-            float mt[4 * Q];
-            const float4* row = modesT + (size_t)j * rowT;
-#pragma unroll
-            for (unsigned q = 0; q < Q; ++q) {
-                const float4 v = q < rowT ? row[q] : make_float4(0.f, 0.f, 0.f, 0.f);
-                mt[4 * q] = v.x; mt[4 * q + 1] = v.y; mt[4 * q + 2] = v.z; mt[4 * q + 3] = v.w;
-            }
-#pragma unroll
-            for (unsigned i = 0; i < 4 * Q; ++i) rowOut[i] = mt[i];
-#pragma unroll
-            for (unsigned m = 0; m < (unsigned)MA; ++m)
-                if (m < M) {
-                    const float a = amp[m];
-                    yx = yx + a * mt[3 * m + 1];
-                    yy = yy + a * mt[3 * m + 2];
-                    yz = yz + a * mt[3 * m + 3];
-                }
-        }
-        return make_float3(yx, yy, yz);
-    }
-};
 
 // reduceModeForce of the ligand (model/reduction_modes.h:28-57) for mode mm
 // over beads f[0..m) (LDS) of a super-chunk starting at bead sc, in bead
@@ -197,7 +155,7 @@ __device__ __forceinline__ float reduce_modes_ref(float red, const float* RT, co
 // (invertDOF, rotate_translate_deform), scored on the ligand grid, its force
 // rotated back (rotate_forces) and projected on the receptor modes.  Phase B:
 // the ligand in super-chunks of at most 256 * W beads, as k_rigid: grid term and list
-// cell per bead (P1), the class-ordered queue (P2), one bead per lane walking
+// cell per bead (P1), the class-ordered queue (P2), one bead per quad of lanes walking
 // its list in the reference's order against the deformed receptor (each
 // receptor bead deformed again from its mode row, so receptors of any size
 // need no LDS) with the reaction projected on the receptor modes (P3), and
@@ -232,7 +190,10 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
     constexpr int MA = MM > 0 ? MM : 1;
     float ampR[MA], ampL[MA];
 #pragma unroll
-    for (int m = 0; m < MA; ++m) { ampR[m] = d[6 + m]; ampL[m] = d[16 + m]; }
+    for (int m = 0; m < MA; ++m) {
+        ampR[m] = m < (int)rec.M ? d[6 + m] : 0.f;
+        ampL[m] = m < (int)lig.M ? d[16 + m] : 0.f;
+    }
     float t[6];
     pose_trig(d[3], d[4], d[5], lane, t);
     float R[9], RT[9], Rinv[9];
@@ -264,20 +225,11 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
     }
 
     // Phase B: ligand beads.
-    const float4* __restrict__ rpos = rec.pos;
-    const float4* __restrict__ rmodesT = rec.modesT;
-    const unsigned Mr = rec.M, rowT = rec.rowT;
-    // The walk takes one list entry at a time, so the reaction of a pair
-    // follows the deformation of the same receptor bead: its mode row is the
-    // one RecPosDeform left in rowBuf.
-    constexpr int kWalkBatch = 1;
-    static_assert(kWalkBatch == 1, "the reaction reads the row of the last deformed bead");
-    float rowBuf[4 * ((3 * MA + 4) / 4)];
-    auto reaction = [&](unsigned, float fx, float fy, float fz) {
-        const float* mt = rowBuf;
+    const unsigned Mr = rec.M;
+    auto reaction = [&](const RecBead<MM>& rb, float fx, float fy, float fz) {
 #pragma unroll
         for (unsigned m = 0; m < (unsigned)MM; ++m)
-            if (m < Mr) mR[m] -= fx * mt[3 * m + 1] + fy * mt[3 * m + 2] + fz * mt[3 * m + 3];
+            if (m < Mr) mR[m] -= fx * rb.row[3 * m + 1] + fy * rb.row[3 * m + 2] + fz * rb.row[3 * m + 3];
     };
     auto place = [&](unsigned i, float4& x) {
         x = lig.pos[i];
@@ -289,6 +241,9 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
         return p;
     };
     const unsigned Ml = lig.M, nL = lig.n;
+    auto place_row = [&](unsigned i, float4& x, unsigned& lt) {
+        return place_from_row<MM>(lig, i, ampL, R, tx, ty, tz, x, lt);
+    };
     float red = 0.f;  // wave 0: E, F, torque tensor; modeWave: ligand modes
     unsigned listed = 0, inside = 0;  // this lane's pair counts (counts != nullptr)
     const unsigned span = super_chunk(nL, kSuper);
@@ -306,21 +261,21 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
         const unsigned qn = class_queue([&](unsigned k) { return s_n[k].x; }, m, s_q, s_cc, tid,
                                         nthr, [] { __syncthreads(); });
         // P3
-        for (unsigned q0 = 0; q0 < qn; q0 += nthr) {
-            if (q0 + tid < qn) {
-                const unsigned k = s_q[q0 + tid];
+        for (unsigned q0 = 0, round = 0; q0 < qn; q0 += nthr / 4, ++round) {
+            const unsigned item = q0 + quad_group<W>(tid, round);
+            if (item < qn) {
+                const unsigned k = s_q[item];
                 float4 x;
-                const V3 p = place(sc + k, x);
-                unsigned np = 0;
-                const float4 a = nl_walk<kWalkBatch>(
-                    nl, par, tab, RecPosDeform<MM>{rpos, rmodesT, rowT, Mr, ampR, rowBuf},
-                    RecTypeG{rec.type}, RecChargeG{rpos}, reaction, p.x, p.y, p.z,
-                    lig.type[sc + k], x.w, s_n[k], &np);
-                listed += s_n[k].x;
-                inside += np;
-                float4 f = s_f[k];
-                f.x = f.x + a.x; f.y = f.y + a.y; f.z = f.z + a.z; f.w = f.w + a.w;
-                s_f[k] = f;
+                unsigned lt;
+                const V3 p = place_row(sc + k, x, lt);
+                const float4 a = nl_walk_quad<MM>(nl, par, tab, rec, ampR, reaction, p.x, p.y, p.z,
+                                                  lt, x.w, s_n[k], lane & 3u, inside);
+                if ((lane & 3u) == 0) {
+                    listed += s_n[k].x;
+                    float4 f = s_f[k];
+                    f.x = f.x + a.x; f.y = f.y + a.y; f.z = f.z + a.z; f.w = f.w + a.w;
+                    s_f[k] = f;
+                }
             }
         }
         __syncthreads();
@@ -481,9 +436,9 @@ __global__ void k_debug_sincosf(const float* x, unsigned n, float* sn, float* cs
     if (i < n) sincosf_libm(x[i], sn + i, cs + i);
 }
 
-__global__ void k_debug_plateau_ratio(float P2, unsigned n, float* ratio) {
+__global__ void k_debug_plateau_ratio(float P2, double c, unsigned n, float* ratio) {
     const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) ratio[i] = plateau_ratio(i, P2);
+    if (i < n) ratio[i] = plateau_ratio_fast(i, P2, c);
 }
 
 // Expands a [grid][z][y][x] float4 grid into voxel octets and, with octE, their
@@ -619,7 +574,8 @@ hipError_t launch_debug_sincosf(const float* x, unsigned n, float* sn, float* cs
 
 hipError_t launch_debug_plateau_ratio(float P2, unsigned n, float* ratio, hipStream_t s) {
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_debug_plateau_ratio, dim3((n + 255) / 256), dim3(256), 0, s, P2, n, ratio);
+    hipLaunchKernelGGL(k_debug_plateau_ratio, dim3((n + 255) / 256), dim3(256), 0, s, P2,
+                       1.0 / (10000.0 * (double)P2), n, ratio);
     return hipGetLastError();
 }
 

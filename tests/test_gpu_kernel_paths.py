@@ -57,3 +57,23 @@ def test_receptor_bead_with_a_non_finite_mode_is_skipped(ctx, W, O):
     ref = O.adjoint_kernel_order(wl)[:, :got.shape[1]].astype(np.float32)
     assert np.isfinite(got).all()
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("nl, mr, ml", [(1, 1, 0), (67, 0, 7), (257, 5, 2), (384, 3, 5), (1030, 10, 10)])
+def test_forward_walk_by_quads_is_the_reference_order(ctx, W, O, nl, mr, ml):
+    """The forward kernels over lists of every length, one to four waves per
+    pose, one to two super-chunks: the oracle's (the reference's) bits; the
+    receptor mode gradients, projected per pair, to 1e-5 of their norm."""
+    wl = W.make_workload("quads forward", 430 + nl, 250, nl, 20, mr, ml, shell=(8.0, 45.0))
+    hs = ctx.upload_workload(wl)
+    g, o = ctx.score_modes(hs, wl.dofs), O.score_modes(wl, nthreads=8)
+    keep = list(range(7)) + list(range(17, 27))
+    assert np.array_equal(g[:, keep].view(np.uint32), o[:, keep].view(np.uint32))
+    r, q = g[:, 7:7 + mr].astype(np.float64), o[:, 7:7 + mr].astype(np.float64)
+    fin = np.isfinite(q).all(axis=1)
+    assert np.array_equal(fin, np.isfinite(r).all(axis=1))
+    off = np.linalg.norm(r[fin] - q[fin], axis=1)
+    assert np.all(off <= 1e-5 * np.linalg.norm(q[fin], axis=1) + 1e-30)
+    d6 = np.ascontiguousarray(wl.dofs[:, :6])
+    rigid = ctx.score_rigid(hs, d6)
+    assert np.array_equal(rigid.view(np.uint32), O.score_rigid(wl, d6, nthreads=8).view(np.uint32))
