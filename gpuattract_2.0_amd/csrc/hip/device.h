@@ -48,12 +48,14 @@ struct DNL {
 // Protein (model/Protein.h:38-167): pos = {x, y, z, charge}.
 struct DProt {
     const float4* pos;
+    const float* soa;     // [x: ns][y: ns][z: ns][1: ns], zero beyond n: the bead-order reductions
     const unsigned* type;
     const unsigned* mtype;
     const float* modes;   // [c][m][n]: coalesced over beads
     const float4* modesT; // per bead one row {type bits, 3*M floats [m][c]}, padded to a float4 multiple
     const float* modeForce;
     unsigned n, M, rowT;  // rowT = float4 per modesT row
+    unsigned ns;          // n rounded up to 64
 };
 
 // Basis grids of the parameter derivative (attached to a DGrid of the same
@@ -910,35 +912,45 @@ __device__ __forceinline__ void wave_sync() {
 // order, one quantity per lane (lanes 0..12 of a wave): reducePotForce's E
 // and F (model/reduction.h:39-75) and reduceTorque's tensor sum of x_l * f_k
 // over the undeformed coordinates (:80-104) in lane 4 + 3k + l.  Each call
-// adds beads f[0..m) (float4 {fx, fy, fz, E}, LDS), whose undeformed
-// coordinates are pos[first..first+m), to the lane's running sum.
+// adds beads f[0..m) (float4 {fx, fy, fz, E}, LDS; zeros up to the next
+// multiple of kReduceStep), the body's beads first.., to the lane's running
+// sum.  Bound by the latency of a serial chain of adds: each lane reads its
+// own component's row (ones where there is no coordinate factor) 16 beads per
+// step, the next step's loads in flight.  With the modes' fold below (20,011
+// flexible poses 3000/800, 5 + 5 modes) 5.08 -> 4.35 ms, a call of 100 poses 254 ->
+// 190 us; 100,000 rigid poses (1000/300) 3.42 -> 3.18 ms, against eight beads
+// per step without the next step's loads.
+constexpr unsigned kReduceStep = 16;
 __device__ __forceinline__ float reduce_beads_ref(float red, unsigned lane, const float4* f,
-                                                  const float4* pos, unsigned first, unsigned m) {
+                                                  const DProt& lig, unsigned first, unsigned m) {
     if (lane >= 13u) return red;
     const unsigned fc = lane == 0 ? 3u : lane < 4u ? lane - 1u : (lane - 4u) / 3u;
-    const unsigned xc = lane < 4u ? 3u : (lane - 4u) % 3u;  // 3: no coordinate factor
-    const float* ff = reinterpret_cast<const float*>(f);
-    // The coordinates are the same for every lane and read-only: read through
-    // the constant address space, they are scalar loads (one per wave, from
-    // the scalar cache) rather than vector loads of one address.
-    typedef const __attribute__((address_space(4))) float* ConstF;
-    const ConstF pc = (ConstF)(const float*)(pos + first);
-    auto px = [pc](unsigned i) { return make_float4(pc[4 * i], pc[4 * i + 1], pc[4 * i + 2], pc[4 * i + 3]); };
-    auto coord = [xc](const float4& x) { return xc == 0u ? x.x : xc == 1u ? x.y : xc == 2u ? x.z : 1.f; };
-    unsigned k = 0;
-    // eight beads' loads are issued together; the sum stays sequential
-    for (; k + 8 <= m; k += 8) {
-        float4 xs[8];
-        float fv[8];
+    const unsigned xc = lane < 4u ? 3u : (lane - 4u) % 3u;
+    const float* ff = reinterpret_cast<const float*>(f) + fc;
+    const float4* xr = reinterpret_cast<const float4*>(lig.soa + (size_t)xc * lig.ns + first);
+    constexpr unsigned Q = kReduceStep / 4;
+    float4 x[Q];
+    float v[kReduceStep];
+    auto load = [&](unsigned k) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            xs[u] = px(k + u);
-            fv[u] = ff[4 * (k + u) + fc];
+        for (unsigned u = 0; u < Q; ++u) x[u] = xr[k / 4 + u];
+#pragma unroll
+        for (unsigned u = 0; u < kReduceStep; ++u) v[u] = ff[4 * (k + u)];
+    };
+    load(0);
+    for (unsigned k = 0; k < m; k += kReduceStep) {
+        float t[kReduceStep];
+#pragma unroll
+        for (unsigned u = 0; u < Q; ++u) {
+            t[4 * u] = x[u].x * v[4 * u];  // 1 * f = f exactly
+            t[4 * u + 1] = x[u].y * v[4 * u + 1];
+            t[4 * u + 2] = x[u].z * v[4 * u + 2];
+            t[4 * u + 3] = x[u].w * v[4 * u + 3];
         }
+        if (k + kReduceStep < m) load(k + kReduceStep);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) red += coord(xs[u]) * fv[u];  // 1 * f = f exactly
+        for (unsigned u = 0; u < kReduceStep; ++u) red += t[u];
     }
-    for (; k < m; ++k) red += coord(px(k)) * ff[4 * k + fc];
     return red;
 }
 

@@ -445,6 +445,17 @@ att_status att_upload_protein(att_ctx* c, const att_protein_desc* d, att_handle*
     if ((st = dev_copy(c, o.get(), pos.data(), n, &dpos)) != ATT_OK) return st;
     if ((st = dev_copy(c, o.get(), d->type, n, &dtype)) != ATT_OK) return st;
     if ((st = dev_copy(c, o.get(), d->mappedType, n, &dmtype)) != ATT_OK) return st;
+    // the same coordinates by component, and ones, padded with zeros
+    const unsigned ns = (n + 63u) & ~63u;
+    std::vector<float> soa4(4 * (size_t)ns, 0.f);
+    for (unsigned i = 0; i < n; ++i) {
+        for (unsigned k = 0; k < 3; ++k) soa4[(size_t)k * ns + i] = d->xyz[(size_t)k * n + i];
+        soa4[3 * (size_t)ns + i] = 1.f;
+    }
+    float* dsoa4;
+    if ((st = dev_copy(c, o.get(), soa4.data(), soa4.size(), &dsoa4)) != ATT_OK) return st;
+    o->d.soa = dsoa4;
+    o->d.ns = ns;
     o->d.pos = dpos;
     o->d.type = dtype;
     o->d.mtype = dmtype;

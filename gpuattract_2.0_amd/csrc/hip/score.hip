@@ -31,7 +31,7 @@ __host__ __device__ inline size_t rigid_wave_offset(unsigned tabSlots) {
     return (sizeof(att_pair_params) * (size_t)tabSlots + 15) & ~(size_t)15;
 }
 
-__global__ __launch_bounds__(256) void k_rigid(DProt rec, DProt lig, DGrid inner, DGrid outer,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_rigid(DProt rec, DProt lig, DGrid inner, DGrid outer,
                                                DNL nl, DPar par, const float* __restrict__ dofs,
                                                float* __restrict__ res, unsigned n,
                                                unsigned tabSlots,
@@ -69,6 +69,8 @@ __global__ __launch_bounds__(256) void k_rigid(DProt rec, DProt lig, DGrid inner
     for (unsigned sc = 0; sc < lig.n; sc += span) {
         const unsigned m = min(span, lig.n - sc);
         // P1: one bead per lane: rotate_translate, potForce, the list's cell.
+        const unsigned padded = (m + kReduceStep - 1) & ~(kReduceStep - 1);
+        if (m + lane < padded) s_f[m + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
         for (unsigned k = lane; k < m; k += kWave) {
             float4 x;
             const V3 p = place(sc + k, x);
@@ -99,7 +101,7 @@ __global__ __launch_bounds__(256) void k_rigid(DProt rec, DProt lig, DGrid inner
         }
         wave_sync();
         // P4: reducePotForce and reduceTorque, in bead order.
-        red = reduce_beads_ref(red, lane, s_f, lig.pos, sc, m);
+        red = reduce_beads_ref(red, lane, s_f, lig, sc, m);
         wave_sync();  // the super-chunk's arrays are reused
     }
     float o[7];
@@ -116,35 +118,44 @@ __global__ __launch_bounds__(256) void k_rigid(DProt rec, DProt lig, DGrid inner
     }
 }
 
-// reduceModeForce of the ligand (model/reduction_modes.h:28-57) for mode mm
-// over beads f[0..m) (LDS) of a super-chunk starting at bead sc, in bead
-// order: red -= (R^T f) . mode.  The mode vectors of eight beads are loaded
-// together.
+// reduceModeForce of the ligand (model/reduction_modes.h:28-57) over beads
+// f[0..m) (LDS) of a super-chunk starting at bead sc, in bead order: red -=
+// (R^T f) . mode, mode mm in lane mm of one wave.  The terms of 64 beads are
+// formed one bead per lane, left in `tile`, and subtracted by the modes'
+// lanes one after the other: only the subtractions are serial.
+template <int MM>
+struct ModeTile {
+    static constexpr unsigned kRow = 68;  // 64 terms, padded: the modes' rows in different banks
+    alignas(16) float t[(MM > 0 ? MM : 1) * kRow];
+};
+template <int MM>
 __device__ __forceinline__ float reduce_modes_ref(float red, const float* RT, const float4* f,
-                                                  const DProt& lig, unsigned mm, unsigned sc,
-                                                  unsigned m) {
-    const size_t nM = (size_t)lig.M * lig.n;
-    const float* mx = lig.modes + (size_t)mm * lig.n + sc;
-    unsigned k = 0;
-    for (; k + 8 <= m; k += 8) {
-        float ax[8], ay[8], az[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            ax[u] = mx[k + u];
-            ay[u] = mx[nM + k + u];
-            az[u] = mx[2 * nM + k + u];
+                                                  const DProt& lig, ModeTile<MM>& tile,
+                                                  unsigned lane, unsigned sc, unsigned m) {
+    for (unsigned c = 0; c < m; c += kWave) {
+        const unsigned k = c + lane;
+        BeadModes<MM> md;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (k < m) {
+            v = f[k];
+            load_modes(lig, sc + k, md);
         }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const float4 v = f[k + u];
-            const V3 fa = matvec(RT, v.x, v.y, v.z);
-            red -= fa.x * ax[u] + fa.y * ay[u] + fa.z * az[u];
-        }
-    }
-    for (; k < m; ++k) {
-        const float4 v = f[k];
         const V3 fa = matvec(RT, v.x, v.y, v.z);
-        red -= fa.x * mx[k] + fa.y * mx[nM + k] + fa.z * mx[2 * nM + k];
+#pragma unroll
+        for (unsigned mm = 0; mm < (unsigned)MM; ++mm)
+            if (mm < lig.M)
+                tile.t[mm * ModeTile<MM>::kRow + lane] =
+                    k < m ? fa.x * md.x[mm] + fa.y * md.y[mm] + fa.z * md.z[mm] : 0.f;
+        wave_sync();
+        if (lane < lig.M) {
+            const float4* row = reinterpret_cast<const float4*>(&tile.t[lane * ModeTile<MM>::kRow]);
+#pragma unroll
+            for (unsigned u = 0; u < kWave / 4; ++u) {
+                const float4 q = row[u];
+                red -= q.x; red -= q.y; red -= q.z; red -= q.w;
+            }
+        }
+        wave_sync();
     }
     return red;
 }
@@ -178,6 +189,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
     __shared__ unsigned s_cc[queue_counters(kSuper)];
     __shared__ float s_red[W][ATT_MODES_MAX];
     __shared__ float s_gl[ATT_MODES_MAX];
+    __shared__ ModeTile<MM> s_tile;
     __shared__ unsigned s_cnt[W][2];
     const PairTab tab = stage_table(par, s_tab);  // visible after phase B's first barrier
     if (blockIdx.x >= n) return;  // uniform per workgroup
@@ -240,16 +252,18 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
         p.x = p.x + tx; p.y = p.y + ty; p.z = p.z + tz;
         return p;
     };
-    const unsigned Ml = lig.M, nL = lig.n;
+    const unsigned nL = lig.n;
     auto place_row = [&](unsigned i, float4& x, unsigned& lt) {
         return place_from_row<MM>(lig, i, ampL, R, tx, ty, tz, x, lt);
     };
-    float red = 0.f;  // wave 0: E, F, torque tensor; modeWave: ligand modes
+    float red = 0.f, redM = 0.f;  // wave 0: E, F, torque tensor; modeWave: ligand modes
     unsigned listed = 0, inside = 0;  // this lane's pair counts (counts != nullptr)
     const unsigned span = super_chunk(nL, kSuper);
     for (unsigned sc = 0; sc < nL; sc += span) {
         const unsigned m = min(span, nL - sc);
         // P1
+        const unsigned padded = (m + kReduceStep - 1) & ~(kReduceStep - 1);
+        if (m + tid < padded) s_f[m + tid] = make_float4(0.f, 0.f, 0.f, 0.f);
         for (unsigned k = tid; k < m; k += nthr) {
             float4 x;
             const V3 p = place(sc + k, x);
@@ -281,9 +295,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
         __syncthreads();
         // P4: reducePotForce, reduceTorque and the ligand's reduceModeForce, in
         // bead order.
-        if (wave == 0) red = reduce_beads_ref(red, lane, s_f, lig.pos, sc, m);
-        const unsigned ml = W > 1 ? lane : lane - 13u;  // mode of this lane in modeWave
-        if (wave == modeWave && ml < Ml) red = reduce_modes_ref(red, RT, s_f, lig, ml, sc, m);
+        if (wave == 0) red = reduce_beads_ref(red, lane, s_f, lig, sc, m);
+        if (MM > 0 && wave == modeWave) redM = reduce_modes_ref<MM>(redM, RT, s_f, lig, s_tile, lane, sc, m);
         __syncthreads();  // the super-chunk's arrays are reused
     }
 
@@ -294,10 +307,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
 #pragma unroll
         for (int m = 0; m < ATT_MODES_MAX; ++m) s_red[wave][m] = m < MM ? mR[m < MM ? m : 0] : 0.f;
     }
-    if (wave == modeWave) {
-        const unsigned ml = W > 1 ? lane : lane - 13u;
-        if (ml < ATT_MODES_MAX) s_gl[ml] = red;
-    }
+    if (wave == modeWave && lane < ATT_MODES_MAX) s_gl[lane] = redM;
     if (counts) {
         listed = wave_sum_u(listed);
         inside = wave_sum_u(inside);
