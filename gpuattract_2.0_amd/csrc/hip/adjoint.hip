@@ -24,6 +24,7 @@
 // written once per workgroup, then k_pgrad_groups and k_pgrad_reduce add the
 // per-workgroup rows in a fixed order.
 #include <algorithm>
+#include <type_traits>
 
 #include "device.h"
 #include "internal.h"
@@ -262,12 +263,10 @@ __device__ __forceinline__ void adj_walk(const PairDesc& P, const PairTab& tab,
     const float ddP = nl.ddP[par.dielec];
     eAcc = 0.f;
     gAcc = make_float3(0.f, 0.f, 0.f);
-    unsigned nxt = lst[min(s, last)];
+    RecStream<MM> recs(P.rec, lst, s, last);
     for (unsigned jj = 0; jj < d.x; jj += 4) {
-        const unsigned j = nxt;
-        nxt = lst[min(jj + 4 + s, last)];  // next step's entry in flight
         RecBead<MM> rb;
-        rb.load(P.rec, j, ampR);
+        recs.next(P.rec, lst, jj + s, last, ampR, rb);
         const unsigned rt = rb.type;
         const float ddx = px - rb.x, ddy = py - rb.y, ddz = pz - rb.z;
         const float dr2 = ddx * ddx + ddy * ddy + ddz * ddz;
@@ -328,22 +327,28 @@ __device__ __forceinline__ void adj_walk(const PairDesc& P, const PairTab& tab,
 }
 
 // The workgroup-shared state of one pose (static LDS), WAVES waves per pose:
-// the ligand is taken in super-chunks of 256 beads per wave (26 B of LDS per
-// bead: four workgroups of two waves, or eight of one, per CU).
-template <int WAVES>
+// the ligand is taken in super-chunks (LDS for eight workgroups of two waves,
+// or sixteen of one, per CU).
+template <int WAVES, int MM>
 struct PoseLDS {
-    static constexpr unsigned kSuper = 256u * WAVES;
+    // Beads per wave of a super-chunk: 256 with modes (26 B each); without, 384
+    // (18 B: the list's cell is found again at the walk), so that the ligands
+    // scored by one wave are one super-chunk, with fewer walk steps
+    // (1000/300 beads: 45 against 57).
+    static constexpr unsigned kChunks = MM > 0 ? 4 : 6;
+    static constexpr unsigned kSuper = 64u * kChunks * WAVES;
+    using Classes = std::conditional_t<(MM > 0), Classes9, Classes16>;
     float4 g[kSuper];     // per bead: dE/dp (grid, then minus the pair forces); energy
-    uint2 nlc[kSuper];    // neighbour-list {count, start}
+    uint2 nlc[MM > 0 ? kSuper : 1];  // neighbour-list {count, start}
     unsigned short q[kSuper];
-    unsigned cc[queue_counters(kSuper)];
-    float red[WAVES][ATT_MODES_MAX];
+    unsigned cc[queue_counters<Classes>(kSuper)];
+    float red[WAVES][MM > 0 ? ATT_MODES_MAX : 1];
     unsigned cnt[WAVES][2];
     float e;
 };
 
 // Adjoint of one pose by one workgroup of WAVES waves, the ligand in
-// super-chunks of equal size, at most PoseLDS<WAVES>::kSuper beads (super_chunk):
+// super-chunks of equal size, at most PoseLDS<WAVES, MM>::kSuper beads (super_chunk):
 //  P1  every bead: transform, grid term with its exact gradient (and the
 //      basis-grid parameter derivatives), neighbour-list cell;
 //  P2  beads with a list, longest lists first (class_queue);
@@ -354,7 +359,7 @@ struct PoseLDS {
 //      by wave 0, bead k on lane k % 64, lane sums reduced by a butterfly.
 // Every sum has a fixed order: results do not depend on timing.
 template <int MM, int WAVES, int PG>
-__device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, PoseLDS<WAVES>& S,
+__device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, PoseLDS<WAVES, MM>& S,
                                              const PairTab& tab, float* s_pg,
                                              size_t recBase) {
     const DProt& lig = P.lig;
@@ -366,20 +371,22 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
     const unsigned Ml = MM > 0 ? lig.M : 0, Mr = MM > 0 ? P.rec.M : 0;
     __syncthreads();  // LDS of the previous pose is no longer read
     const float* d = P.dofs + (size_t)P.dofStride * pose;
-    const float tx = d[0], ty = d[1], tz = d[2];
+    const float tx = uniform(d[0]), ty = uniform(d[1]), tz = uniform(d[2]);
     const float wp = P.wts ? P.wts[pose] : 1.f;
     const PGrad pg{PG != kPgNone ? s_pg + wave * 3 * par.T * par.T : nullptr, tab, par.T, wp,
                    P.recKey, P.recPos4, P.recPos3, P.recCellsIn, P.recInvalid};
     float ampR[MA], ampL[MA];
 #pragma unroll
     for (int m = 0; m < MA; ++m) {
-        ampR[m] = MM > 0 && m < (int)Mr ? d[6 + m] : 0.f;
-        ampL[m] = MM > 0 && m < (int)Ml ? d[16 + m] : 0.f;
+        ampR[m] = MM > 0 && m < (int)Mr ? uniform(d[6 + m]) : 0.f;
+        ampL[m] = MM > 0 && m < (int)Ml ? uniform(d[16 + m]) : 0.f;
     }
     float t[6];
     pose_trig(d[3], d[4], d[5], lane, t);
     float R[9];
     rotmat_from_trig(t[0], t[1], t[2], t[3], t[4], t[5], R);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) R[k] = uniform(R[k]);
     // wave 0: dE/dt (3), sum G (x) x~ (9), ligand modes; all waves: receptor modes
     float acc[12], gR[MA], gL[MA];
 #pragma unroll
@@ -406,11 +413,12 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
         return place_from_row<MM>(lig, i, ampL, R, tx, ty, tz, x, lt);
     };
 
-    const unsigned span = super_chunk(lig.n, PoseLDS<WAVES>::kSuper);
+    const unsigned span = super_chunk(lig.n, PoseLDS<WAVES, MM>::kSuper);
     for (unsigned sc = 0; sc < lig.n; sc += span) {
         const unsigned m = min(span, lig.n - sc);
         // P1
-        for (unsigned k = tid; k < m; k += nthr) {
+        unsigned classes = 0;
+        for (unsigned k = tid, u = 0; k < m; k += nthr, ++u) {
             float4 x;
             const V3 p = place(sc + k, x);
             float3 G;
@@ -418,12 +426,15 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
                                           lig.mtype[sc + k], lig.type[sc + k], x.w, G, pg,
                                           recBase + sc + k);
             S.g[k] = make_float4(G.x, G.y, G.z, eg);
-            S.nlc[k] = nl_cell(P.nl, p.x, p.y, p.z, lig.type[sc + k]);
+            const uint2 cell = nl_cell(P.nl, p.x, p.y, p.z, lig.type[sc + k]);
+            if (MM > 0) S.nlc[k] = cell;
+            classes = pack_class<typename PoseLDS<WAVES, MM>::Classes>(classes, u, cell.x);
         }
         __syncthreads();
         // P2
-        const unsigned qn = class_queue([&](unsigned k) { return S.nlc[k].x; }, m, S.q, S.cc, tid,
-                                        nthr, [] { __syncthreads(); });
+        const unsigned qn = class_queue<typename PoseLDS<WAVES, MM>::Classes, WAVES,
+                                        PoseLDS<WAVES, MM>::kChunks>(classes, m, S.q, S.cc, tid,
+                                                                     [] { __syncthreads(); });
         // P3
         for (unsigned q0 = 0; q0 < qn; q0 += nthr) {
             for (unsigned sub = 0; sub < 4; ++sub) {
@@ -441,7 +452,7 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
                     float3 gAcc;
 #pragma unroll
                     for (int m = 0; m < MA; ++m) g4[m] = MM > 0 ? __shfl(gR[m], (lane & ~3u) | sub) : 0.f;
-                    const uint2 nlc = S.nlc[k];
+                    const uint2 nlc = MM > 0 ? S.nlc[k] : nl_cell(P.nl, p.x, p.y, p.z, lt);
                     adj_walk<MM, PG>(P, tab, pg, p.x, p.y, p.z, x.w, lt, nlc, lane & 3u, ampR, g4,
                                      eAcc, gAcc, inside);
 #pragma unroll
@@ -513,7 +524,7 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
     }
     if (lane == 0) {
 #pragma unroll
-        for (int m = 0; m < ATT_MODES_MAX; ++m) S.red[wave][m] = m < MA ? gR[m < MA ? m : 0] : 0.f;
+        for (int m = 0; MM > 0 && m < ATT_MODES_MAX; ++m) S.red[wave][m] = m < MA ? gR[m < MA ? m : 0] : 0.f;
     }
     if (tid == eThread) S.e = esum;
     if (P.counts) {
@@ -537,8 +548,8 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
         if (P.outStride >= 27)
 #pragma unroll
             for (unsigned m = 0; m < ATT_MODES_MAX; ++m) {
-                float s = S.red[0][m];
-                for (unsigned w = 1; w < (unsigned)WAVES; ++w) s += S.red[w][m];
+                float s = MM > 0 ? S.red[0][m] : 0.f;
+                for (unsigned w = 1; MM > 0 && w < (unsigned)WAVES; ++w) s += S.red[w][m];
                 o[7 + m] = m < Mr ? wp * s : 0.f;
                 o[17 + m] = m < Ml ? wp * gL[m < MA ? m : 0] : 0.f;
             }
@@ -560,7 +571,7 @@ template <int MM, int WAVES, int PG>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(adjoint_waves_per_simd<MM>()))) void k_adjoint(
     PairDesc P, float* __restrict__ pgPartial) {
     extern __shared__ att_pair_params s_dyn[];
-    __shared__ PoseLDS<WAVES> S;
+    __shared__ PoseLDS<WAVES, MM> S;
     char* dyn = reinterpret_cast<char*>(s_dyn);
     const PairTab tab = stage_table(P.par, s_dyn);
     // Parameter derivatives: one LDS slice per wave, so that every slice is
@@ -606,7 +617,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(adjo
     const PairDesc* __restrict__ pairs, const BatchTile* __restrict__ tiles,
     const unsigned* __restrict__ queueStart, unsigned* __restrict__ counters) {
     extern __shared__ att_pair_params s_dyn[];
-    __shared__ PoseLDS<WAVES> S;
+    __shared__ PoseLDS<WAVES, MM> S;
     __shared__ unsigned s_tile;
     unsigned cur = 0xFFFFFFFFu;
     PairTab tab{nullptr, false};
@@ -713,9 +724,9 @@ size_t adjoint_lds_bytes(const DProt& rec, const DProt& lig, const DPar& par, bo
 
 size_t adjoint_static_lds(int waves) {
     switch (waves) {
-        case 1: return sizeof(PoseLDS<1>) + 16;
-        case 2: return sizeof(PoseLDS<2>) + 16;
-        default: return sizeof(PoseLDS<4>) + 16;
+        case 1: return std::max(sizeof(PoseLDS<1, 0>), sizeof(PoseLDS<1, ATT_MODES_MAX>)) + 16;
+        case 2: return std::max(sizeof(PoseLDS<2, 0>), sizeof(PoseLDS<2, ATT_MODES_MAX>)) + 16;
+        default: return std::max(sizeof(PoseLDS<4, 0>), sizeof(PoseLDS<4, ATT_MODES_MAX>)) + 16;
     }
 }
 

@@ -146,6 +146,13 @@ __device__ __forceinline__ void torque_reduce(float cSSI, float cPHI, float sSSI
     out[0] = r0; out[1] = r1; out[2] = r2;
 }
 
+// A value that is the same on every lane, in a scalar register: a pose's
+// rotation, translation and amplitudes would otherwise hold some 30 vector
+// registers through the walks (and spill: 96 -> 0 B per lane in the 5-mode adjoint).
+__device__ __forceinline__ float uniform(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+
 // The six trig values of a pose, evaluated once per wave: lanes 0..2 take
 // sin and cos of (ssi, phi, rot) with the C library's single-precision values
 // (sincosf_libm, as the reference's std::sin/std::cos(float)), then every lane
@@ -153,12 +160,13 @@ __device__ __forceinline__ void torque_reduce(float cSSI, float cPHI, float sSSI
 __device__ __forceinline__ void pose_trig(float phi, float ssi, float rot, int lane, float* t) {
     float c = 0.f, s = 0.f;
     if (lane < 3) sincosf_libm(lane == 0 ? ssi : lane == 1 ? phi : rot, &s, &c);
-    t[0] = __shfl(c, 0);  // cSSI
-    t[1] = __shfl(c, 1);  // cPHI
-    t[2] = __shfl(s, 0);  // sSSI
-    t[3] = __shfl(s, 1);  // sPHI
-    t[4] = __shfl(c, 2);  // cROT
-    t[5] = __shfl(s, 2);  // sROT
+    auto at = [](float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); };
+    t[0] = at(c, 0);  // cSSI
+    t[1] = at(c, 1);  // cPHI
+    t[2] = at(s, 0);  // sSSI
+    t[3] = at(s, 1);  // sPHI
+    t[4] = at(c, 2);  // cROT
+    t[5] = at(s, 2);  // sROT
 }
 
 // IntrplGrid::outOfBounds_byPos (model/IntrplGrid.h:113-117).
@@ -515,62 +523,115 @@ __device__ __forceinline__ bool nl_bead(const DNL& nl, const DPar& par,
 }
 
 // Beads whose neighbour lists are walked one per quad are ordered by list
-// length: nine classes, longest first (>= 64, 48, 36, 28, 22, 16, 11, 6, 1
-// pairs), bead order inside a class, so that the quads of a wave walk lists of
-// similar length.  The class of a bead with cnt > 0 listed neighbours:
-constexpr unsigned kQueueClasses = 9;
-__device__ __forceinline__ unsigned queue_class(unsigned cnt) {
-    return (unsigned)(cnt < 64u) + (cnt < 48u) + (cnt < 36u) + (cnt < 28u) + (cnt < 22u) +
-           (cnt < 16u) + (cnt < 11u) + (cnt < 6u);
-}
+// length, longest first, bead order inside a class, so that the quads of a
+// wave walk lists of similar length.  Nine classes (>= 64, 48, 36, 28, 22, 16,
+// 11, 6, 1 pairs) where the order decides which thread sums a bead's receptor
+// mode gradients; sixteen by the number of four-entry steps (>= 19, 18, 16,
+// 14, 12, then one class per number) where it decides no bit or only the last: the rigid kernels,
+// whose walks take 6 % fewer steps for 7 ballots more per 64 beads (1000/300).
+// The class of a bead with cnt > 0 listed neighbours:
+struct Classes9 {
+    static constexpr unsigned kNum = 9;
+    static __device__ __forceinline__ unsigned of(unsigned cnt) {
+        return (unsigned)(cnt < 64u) + (cnt < 48u) + (cnt < 36u) + (cnt < 28u) + (cnt < 22u) +
+               (cnt < 16u) + (cnt < 11u) + (cnt < 6u);
+    }
+};
+struct Classes16 {
+    static constexpr unsigned kNum = 16;
+    static __device__ __forceinline__ unsigned of(unsigned cnt) {
+        const unsigned steps = (min(cnt, 76u) + 3u) / 4u;
+        return steps <= 12u ? 16u - steps : (21u - steps) / 2u - (steps == 19u ? 1u : 0u);
+    }
+};
+constexpr unsigned kQueueChunks = 6;  // chunks of 64 beads per wave at most (5 bits each, packed)
+template <class Classes>
 __host__ __device__ constexpr unsigned queue_counters(unsigned beads) {
-    return kQueueClasses * ((beads + 63) / 64) + 1;
+    return Classes::kNum * ((beads + 63) / 64) + 1;
 }
 
-// The listed beads (cnt(k) > 0) among beads 0..m-1 of a super-chunk, in the
-// class order above, into s_q; returns their number.  Run by nthr threads (a
-// multiple of 64, thread tid) with sync() a barrier over them; s_cc holds
-// queue_counters(m) counters: per (class, chunk of 64 beads) the number of
-// listed beads, then their exclusive prefix in (class, chunk) order.
-template <class Cnt, class Sync>
-__device__ __forceinline__ unsigned class_queue(Cnt cnt, unsigned m, unsigned short* s_q,
-                                                unsigned* s_cc, unsigned tid, unsigned nthr,
-                                                Sync sync) {
-    const unsigned lane = tid & (kWave - 1), wv = tid / kWave, nw = nthr / kWave;
+// The classes of a thread's beads of a super-chunk (beads tid, tid + threads,
+// ...: at most kQueueChunks), five bits each.
+template <class Classes>
+__device__ __forceinline__ unsigned pack_class(unsigned packed, unsigned u, unsigned cnt) {
+    return packed | (cnt ? Classes::of(cnt) : Classes::kNum) << (5 * u);
+}
+
+// Inclusive prefix sum over the 64 lanes of a wave (DPP: row shifts of 1, 2, 4
+// and 8 lanes, then the row totals broadcast).
+__device__ __forceinline__ unsigned wave_scan(unsigned v) {
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);
+    v += (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+
+// The listed beads among beads 0..m-1 of a super-chunk (m <= 64 * CHUNKS per
+// wave), in class order, into s_q; returns their number.  Run by WAVES waves
+// with sync() a barrier over them; `classes` are each thread's (pack_class);
+// s_cc holds queue_counters(m) counters: per (class, chunk of 64 beads) the
+// number of listed beads, then their exclusive prefix in (class, chunk) order.
+// Bound by latency (14k cycles per super-chunk with a serial scan by one
+// thread, 5k so): one set of ballots gives every bead its rank among the
+// chunk's beads of its class, and one wave scans the counters.
+template <class Classes, int WAVES, unsigned CHUNKS, class Sync>
+__device__ __forceinline__ unsigned class_queue(unsigned classes, unsigned m, unsigned short* s_q,
+                                                unsigned* s_cc, unsigned tid, Sync sync) {
+    constexpr unsigned K = Classes::kNum;
+    static_assert(CHUNKS <= kQueueChunks, "packed classes");
+    const unsigned lane = tid & (kWave - 1), wv = tid / kWave;
     const unsigned chunks = (m + kWave - 1) / kWave;
-    const unsigned long long below = (1ull << lane) - 1ull;
-    for (unsigned ch = wv; ch < chunks; ch += nw) {
-        const unsigned k = ch * kWave + lane;
-        const unsigned c = k < m ? cnt(k) : 0u;
-        const unsigned cls = c ? queue_class(c) : kQueueClasses;
+    unsigned rank[CHUNKS];
 #pragma unroll
-        for (unsigned q = 0; q < kQueueClasses; ++q) {
+    for (unsigned u = 0; u < CHUNKS; ++u) {
+        rank[u] = 0;
+        const unsigned ch = wv + u * WAVES;
+        if (ch >= chunks) continue;  // uniform per wave
+        const unsigned cls = ch * kWave + lane < m ? (classes >> (5 * u)) & 31u : K;
+        unsigned total = 0;
+#pragma unroll
+        for (unsigned q = 0; q < K; ++q) {
             const unsigned long long b = __ballot(cls == q);
-            if (lane == 0) s_cc[q * chunks + ch] = (unsigned)__popcll(b);
+            const unsigned below = __builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32),
+                                                             __builtin_amdgcn_mbcnt_lo((unsigned)b, 0u));
+            rank[u] = cls == q ? below : rank[u];
+            total = lane == q ? (unsigned)__popcll(b) : total;
         }
+        if (lane < K) s_cc[lane * chunks + ch] = total;
     }
     sync();
-    if (tid == 0) {
-        unsigned sum = 0;
-        for (unsigned e = 0; e < kQueueClasses * chunks; ++e) {
-            const unsigned v = s_cc[e];
-            s_cc[e] = sum;
-            sum += v;
+    const unsigned entries = K * chunks;
+    if (wv == 0) {
+        constexpr unsigned kPer = (K * CHUNKS * WAVES + kWave - 1) / kWave;  // consecutive, per lane
+        unsigned v[kPer], sum = 0;
+#pragma unroll
+        for (unsigned i = 0; i < kPer; ++i) {
+            const unsigned e = lane * kPer + i;
+            v[i] = e < entries ? s_cc[e] : 0u;
+            sum += v[i];
         }
-        s_cc[kQueueClasses * chunks] = sum;
+        const unsigned incl = wave_scan(sum);
+        unsigned run = incl - sum;
+#pragma unroll
+        for (unsigned i = 0; i < kPer; ++i) {
+            const unsigned e = lane * kPer + i;
+            if (e < entries) s_cc[e] = run;
+            run += v[i];
+        }
+        if (lane == kWave - 1) s_cc[entries] = incl;
     }
     sync();
-    for (unsigned ch = wv; ch < chunks; ch += nw) {
-        const unsigned k = ch * kWave + lane;
-        const unsigned c = k < m ? cnt(k) : 0u;
-        const unsigned cls = c ? queue_class(c) : kQueueClasses;
 #pragma unroll
-        for (unsigned q = 0; q < kQueueClasses; ++q) {
-            const unsigned long long b = __ballot(cls == q);
-            if (cls == q) s_q[s_cc[q * chunks + ch] + (unsigned)__popcll(b & below)] = (unsigned short)k;
-        }
+    for (unsigned u = 0; u < CHUNKS; ++u) {
+        const unsigned ch = wv + u * WAVES;
+        if (ch >= chunks) continue;
+        const unsigned cls = ch * kWave + lane < m ? (classes >> (5 * u)) & 31u : K;
+        if (cls < K) s_q[s_cc[cls * chunks + ch] + rank[u]] = (unsigned short)(ch * kWave + lane);
     }
-    const unsigned total = s_cc[kQueueClasses * chunks];
+    const unsigned total = s_cc[entries];
     sync();
     return total;
 }
@@ -747,17 +808,46 @@ struct RecBead {
     __device__ __forceinline__ void load(const DProt& rec, unsigned j, const float* amp) {
         const float4 p = rec.pos[j];
         x = p.x; y = p.y; z = p.z; q = p.w;
-        if constexpr (MM > 0) {
-            load_row<MM>(rec, j, row);
-            type = __float_as_uint(row[0]);
+        load_row<MM>(rec, j, row);
+        type = __float_as_uint(row[0]);
 #pragma unroll
-            for (unsigned m = 0; m < (unsigned)MM; ++m) {
-                x = x + amp[m] * row[3 * m + 1];
-                y = y + amp[m] * row[3 * m + 2];
-                z = z + amp[m] * row[3 * m + 3];
-            }
-        } else {
+        for (unsigned m = 0; m < (unsigned)MM; ++m) {
+            x = x + amp[m] * row[3 * m + 1];
+            y = y + amp[m] * row[3 * m + 2];
+            z = z + amp[m] * row[3 * m + 3];
+        }
+    }
+};
+
+// The receptor beads of a list, every fourth entry from entry `at` on (clamped
+// to the last one).  With modes the next entry's index is loaded one step
+// ahead; without, the next bead itself and the index after it: five registers,
+// 3 % of the rigid kernels.  (With modes the row ahead is 20 or 36 registers,
+// and its spills cost more than the latency: 3 and 9 % slower.)
+template <int MM>
+struct RecStream {
+    unsigned idx, type;
+    float4 p;
+    __device__ __forceinline__ RecStream(const DProt& rec, const uint32_t* lst, unsigned at, unsigned last) {
+        idx = lst[min(at, last)];
+        if constexpr (MM == 0) {
+            p = rec.pos[idx];
+            type = rec.type[idx];
+            idx = lst[min(at + 4, last)];
+        }
+    }
+    __device__ __forceinline__ void next(const DProt& rec, const uint32_t* lst, unsigned at,
+                                         unsigned last, const float* amp, RecBead<MM>& rb) {
+        const unsigned j = idx;
+        if constexpr (MM == 0) {
+            rb.x = p.x; rb.y = p.y; rb.z = p.z; rb.q = p.w;
+            rb.type = type;
+            p = rec.pos[j];
             type = rec.type[j];
+            idx = lst[min(at + 8, last)];
+        } else {
+            idx = lst[min(at + 4, last)];
+            rb.load(rec, j, amp);
         }
     }
 };
@@ -781,12 +871,10 @@ __device__ __forceinline__ float4 nl_walk_quad(const DNL& nl, const DPar& par, c
     float fx = 0.f, fy = 0.f, fz = 0.f, e = 0.f;
     const unsigned lt1 = ligType - 1, last = d.x - 1;
     const uint32_t* lst = nl.list + d.y;
-    unsigned nxt = lst[min(s, last)];
+    RecStream<MM> recs(rec, lst, s, last);
     for (unsigned jj = 0; jj < d.x; jj += 4) {
-        const unsigned j = nxt;
-        nxt = lst[min(jj + 4 + s, last)];  // next step's entry in flight
         RecBead<MM> rb;
-        rb.load(rec, j, ampR);
+        recs.next(rec, lst, jj + s, last, ampR, rb);
         const float ddx = px - rb.x, ddy = py - rb.y, ddz = pz - rb.z;
         const float dr2 = ddx * ddx + ddy * ddy + ddz * ddz;
         const bool in = jj + s < d.x && dr2 <= nl.P2 && rb.type - 1u < par.T;

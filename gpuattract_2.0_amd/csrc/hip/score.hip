@@ -22,11 +22,10 @@
 namespace att {
 
 // Beads per super-chunk of k_rigid (per wave) and their LDS: bead force and
-// energy (float4), neighbour-list {count, start} (uint2), the class-ordered
-// queue (u16) and its counters.
-constexpr unsigned kRigidSuper = 256;
+// energy (float4), the class-ordered queue (u16) and its counters.
+constexpr unsigned kRigidSuper = 64 * kQueueChunks;
 constexpr size_t kRigidWaveBytes =
-    (kRigidSuper * (16 + 8 + 2) + sizeof(unsigned) * queue_counters(kRigidSuper) + 15) & ~(size_t)15;
+    (kRigidSuper * (16 + 2) + sizeof(unsigned) * queue_counters<Classes16>(kRigidSuper) + 15) & ~(size_t)15;
 __host__ __device__ inline size_t rigid_wave_offset(unsigned tabSlots) {
     return (sizeof(att_pair_params) * (size_t)tabSlots + 15) & ~(size_t)15;
 }
@@ -44,19 +43,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const unsigned wave = threadIdx.x / kWave;
     char* wb = reinterpret_cast<char*>(s_tab) + rigid_wave_offset(tabSlots) + wave * kRigidWaveBytes;
     float4* s_f = reinterpret_cast<float4*>(wb);
-    uint2* s_n = reinterpret_cast<uint2*>(s_f + kRigidSuper);
-    unsigned short* s_q = reinterpret_cast<unsigned short*>(s_n + kRigidSuper);
+    unsigned short* s_q = reinterpret_cast<unsigned short*>(s_f + kRigidSuper);
     unsigned* s_cc = reinterpret_cast<unsigned*>(s_q + kRigidSuper);
     const unsigned wg = order ? xcd_slot(blockIdx.x, gridDim.x) : blockIdx.x;
     const unsigned slot = wg * (blockDim.x / kWave) + wave;
     if (slot >= n) return;  // uniform per wave; no workgroup barrier follows
     const unsigned pose = order ? order[slot] : slot;
     const float* d = dofs + 6 * (size_t)pose;
-    const float tx = d[0], ty = d[1], tz = d[2];
+    const float tx = uniform(d[0]), ty = uniform(d[1]), tz = uniform(d[2]);
     float t[6];
     pose_trig(d[3], d[4], d[5], lane, t);
     float R[9];
     rotmat_from_trig(t[0], t[1], t[2], t[3], t[4], t[5], R);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) R[k] = uniform(R[k]);
     auto place = [&](unsigned i, float4& x) {
         x = lig.pos[i];
         V3 p = matvec(R, x.x, x.y, x.z);
@@ -71,16 +71,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         // P1: one bead per lane: rotate_translate, potForce, the list's cell.
         const unsigned padded = (m + kReduceStep - 1) & ~(kReduceStep - 1);
         if (m + lane < padded) s_f[m + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (unsigned k = lane; k < m; k += kWave) {
+        unsigned classes = 0;
+        for (unsigned k = lane, u = 0; k < m; k += kWave, ++u) {
             float4 x;
             const V3 p = place(sc + k, x);
             s_f[k] = pot_bead(inner, outer, p.x, p.y, p.z, lig.mtype[sc + k], x.w, nullptr);
-            s_n[k] = nl_cell(nl, p.x, p.y, p.z, lig.type[sc + k]);
+            classes = pack_class<Classes16>(classes, u, nl_cell(nl, p.x, p.y, p.z, lig.type[sc + k]).x);
         }
         wave_sync();
         // P2: beads with a list, longest lists first.
-        const unsigned qn = class_queue([&](unsigned k) { return s_n[k].x; }, m, s_q, s_cc, lane,
-                                        kWave, wave_sync);
+        const unsigned qn = class_queue<Classes16, 1, kQueueChunks>(classes, m, s_q, s_cc, lane, wave_sync);
         // P3: one bead per quad of lanes walks its list in the reference's
         // order (NLPotForce); its sums are added to the bead's grid values as
         // outLig[i] += fAcc.
@@ -89,10 +89,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 const unsigned k = s_q[q0 + (lane >> 2)];
                 float4 x;
                 const V3 p = place(sc + k, x);
+                const unsigned lt = lig.type[sc + k];
+                const uint2 cell = nl_cell(nl, p.x, p.y, p.z, lt);
                 const float4 a = nl_walk_quad<0>(nl, par, tab, rec, nullptr, NoReaction{}, p.x, p.y,
-                                                 p.z, lig.type[sc + k], x.w, s_n[k], lane & 3u, inside);
+                                                 p.z, lt, x.w, cell, lane & 3u, inside);
                 if ((lane & 3u) == 0) {
-                    listed += s_n[k].x;
+                    listed += cell.x;
                     float4 f = s_f[k];
                     f.x = f.x + a.x; f.y = f.y + a.y; f.z = f.z + a.z; f.w = f.w + a.w;
                     s_f[k] = f;
@@ -186,7 +188,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
     __shared__ float4 s_f[kSuper];
     __shared__ uint2 s_n[kSuper];
     __shared__ unsigned short s_q[kSuper];
-    __shared__ unsigned s_cc[queue_counters(kSuper)];
+    __shared__ unsigned s_cc[queue_counters<Classes16>(kSuper)];
     __shared__ float s_red[W][ATT_MODES_MAX];
     __shared__ float s_gl[ATT_MODES_MAX];
     __shared__ ModeTile<MM> s_tile;
@@ -198,25 +200,30 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
     constexpr unsigned nthr = 64u * W;
     constexpr unsigned modeWave = W - 1;  // runs the ligand's reduceModeForce
     const float* d = dofs + 26 * (size_t)pose;
-    const float tx = d[0], ty = d[1], tz = d[2];
+    const float tx = uniform(d[0]), ty = uniform(d[1]), tz = uniform(d[2]);
     constexpr int MA = MM > 0 ? MM : 1;
     float ampR[MA], ampL[MA];
 #pragma unroll
     for (int m = 0; m < MA; ++m) {
-        ampR[m] = m < (int)rec.M ? d[6 + m] : 0.f;
-        ampL[m] = m < (int)lig.M ? d[16 + m] : 0.f;
+        ampR[m] = m < (int)rec.M ? uniform(d[6 + m]) : 0.f;
+        ampL[m] = m < (int)lig.M ? uniform(d[16 + m]) : 0.f;
     }
     float t[6];
     pose_trig(d[3], d[4], d[5], lane, t);
     float R[9], RT[9], Rinv[9];
     rotmat_from_trig(t[0], t[1], t[2], t[3], t[4], t[5], R);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) R[k] = uniform(R[k]);
     RT[0] = R[0]; RT[1] = R[3]; RT[2] = R[6];
     RT[3] = R[1]; RT[4] = R[4]; RT[5] = R[7];
     RT[6] = R[2]; RT[7] = R[5]; RT[8] = R[8];
     // invertDOF (model/transform_modes.h:26-41): rotation R(-ang) (cos even,
     // sin odd), translation R^T (-pos).
     rotmat_from_trig(t[0], t[1], -t[2], -t[3], t[4], -t[5], Rinv);
-    const V3 pinv = matvec(RT, -tx, -ty, -tz);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) Rinv[k] = uniform(Rinv[k]);
+    V3 pinv = matvec(RT, -tx, -ty, -tz);
+    pinv.x = uniform(pinv.x); pinv.y = uniform(pinv.y); pinv.z = uniform(pinv.z);
 
     float mR[MA];
 #pragma unroll
@@ -264,16 +271,18 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
         // P1
         const unsigned padded = (m + kReduceStep - 1) & ~(kReduceStep - 1);
         if (m + tid < padded) s_f[m + tid] = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (unsigned k = tid; k < m; k += nthr) {
+        unsigned classes = 0;
+        for (unsigned k = tid, u = 0; k < m; k += nthr, ++u) {
             float4 x;
             const V3 p = place(sc + k, x);
             s_f[k] = pot_bead(rInner, rOuter, p.x, p.y, p.z, lig.mtype[sc + k], x.w, nullptr);
-            s_n[k] = nl_cell(nl, p.x, p.y, p.z, lig.type[sc + k]);
+            const uint2 cell = nl_cell(nl, p.x, p.y, p.z, lig.type[sc + k]);
+            s_n[k] = cell;
+            classes = pack_class<Classes16>(classes, u, cell.x);
         }
         __syncthreads();
         // P2
-        const unsigned qn = class_queue([&](unsigned k) { return s_n[k].x; }, m, s_q, s_cc, tid,
-                                        nthr, [] { __syncthreads(); });
+        const unsigned qn = class_queue<Classes16, W, 4>(classes, m, s_q, s_cc, tid, [] { __syncthreads(); });
         // P3
         for (unsigned q0 = 0, round = 0; q0 < qn; q0 += nthr / 4, ++round) {
             const unsigned item = q0 + quad_group<W>(tid, round);
