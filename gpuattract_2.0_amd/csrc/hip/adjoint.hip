@@ -326,29 +326,33 @@ __device__ __forceinline__ void adj_walk(const PairDesc& P, const PairTab& tab,
     }
 }
 
-// The workgroup-shared state of one pose (static LDS), WAVES waves per pose:
-// the ligand is taken in super-chunks (LDS for eight workgroups of two waves,
-// or sixteen of one, per CU).
-template <int WAVES, int MM>
+// The workgroup-shared state of one pose (static LDS): the ligand is taken in
+// super-chunks (LDS for eight workgroups of two waves, or sixteen of one, per
+// CU).  The order of the sums is that of VW waves, VW a function of the pair;
+// PW waves do the work: VW of them, or for calls of few poses 4 VW, which
+// changes no bit of a pose's results (the super-chunks, the queue and the
+// thread that a bead's receptor-mode sums belong to are VW's).
+template <int VW, int PW, int MM>
 struct PoseLDS {
+    static_assert(PW == VW || (PW == 4 * VW && MM > 0), "waves per pose");
     // Beads per wave of a super-chunk: 256 with modes (26 B each); without, 384
     // (18 B: the list's cell is found again at the walk), so that the ligands
     // scored by one wave are one super-chunk, with fewer walk steps
     // (1000/300 beads: 45 against 57).
-    static constexpr unsigned kChunks = MM > 0 ? 4 : 6;
-    static constexpr unsigned kSuper = 64u * kChunks * WAVES;
+    static constexpr unsigned kSuper = 64u * (MM > 0 ? 4 : 6) * VW;
+    static constexpr unsigned kChunks = kSuper / (64u * PW);
     using Classes = std::conditional_t<(MM > 0), Classes9, Classes16>;
     float4 g[kSuper];     // per bead: dE/dp (grid, then minus the pair forces); energy
     uint2 nlc[MM > 0 ? kSuper : 1];  // neighbour-list {count, start}
     unsigned short q[kSuper];
     unsigned cc[queue_counters<Classes>(kSuper)];
-    float red[WAVES][MM > 0 ? ATT_MODES_MAX : 1];
-    unsigned cnt[WAVES][2];
+    float red[VW][MM > 0 ? ATT_MODES_MAX : 1];
+    unsigned cnt[PW][2];
     float e;
 };
 
-// Adjoint of one pose by one workgroup of WAVES waves, the ligand in
-// super-chunks of equal size, at most PoseLDS<WAVES, MM>::kSuper beads (super_chunk):
+// Adjoint of one pose by one workgroup of PW waves in the order of VW, the ligand
+// in super-chunks of equal size, at most PoseLDS::kSuper beads (super_chunk):
 //  P1  every bead: transform, grid term with its exact gradient (and the
 //      basis-grid parameter derivatives), neighbour-list cell;
 //  P2  beads with a list, longest lists first (class_queue);
@@ -358,15 +362,18 @@ struct PoseLDS {
 //      energy is the reference's bits), and the chain rule through p = R x~ + t
 //      by wave 0, bead k on lane k % 64, lane sums reduced by a butterfly.
 // Every sum has a fixed order: results do not depend on timing.
-template <int MM, int WAVES, int PG>
-__device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, PoseLDS<WAVES, MM>& S,
+template <int MM, int VW, int PW, int PG>
+__device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, PoseLDS<VW, PW, MM>& S,
                                              const PairTab& tab, float* s_pg,
                                              size_t recBase) {
     const DProt& lig = P.lig;
     const DPar& par = P.par;
     const unsigned tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    constexpr unsigned nthr = 64u * WAVES;
-    constexpr unsigned eThread = WAVES > 1 ? 64u : 0u;  // sums the energy
+    using LDS = PoseLDS<VW, PW, MM>;
+    constexpr unsigned nthr = 64u * PW;
+    constexpr unsigned owners = 64u * VW;           // threads that own receptor-mode sums
+    constexpr unsigned subs = owners / (nthr / 4);  // sub-rounds of the quads per round of owners
+    constexpr unsigned eThread = PW > 1 ? 64u : 0u;  // sums the energy
     constexpr int MA = MM > 0 ? MM : 1;
     const unsigned Ml = MM > 0 ? lig.M : 0, Mr = MM > 0 ? P.rec.M : 0;
     __syncthreads();  // LDS of the previous pose is no longer read
@@ -413,7 +420,7 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
         return place_from_row<MM>(lig, i, ampL, R, tx, ty, tz, x, lt);
     };
 
-    const unsigned span = super_chunk(lig.n, PoseLDS<WAVES, MM>::kSuper);
+    const unsigned span = super_chunk(lig.n, LDS::kSuper);
     for (unsigned sc = 0; sc < lig.n; sc += span) {
         const unsigned m = min(span, lig.n - sc);
         // P1
@@ -428,21 +435,21 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
             S.g[k] = make_float4(G.x, G.y, G.z, eg);
             const uint2 cell = nl_cell(P.nl, p.x, p.y, p.z, lig.type[sc + k]);
             if (MM > 0) S.nlc[k] = cell;
-            classes = pack_class<typename PoseLDS<WAVES, MM>::Classes>(classes, u, cell.x);
+            classes = pack_class<typename LDS::Classes>(classes, u, cell.x);
         }
         __syncthreads();
         // P2
-        const unsigned qn = class_queue<typename PoseLDS<WAVES, MM>::Classes, WAVES,
-                                        PoseLDS<WAVES, MM>::kChunks>(classes, m, S.q, S.cc, tid,
-                                                                     [] { __syncthreads(); });
+        const unsigned qn = class_queue<typename LDS::Classes, PW, LDS::kChunks>(
+            classes, m, S.q, S.cc, tid, [] { __syncthreads(); });
         // P3
-        for (unsigned q0 = 0; q0 < qn; q0 += nthr) {
-            for (unsigned sub = 0; sub < 4; ++sub) {
-                // Quad sums of queue item i belong to thread i % nthr: item
-                // q0 + sub * nthr / 4 + group, kept by the quad's lane `sub`.
+        for (unsigned q0 = 0; q0 < qn; q0 += owners) {
+            for (unsigned sub = 0; sub < subs; ++sub) {
+                // Quad sums of queue item i belong to thread i % owners: item
+                // q0 + sub * nthr / 4 + group, kept by the quad's lane `sub`
+                // (by all four where there is one sub-round).
                 // Odd sub-rounds give the waves the groups in reverse order
                 // (the queue is sorted: a later group's lists are shorter).
-                const unsigned item = q0 + sub * (nthr / 4) + quad_group<WAVES>(tid, sub);
+                const unsigned item = q0 + sub * (nthr / 4) + quad_group<PW>(tid, sub);
                 if (item < qn) {
                     const unsigned k = S.q[item];
                     float4 x;
@@ -451,13 +458,13 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
                     float eAcc, g4[MA];
                     float3 gAcc;
 #pragma unroll
-                    for (int m = 0; m < MA; ++m) g4[m] = MM > 0 ? __shfl(gR[m], (lane & ~3u) | sub) : 0.f;
+                    for (int m = 0; m < MA; ++m) g4[m] = MM == 0 ? 0.f : subs == 1 ? gR[m] : __shfl(gR[m], (lane & ~3u) | sub);
                     const uint2 nlc = MM > 0 ? S.nlc[k] : nl_cell(P.nl, p.x, p.y, p.z, lt);
                     adj_walk<MM, PG>(P, tab, pg, p.x, p.y, p.z, x.w, lt, nlc, lane & 3u, ampR, g4,
                                      eAcc, gAcc, inside);
 #pragma unroll
                     for (int m = 0; m < MA; ++m)
-                        if (MM > 0 && (lane & 3u) == sub) gR[m] = g4[m];
+                        if (MM > 0 && (subs == 1 || (lane & 3u) == sub)) gR[m] = g4[m];
                     if ((lane & 3u) == 0) {
                         listed += nlc.x;
                         float4 g = S.g[k];
@@ -513,18 +520,22 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
     }
     if (MM > 0) {
         // the quads' receptor-mode sums to the threads they belong to (the
-        // beads' array is free), then the wave butterflies
+        // beads' array is free), then the owners' wave butterflies
         float* t = reinterpret_cast<float*>(S.g);
-        const unsigned owner = (lane & 3u) * (nthr / 4) + quad_group<WAVES>(tid, lane & 3u);
+        const unsigned owner = (lane & 3u) * (nthr / 4) + quad_group<PW>(tid, lane & 3u);
+        if ((lane & 3u) < subs) {
 #pragma unroll
-        for (int m = 0; m < MA; ++m) t[m * nthr + owner] = gR[m];
+            for (int m = 0; m < MA; ++m) t[m * owners + owner] = gR[m];
+        }
         __syncthreads();
+        if (wave < (unsigned)VW) {
 #pragma unroll
-        for (int m = 0; m < MA; ++m) gR[m] = wave_sum(t[m * nthr + tid]);
-    }
-    if (lane == 0) {
+            for (int m = 0; m < MA; ++m) gR[m] = wave_sum(t[m * owners + tid]);
+            if (lane == 0) {
 #pragma unroll
-        for (int m = 0; MM > 0 && m < ATT_MODES_MAX; ++m) S.red[wave][m] = m < MA ? gR[m < MA ? m : 0] : 0.f;
+                for (int m = 0; m < ATT_MODES_MAX; ++m) S.red[wave][m] = m < MA ? gR[m < MA ? m : 0] : 0.f;
+            }
+        }
     }
     if (tid == eThread) S.e = esum;
     if (P.counts) {
@@ -535,7 +546,7 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
     __syncthreads();
     if (P.counts && tid == 0) {
         uint2 c = make_uint2(0u, 0u);
-        for (unsigned w = 0; w < (unsigned)WAVES; ++w) { c.x += S.cnt[w][0]; c.y += S.cnt[w][1]; }
+        for (unsigned w = 0; w < (unsigned)PW; ++w) { c.x += S.cnt[w][0]; c.y += S.cnt[w][1]; }
         P.counts[pose] = c;
     }
     if (tid == 0) {
@@ -549,7 +560,7 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
 #pragma unroll
             for (unsigned m = 0; m < ATT_MODES_MAX; ++m) {
                 float s = MM > 0 ? S.red[0][m] : 0.f;
-                for (unsigned w = 1; MM > 0 && w < (unsigned)WAVES; ++w) s += S.red[w][m];
+                for (unsigned w = 1; MM > 0 && w < (unsigned)VW; ++w) s += S.red[w][m];
                 o[7 + m] = m < Mr ? wp * s : 0.f;
                 o[17 + m] = m < Ml ? wp * gL[m < MA ? m : 0] : 0.f;
             }
@@ -567,11 +578,11 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
 template <int MM>
 constexpr int adjoint_waves_per_simd() { return MM >= 10 ? 3 : 4; }
 
-template <int MM, int WAVES, int PG>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(adjoint_waves_per_simd<MM>()))) void k_adjoint(
+template <int MM, int VW, int PW, int PG>
+__global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(adjoint_waves_per_simd<MM>()))) void k_adjoint(
     PairDesc P, float* __restrict__ pgPartial) {
     extern __shared__ att_pair_params s_dyn[];
-    __shared__ PoseLDS<WAVES, MM> S;
+    __shared__ PoseLDS<VW, PW, MM> S;
     char* dyn = reinterpret_cast<char*>(s_dyn);
     const PairTab tab = stage_table(P.par, s_dyn);
     // Parameter derivatives: one LDS slice per wave, so that every slice is
@@ -580,7 +591,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(adjo
     float* s_pg = PG != kPgNone ? reinterpret_cast<float*>(dyn + adjoint_pg_offset(P.tabSlots)) : nullptr;
     const unsigned npg = 3 * P.par.T * P.par.T;
     if (PG != kPgNone)
-        for (unsigned k = threadIdx.x; k < npg * WAVES; k += blockDim.x) s_pg[k] = 0.f;
+        for (unsigned k = threadIdx.x; k < npg * PW; k += blockDim.x) s_pg[k] = 0.f;
     const unsigned n = P.nDev ? min(P.nDev[0], P.n) : P.n;
     // With a spatial order (and at least 8 workgroups), workgroup b (on XCD
     // b % 8) walks the (b % 8)-th eighth of it; otherwise the poses in input
@@ -595,12 +606,12 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(adjo
     }
     // grid-cell records of slot i (kPgRecords) start at i * ligand beads
     for (unsigned i = first; i < end; i += step)
-        adjoint_pose<MM, WAVES, PG>(P, P.order ? P.order[i] : i, S, tab, s_pg, (size_t)i * P.lig.n);
+        adjoint_pose<MM, VW, PW, PG>(P, P.order ? P.order[i] : i, S, tab, s_pg, (size_t)i * P.lig.n);
     if (PG != kPgNone) {
         __syncthreads();
         for (unsigned k = threadIdx.x; k < npg; k += blockDim.x) {
             float v = s_pg[k];
-            for (unsigned w = 1; w < (unsigned)WAVES; ++w) v += s_pg[w * npg + k];
+            for (unsigned w = 1; w < (unsigned)PW; ++w) v += s_pg[w * npg + k];
             pgPartial[(size_t)blockIdx.x * npg + k] = v;
         }
     }
@@ -617,7 +628,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(adjo
     const PairDesc* __restrict__ pairs, const BatchTile* __restrict__ tiles,
     const unsigned* __restrict__ queueStart, unsigned* __restrict__ counters) {
     extern __shared__ att_pair_params s_dyn[];
-    __shared__ PoseLDS<WAVES, MM> S;
+    __shared__ PoseLDS<WAVES, WAVES, MM> S;
     __shared__ unsigned s_tile;
     unsigned cur = 0xFFFFFFFFu;
     PairTab tab{nullptr, false};
@@ -637,7 +648,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(adjo
                 cur = tile.pair;
             }
             for (unsigned i = tile.first; i < tile.first + tile.count; ++i)
-                adjoint_pose<MM, WAVES, kPgNone>(P, P.order ? P.order[i] : i, S, tab, nullptr, 0);
+                adjoint_pose<MM, WAVES, WAVES, kPgNone>(P, P.order ? P.order[i] : i, S, tab, nullptr, 0);
         }
     }
 }
@@ -722,62 +733,76 @@ size_t adjoint_lds_bytes(const DProt& rec, const DProt& lig, const DPar& par, bo
            (pgrad ? sizeof(float) * 3 * (size_t)par.T * par.T * (size_t)waves : 0);
 }
 
-size_t adjoint_static_lds(int waves) {
-    switch (waves) {
-        case 1: return std::max(sizeof(PoseLDS<1, 0>), sizeof(PoseLDS<1, ATT_MODES_MAX>)) + 16;
-        case 2: return std::max(sizeof(PoseLDS<2, 0>), sizeof(PoseLDS<2, ATT_MODES_MAX>)) + 16;
-        default: return std::max(sizeof(PoseLDS<4, 0>), sizeof(PoseLDS<4, ATT_MODES_MAX>)) + 16;
+size_t adjoint_static_lds(AdjWidth w) {
+    constexpr int M = ATT_MODES_MAX;
+    if (w.work != w.order)
+        return (w.order == 1 ? sizeof(PoseLDS<1, 4, M>) : sizeof(PoseLDS<2, 8, M>)) + 16;
+    switch (w.order) {
+        case 1: return std::max(sizeof(PoseLDS<1, 1, 0>), sizeof(PoseLDS<1, 1, M>)) + 16;
+        case 2: return std::max(sizeof(PoseLDS<2, 2, 0>), sizeof(PoseLDS<2, 2, M>)) + 16;
+        default: return std::max(sizeof(PoseLDS<4, 4, 0>), sizeof(PoseLDS<4, 4, M>)) + 16;
     }
 }
 
 namespace {
 template <int MM, int PG>
-const void* adjoint_kernel(int waves, bool batch) {
-    switch (waves) {
-        case 1: return batch ? (const void*)k_adjoint_batch<MM, 1> : (const void*)k_adjoint<MM, 1, PG>;
-        case 2: return batch ? (const void*)k_adjoint_batch<MM, 2> : (const void*)k_adjoint<MM, 2, PG>;
-        default: return batch ? (const void*)k_adjoint_batch<MM, 4> : (const void*)k_adjoint<MM, 4, PG>;
+const void* adjoint_kernel(AdjWidth w) {
+    if constexpr (MM > 0)
+        if (w.work != w.order)
+            return w.order == 1 ? (const void*)k_adjoint<MM, 1, 4, PG> : (const void*)k_adjoint<MM, 2, 8, PG>;
+    switch (w.order) {
+        case 1: return (const void*)k_adjoint<MM, 1, 1, PG>;
+        case 2: return (const void*)k_adjoint<MM, 2, 2, PG>;
+        default: return (const void*)k_adjoint<MM, 4, 4, PG>;
     }
 }
-template <int PG>
-const void* adjoint_kernel_pg(unsigned mm, int waves, bool batch) {
-    if (mm == 0) return adjoint_kernel<0, PG>(waves, batch);
-    if (mm <= 5) return adjoint_kernel<5, PG>(waves, batch);
-    return adjoint_kernel<ATT_MODES_MAX, PG>(waves, batch);
+template <int MM>
+const void* adjoint_batch_kernel(AdjWidth w) {
+    switch (w.order) {
+        case 1: return (const void*)k_adjoint_batch<MM, 1>;
+        case 2: return (const void*)k_adjoint_batch<MM, 2>;
+        default: return (const void*)k_adjoint_batch<MM, 4>;
+    }
 }
-const void* adjoint_kernel_for(unsigned mm, int waves, bool batch, int pg = kPgNone) {
-    if (batch || pg == kPgNone) return adjoint_kernel_pg<kPgNone>(mm, waves, batch);
-    if (pg == kPgFused) return adjoint_kernel_pg<kPgFused>(mm, waves, false);
-    return adjoint_kernel_pg<kPgRecords>(mm, waves, false);
+template <int MM>
+const void* adjoint_kernel_mm(AdjWidth w, bool batch, int pg) {
+    if (batch) return adjoint_batch_kernel<MM>(w);
+    if (pg == kPgNone) return adjoint_kernel<MM, kPgNone>(w);
+    if (pg == kPgFused) return adjoint_kernel<MM, kPgFused>(w);
+    return adjoint_kernel<MM, kPgRecords>(w);
+}
+const void* adjoint_kernel_for(unsigned mm, AdjWidth w, bool batch, int pg = kPgNone) {
+    if (mm == 0) return adjoint_kernel_mm<0>(w, batch, pg);
+    if (mm <= 5) return adjoint_kernel_mm<5>(w, batch, pg);
+    return adjoint_kernel_mm<ATT_MODES_MAX>(w, batch, pg);
 }
 }  // namespace
 
-unsigned adjoint_blocks_per_cu(unsigned mm, int waves, bool batch, size_t lds, int pg) {
+unsigned adjoint_blocks_per_cu(unsigned mm, AdjWidth w, bool batch, size_t lds, int pg) {
     int b = 0;
     const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &b, adjoint_kernel_for(mm, waves, batch, pg), 64 * waves, lds);
+        &b, adjoint_kernel_for(mm, w, batch, pg), 64 * w.work, lds);
     return e == hipSuccess && b > 0 ? (unsigned)b : 1u;
 }
 
 hipError_t launch_adjoint(const PairDesc& P, bool modes, float* pgPartial, unsigned blocks,
-                          int waves, size_t lds, hipStream_t s) {
+                          AdjWidth w, size_t lds, hipStream_t s) {
     if (P.n == 0) return hipSuccess;
     const unsigned mm = modes ? (P.rec.M > P.lig.M ? P.rec.M : P.lig.M) : 0;
     const int pg = !pgPartial ? kPgNone : P.recKey ? kPgRecords : kPgFused;
     void* args[] = {const_cast<PairDesc*>(&P), &pgPartial};
-    return hipLaunchKernel(adjoint_kernel_for(mm, waves, false, pg), dim3(blocks), dim3(64 * waves),
+    return hipLaunchKernel(adjoint_kernel_for(mm, w, false, pg), dim3(blocks), dim3(64 * w.work),
                            args, lds, s);
 }
 
-hipError_t launch_adjoint_batch(unsigned mm, int waves, const PairDesc* pairs, const BatchTile* tiles,
+hipError_t launch_adjoint_batch(unsigned mm, AdjWidth w, const PairDesc* pairs, const BatchTile* tiles,
                                 const unsigned* queueStart, unsigned ntiles, unsigned* counters,
                                 unsigned blocks, size_t lds, hipStream_t s) {
     hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, counters, kBatchQueues);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || ntiles == 0) return e;
     void* args[] = {&pairs, &tiles, &queueStart, &counters};
-    return hipLaunchKernel(adjoint_kernel_for(mm, waves, true), dim3(blocks), dim3(64 * waves), args,
-                           lds, s);
+    return hipLaunchKernel(adjoint_kernel_for(mm, w, true), dim3(blocks), dim3(64 * w.work), args, lds, s);
 }
 
 hipError_t launch_pgrad_reduce(const float* partial, unsigned rows, unsigned cols, double* groups,

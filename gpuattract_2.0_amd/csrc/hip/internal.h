@@ -11,10 +11,11 @@ namespace att {
 // `order`: a spatial permutation of the poses (or null); workgroups of one
 // XCD then take a contiguous range of it (xcd_slot).
 // `counts` (or null): per pose {listed neighbours of the beads walked, pairs
-// inside the plateau}.
+// inside the plateau}.  Calls of few poses per CU get
+// more waves per pose.
 hipError_t launch_rigid(const DProt& rec, const DProt& lig, const DGrid& inner, const DGrid& outer,
                         const DNL& nl, const DPar& par, const float* dofs, float* res, unsigned n,
-                        const unsigned* order, uint2* counts, hipStream_t s);
+                        const unsigned* order, uint2* counts, unsigned numCU, hipStream_t s);
 
 size_t modes_lds_bytes(const DProt& rec, const DProt& lig, const DPar& par, unsigned* tabSlots);
 
@@ -47,10 +48,16 @@ hipError_t launch_octets(const float4* grid, float4* oct, float4* octE, unsigned
 
 size_t adjoint_lds_bytes(const DProt& rec, const DProt& lig, const DPar& par, bool pgrad,
                          int waves, unsigned* tabSlots);
-// Static LDS of the adjoint kernels with `waves` waves per pose, and how many
-// of their workgroups one CU holds with `lds` bytes of dynamic LDS.
-size_t adjoint_static_lds(int waves);
-unsigned adjoint_blocks_per_cu(unsigned mm, int waves, bool batch, size_t lds, int pg = 0);
+// Waves per pose of the adjoint: `order` (1, 2 or 4) sets the order of its sums,
+// `work` waves share it: the same number, or for calls of few poses four times
+// as many (order 1 or 2, with modes; the same bits).
+struct AdjWidth {
+    int order, work;
+};
+// Static LDS of the adjoint kernels of a width, and how many of their workgroups
+// one CU holds with `lds` bytes of dynamic LDS.
+size_t adjoint_static_lds(AdjWidth w);
+unsigned adjoint_blocks_per_cu(unsigned mm, AdjWidth w, bool batch, size_t lds, int pg = 0);
 
 // How k_adjoint takes the grid part of the parameter gradient: not at all (no
 // parameter gradient), from the basis grids at every bead (kPgFused), or as
@@ -83,13 +90,13 @@ PgCellBufs pg_cells_layout(void* scratch, size_t records, unsigned endBit, bool 
 hipError_t launch_pg_cells(const PairDesc& P, const PgCellBufs& B, size_t records, unsigned endBit,
                            float* rows, unsigned blocks, hipStream_t s);
 
-// One pair: persistent grid of `blocks` workgroups of 64*waves threads.
+// One pair: persistent grid of `blocks` workgroups of 64 * w.work threads.
 hipError_t launch_adjoint(const PairDesc& P, bool modes, float* pgPartial, unsigned blocks,
-                          int waves, size_t lds, hipStream_t s);
+                          AdjWidth w, size_t lds, hipStream_t s);
 // Many pairs of one mode-capacity class: resets the kBatchQueues tile
 // counters, then the persistent batch kernel over the tile queues
 // [queueStart[x], queueStart[x+1]) (graph-capturable: no memset, no host sync).
-hipError_t launch_adjoint_batch(unsigned mm, int waves, const PairDesc* pairs, const BatchTile* tiles,
+hipError_t launch_adjoint_batch(unsigned mm, AdjWidth w, const PairDesc* pairs, const BatchTile* tiles,
                                 const unsigned* queueStart, unsigned ntiles, unsigned* counters,
                                 unsigned blocks, size_t lds, hipStream_t s);
 

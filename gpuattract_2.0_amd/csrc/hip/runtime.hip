@@ -302,6 +302,22 @@ namespace {
 // two of 1, 2, 4).  Both paths use it, so a point scored by either gives the
 // same bits.
 int pair_waves(unsigned ligN) { return ligN < 384 ? 1 : 2; }
+// Waves per pose of an adjoint call of n poses: pair_waves order the sums; a
+// call whose poses would leave wave slots empty (16 per CU) gets four times as
+// many to share a pose's work, with modes; without, the order decides no bit and
+// four waves do.  The same bits either way, so the line lies where the CUs are
+// full: 512 poses 3000/800 with 5 + 5 modes 184 -> 100 us, 1024 poses 1000/300
+// rigid 100 -> 47 us, but 2048 and 4096 of them 277 -> 382 and 142 -> 170 us.
+AdjWidth adjoint_width(const att_ctx* c, const DProt& rec, const DProt& lig, const DPar& par,
+                       unsigned mm, size_t n, bool pgrad) {
+    const int order = pair_waves(lig.n);
+    const AdjWidth few = mm == 0 ? AdjWidth{4, 4} : AdjWidth{order, 4 * order};
+    if (n * (size_t)few.work <= 16 * (size_t)c->numCU &&
+        adjoint_lds_bytes(rec, lig, par, pgrad, few.work, nullptr) + adjoint_static_lds(few) <=
+            c->maxLdsPerBlock)
+        return few;
+    return AdjWidth{order, order};
+}
 // Parameter-gradient records per call up to which the cell pass takes the
 // grid part (68 B of scratch per record without pose weights, 76 B with:
 // 9-10 GB at the cap), and the workgroups of that pass (one parameter row
@@ -655,7 +671,7 @@ att_status att_score_rigid_dev(att_ctx* c, att_handle hr, att_handle hl, att_han
         return st;
     ATT_HIP(c, launch_rigid(rec->d, lig->d, g->inner, g->outer, g->nl, p->d,
                             reinterpret_cast<const float*>(d_dofs), reinterpret_cast<float*>(d_out),
-                            (unsigned)n, order, counts, s));
+                            (unsigned)n, order, counts, c->numCU, s));
     if (order) ATT_HIP(c, hipEventRecord(c->scratchEv, s));
     return ATT_OK;
 }
@@ -787,9 +803,10 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
     if (pgrad && (!g->bin.oct || g->bin.nb != 2 * p->d.T))
         return fail(c, ATT_ERR_INVALID, "parameter gradients need basis grids for this table (att_upload_basis)");
     unsigned slots = 0;
-    const int kWaves = pair_waves(lig->d.n);
-    const size_t dyn = adjoint_lds_bytes(rec->d, lig->d, p->d, pgrad, kWaves, &slots);
-    if (dyn + adjoint_static_lds(kWaves) > c->maxLdsPerBlock)
+    const unsigned mm = modes ? std::max(rec->d.M, lig->d.M) : 0;
+    const AdjWidth width = adjoint_width(c, rec->d, lig->d, p->d, mm, n, pgrad);
+    const size_t dyn = adjoint_lds_bytes(rec->d, lig->d, p->d, pgrad, width.work, &slots);
+    if (dyn + adjoint_static_lds(width) > c->maxLdsPerBlock)
         return fail(c, ATT_ERR_UNSUPPORTED, "ligand too large for the LDS of the adjoint kernel");
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     const unsigned cols = 3 * p->d.T * p->d.T;
@@ -804,8 +821,7 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
                         sizeof(float) * cols <= c->maxLdsPerBlock;
     const int pgMode = !pgrad ? kPgNone : useRec ? kPgRecords : kPgFused;
     // persistent grid: as many workgroups as the device holds at once
-    const unsigned mm = modes ? std::max(rec->d.M, lig->d.M) : 0;
-    const size_t resident = (size_t)c->numCU * adjoint_blocks_per_cu(mm, kWaves, false, dyn, pgMode);
+    const size_t resident = (size_t)c->numCU * adjoint_blocks_per_cu(mm, width, false, dyn, pgMode);
     const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(n, resident));
     const unsigned cellBlocks = useRec ? kPgCellBlocks : 0;
     // per-workgroup rows (the adjoint's, then the cell pass's), then the
@@ -848,7 +864,7 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
     const bool scratch = pgrad || P.order;
     if (pgrad && !P.order) ATT_HIP(c, hipStreamWaitEvent(s, c->scratchEv, 0));
     float* rows = pgrad ? static_cast<float*>(c->d_pg) : nullptr;
-    ATT_HIP(c, launch_adjoint(P, modes != 0, rows, blocks, kWaves, dyn, s));
+    ATT_HIP(c, launch_adjoint(P, modes != 0, rows, blocks, width, dyn, s));
     if (useRec)
         ATT_HIP(c, launch_pg_cells(P, B, records, endBit, rows + (size_t)blocks * cols, cellBlocks, s));
     if (pgrad)
@@ -881,14 +897,14 @@ att_status att_score_adjoint_dev_noalloc(att_ctx* c, att_handle hr, att_handle h
     if (pgrad && cols > kNoAllocCols)
         return fail(c, ATT_ERR_UNSUPPORTED, "parameter gradients without allocation: at most 16 pair types");
     unsigned slots = 0;
-    const int kWaves = pair_waves(lig->d.n);
-    const size_t dyn = adjoint_lds_bytes(rec->d, lig->d, p->d, pgrad, kWaves, &slots);
-    if (dyn + adjoint_static_lds(kWaves) > c->maxLdsPerBlock)
+    const unsigned mm = modes ? std::max(rec->d.M, lig->d.M) : 0;
+    const AdjWidth width = adjoint_width(c, rec->d, lig->d, p->d, mm, n, pgrad);
+    const size_t dyn = adjoint_lds_bytes(rec->d, lig->d, p->d, pgrad, width.work, &slots);
+    if (dyn + adjoint_static_lds(width) > c->maxLdsPerBlock)
         return fail(c, ATT_ERR_UNSUPPORTED, "pair table too large for the LDS of the adjoint kernel");
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
-    const unsigned mm = modes ? std::max(rec->d.M, lig->d.M) : 0;
     const size_t resident =
-        (size_t)c->numCU * adjoint_blocks_per_cu(mm, kWaves, false, dyn, pgrad ? kPgFused : kPgNone);
+        (size_t)c->numCU * adjoint_blocks_per_cu(mm, width, false, dyn, pgrad ? kPgFused : kPgNone);
     const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(n, resident));
     if (pgrad && blocks > kNoAllocBlocks)
         return fail(c, ATT_ERR_UNSUPPORTED, "more resident workgroups than the no-allocation scratch holds");
@@ -910,7 +926,7 @@ att_status att_score_adjoint_dev_noalloc(att_ctx* c, att_handle hr, att_handle h
     // so the scratch needs no clearing between calls.
     float* rows = static_cast<float*>(c->noallocScratch);
     double* groups = reinterpret_cast<double*>(static_cast<char*>(c->noallocScratch) + kNoAllocRowBytes);
-    ATT_HIP(c, launch_adjoint(P, modes != 0, pgrad ? rows : nullptr, blocks, kWaves, dyn, s));
+    ATT_HIP(c, launch_adjoint(P, modes != 0, pgrad ? rows : nullptr, blocks, width, dyn, s));
     if (pgrad) ATT_HIP(c, launch_pgrad_reduce(rows, blocks, cols, groups, d_pgrad, s));
     return ATT_OK;
 }
@@ -1316,10 +1332,10 @@ att_status batch_tiles(att_ctx* c, att_batch* b, att_batch::Bucket& k) {
 hipError_t batch_launch(att_ctx* c, att_batch* b, size_t i, hipStream_t s) {
     att_batch::Bucket& k = b->buckets[i];
     const size_t resident =
-        (size_t)c->numCU * adjoint_blocks_per_cu(k.mm, k.waves, true, k.lds);
+        (size_t)c->numCU * adjoint_blocks_per_cu(k.mm, AdjWidth{k.waves, k.waves}, true, k.lds);
     const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(k.tiles.size(), resident));
     const unsigned* qs = reinterpret_cast<const unsigned*>(k.d_tiles + k.tiles.size());
-    return launch_adjoint_batch(k.mm, k.waves, b->d_pairs, k.d_tiles, qs, (unsigned)k.tiles.size(),
+    return launch_adjoint_batch(k.mm, AdjWidth{k.waves, k.waves}, b->d_pairs, k.d_tiles, qs, (unsigned)k.tiles.size(),
                                 b->d_counters + kBatchQueues * i, blocks, k.lds, s);
 }
 
@@ -1387,7 +1403,7 @@ att_status batch_fill(att_ctx* c, att_batch* b, const att_batch_pair* in, unsign
         if (q.n && (!q.d_dofs || !q.d_out)) return fail(c, ATT_ERR_INVALID, "null buffer");
         unsigned slots = 0;
         const size_t dyn = adjoint_lds_bytes(rec->d, lig->d, p->d, false, 1, &slots);
-        if (dyn + adjoint_static_lds(4) > c->maxLdsPerBlock)
+        if (dyn + adjoint_static_lds(AdjWidth{4, 4}) > c->maxLdsPerBlock)
             return fail(c, ATT_ERR_UNSUPPORTED, "ligand too large for the LDS of the adjoint kernel");
         PairDesc P{};
         P.rec = rec->d; P.lig = lig->d;
@@ -1495,7 +1511,7 @@ att_status att_batch_set_shape(att_ctx* c, att_batch* b, unsigned bucket, int wa
         return fail(c, ATT_ERR_INVALID, "waves per pose must be 1, 2 or 4 and tiles non-empty");
     ATT_HIP(c, hipSetDevice(c->device));
     att_batch::Bucket& k = b->buckets[bucket];
-    if (k.lds + adjoint_static_lds(wavesPerPose) > c->maxLdsPerBlock)
+    if (k.lds + adjoint_static_lds(AdjWidth{wavesPerPose, wavesPerPose}) > c->maxLdsPerBlock)
         return fail(c, ATT_ERR_UNSUPPORTED, "shape does not fit the LDS");
     k.waves = wavesPerPose;
     k.ms = -1.f;
@@ -1525,7 +1541,7 @@ att_status att_batch_tune(att_ctx* c, att_batch* b, void* stream) {
         int bw = 4;
         unsigned bt = 16;
         for (int w : kWaves) {
-            if (k.lds + adjoint_static_lds(w) > c->maxLdsPerBlock) continue;
+            if (k.lds + adjoint_static_lds(AdjWidth{w, w}) > c->maxLdsPerBlock) continue;
             for (unsigned tl : kTiles) {
                 if ((st = att_batch_set_shape(c, b, (unsigned)i, w, tl)) != ATT_OK) break;
                 hipError_t e = batch_launch(c, b, i, s);  // warm-up
@@ -1593,8 +1609,10 @@ struct att_minjob {
     PairDesc P{};
     bool modes = false;
     size_t dyn = 0;
-    unsigned blocks = 1;
-    int waves = 2;
+    unsigned blocks[2] = {1, 1};      // of a round of many poses, of few
+    AdjWidth width[2] = {{2, 2}, {2, 2}};
+    unsigned few = 0;                 // rounds of at most this many poses take width[1]
+    unsigned running = 0;             // at most (att_minjob_set_running)
     void* mem = nullptr;
     size_t bytes = 0;
     unsigned* list[2] = {nullptr, nullptr};
@@ -1644,9 +1662,11 @@ att_status att_minjob_create(att_ctx* c, att_handle hr, att_handle hl, att_handl
     std::unique_ptr<att_minjob> j(new att_minjob);
     unsigned slots = 0;
     j->dyn = adjoint_lds_bytes(rec->d, lig->d, p->d, false, 1, &slots);
-    const int kWaves = pair_waves(lig->d.n);  // the single-pair adjoint's shape: same results
-    j->waves = kWaves;
-    if (j->dyn + adjoint_static_lds(kWaves) > c->maxLdsPerBlock)
+    const unsigned mm = modes ? std::max(rec->d.M, lig->d.M) : 0;
+    // the single-pair adjoint's shapes: same results
+    j->width[0] = AdjWidth{pair_waves(lig->d.n), pair_waves(lig->d.n)};
+    j->width[1] = adjoint_width(c, rec->d, lig->d, p->d, mm, 1, false);
+    if (j->dyn + adjoint_static_lds(j->width[0]) > c->maxLdsPerBlock)
         return fail(c, ATT_ERR_UNSUPPORTED, "ligand too large for the LDS of the adjoint kernel");
     MinRun& R = j->R;
     R.npose = (unsigned)n;
@@ -1684,9 +1704,12 @@ att_status att_minjob_create(att_ctx* c, att_handle hr, att_handle hl, att_handl
     P.dofStride = R.ds; P.outStride = R.os;
     P.n = (unsigned)n; P.tabSlots = slots;
     j->modes = modes != 0;
-    const unsigned mm = modes ? std::max(rec->d.M, lig->d.M) : 0;
-    const size_t resident = (size_t)c->numCU * adjoint_blocks_per_cu(mm, kWaves, false, j->dyn);
-    j->blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(n, resident));
+    for (int k = 0; k < 2; ++k) {
+        const size_t resident = (size_t)c->numCU * adjoint_blocks_per_cu(mm, j->width[k], false, j->dyn);
+        j->blocks[k] = (unsigned)std::max<size_t>(1, std::min<size_t>(n, resident));
+    }
+    if (j->width[1].work > j->width[0].work) j->few = 16 * c->numCU / (unsigned)j->width[1].work;
+    j->running = (unsigned)n;
     *out = j.release();
     return ATT_OK;
 }
@@ -1698,6 +1721,7 @@ att_status att_minjob_start(att_ctx* c, att_minjob* j, const float* d_dofs, void
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     j->cur = 0;
     j->rounds = 0;
+    j->running = j->R.npose;
     j->R.list = j->list[0]; j->R.count = j->count[0]; j->R.req = j->req[0];
     ATT_HIP(c, launch_min_start(j->R, d_dofs, s));
     return ATT_OK;
@@ -1710,9 +1734,10 @@ att_status att_minjob_rounds(att_ctx* c, att_minjob* j, int rounds, void* stream
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     for (int r = 0; r < rounds; ++r) {
         const int cur = j->cur, nxt = cur ^ 1;
+        const int w = j->running <= j->few ? 1 : 0;
         j->P.dofs = j->req[cur];
         j->P.nDev = j->count[cur];
-        ATT_HIP(c, launch_adjoint(j->P, j->modes, nullptr, j->blocks, j->waves, j->dyn, s));
+        ATT_HIP(c, launch_adjoint(j->P, j->modes, nullptr, j->blocks[w], j->width[w], j->dyn, s));
         j->R.list = j->list[nxt]; j->R.count = j->count[nxt]; j->R.req = j->req[nxt];
         ATT_HIP(c, launch_min_step(j->R, j->list[cur], j->count[cur], j->req[cur], j->res, s));
         j->cur = nxt;
@@ -1722,6 +1747,10 @@ att_status att_minjob_rounds(att_ctx* c, att_minjob* j, int rounds, void* stream
 }
 
 int att_minjob_round_limit(const att_minjob* j) { return j ? j->R.ivmax + 2 : 0; }
+
+void att_minjob_set_running(att_minjob* j, unsigned running) {
+    if (j) j->running = running;
+}
 
 att_status att_minjob_running(att_ctx* c, att_minjob* j, unsigned* h_count, void* stream) {
     if (!c) return ATT_ERR_INVALID;
@@ -1774,6 +1803,7 @@ att_status att_minimize_dev(att_ctx* c, att_handle hr, att_handle hl, att_handle
         if (st == ATT_OK) st = att_minjob_running(c, j, running, s);
         if (st == ATT_OK && hipStreamSynchronize(s) != hipSuccess) st = fail(c, ATT_ERR_HIP, "synchronize");
         if (st == ATT_OK && *running == 0) break;
+        att_minjob_set_running(j, *running);
     }
     if (st == ATT_OK && hipStreamSynchronize(s) != hipSuccess) st = fail(c, ATT_ERR_HIP, "synchronize");
     (void)hipHostFree(running);

@@ -21,33 +21,41 @@
 
 namespace att {
 
-// Beads per super-chunk of k_rigid (per wave) and their LDS: bead force and
-// energy (float4), the class-ordered queue (u16) and its counters.
-constexpr unsigned kRigidSuper = 64 * kQueueChunks;
-constexpr size_t kRigidWaveBytes =
-    (kRigidSuper * (16 + 2) + sizeof(unsigned) * queue_counters<Classes16>(kRigidSuper) + 15) & ~(size_t)15;
-__host__ __device__ inline size_t rigid_wave_offset(unsigned tabSlots) {
-    return (sizeof(att_pair_params) * (size_t)tabSlots + 15) & ~(size_t)15;
-}
+// The LDS of one pose of k_rigid with WP waves per pose: a super-chunk's beads'
+// force and energy, the class-ordered queue and its counters, pair counts.
+template <int WP>
+struct RigidLDS {
+    static constexpr unsigned kChunks = WP > 4 ? 3 : kQueueChunks;  // per wave
+    static constexpr unsigned kSuper = 64 * kChunks * WP;
+    float4 f[kSuper];
+    unsigned short q[kSuper];
+    unsigned cc[queue_counters<Classes16>(kSuper)];
+    unsigned cnt[WP][2];
+};
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_rigid(DProt rec, DProt lig, DGrid inner, DGrid outer,
-                                               DNL nl, DPar par, const float* __restrict__ dofs,
-                                               float* __restrict__ res, unsigned n,
-                                               unsigned tabSlots,
-                                               const unsigned* __restrict__ order,
-                                               uint2* __restrict__ counts) {
+// WP waves per pose: one (four poses per workgroup) or, for calls of few poses,
+// a workgroup of four or eight.  Every per-bead sum and the bead-order
+// reductions are the same in any of them: the same bits.
+template <int WP>
+__global__ __launch_bounds__(WP > 4 ? 64 * WP : 256) __attribute__((amdgpu_waves_per_eu(4))) void k_rigid(
+    DProt rec, DProt lig, DGrid inner, DGrid outer, DNL nl, DPar par, const float* __restrict__ dofs,
+    float* __restrict__ res, unsigned n, unsigned tabBytes, const unsigned* __restrict__ order,
+    uint2* __restrict__ counts) {
     extern __shared__ __align__(16) att_pair_params s_tab[];
+    using LDS = RigidLDS<WP>;
     const PairTab tab = stage_table(par, s_tab);
     __syncthreads();
-    const unsigned lane = threadIdx.x & (kWave - 1);
-    const unsigned wave = threadIdx.x / kWave;
-    char* wb = reinterpret_cast<char*>(s_tab) + rigid_wave_offset(tabSlots) + wave * kRigidWaveBytes;
-    float4* s_f = reinterpret_cast<float4*>(wb);
-    unsigned short* s_q = reinterpret_cast<unsigned short*>(s_f + kRigidSuper);
-    unsigned* s_cc = reinterpret_cast<unsigned*>(s_q + kRigidSuper);
+    constexpr unsigned nthr = kWave * WP;
+    const unsigned group = threadIdx.x / nthr, tid = threadIdx.x % nthr;  // group: pose of the workgroup
+    const unsigned lane = tid & (kWave - 1), wave = tid / kWave;
+    LDS& L = reinterpret_cast<LDS*>(reinterpret_cast<char*>(s_tab) + tabBytes)[group];
+    float4* s_f = L.f;
+    auto sync = [] {
+        if constexpr (WP == 1) wave_sync(); else __syncthreads();
+    };
     const unsigned wg = order ? xcd_slot(blockIdx.x, gridDim.x) : blockIdx.x;
-    const unsigned slot = wg * (blockDim.x / kWave) + wave;
-    if (slot >= n) return;  // uniform per wave; no workgroup barrier follows
+    const unsigned slot = wg * (blockDim.x / nthr) + group;
+    if (slot >= n) return;  // uniform per pose; with one wave per pose no workgroup barrier follows
     const unsigned pose = order ? order[slot] : slot;
     const float* d = dofs + 6 * (size_t)pose;
     const float tx = uniform(d[0]), ty = uniform(d[1]), tz = uniform(d[2]);
@@ -65,28 +73,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     };
     float red = 0.f;  // the reference's reduction held by this lane (reduce_beads_ref)
     unsigned listed = 0, inside = 0;  // this lane's pair counts (counts != nullptr)
-    const unsigned span = super_chunk(lig.n, kRigidSuper);
+    const unsigned span = super_chunk(lig.n, LDS::kSuper);
     for (unsigned sc = 0; sc < lig.n; sc += span) {
         const unsigned m = min(span, lig.n - sc);
         // P1: one bead per lane: rotate_translate, potForce, the list's cell.
         const unsigned padded = (m + kReduceStep - 1) & ~(kReduceStep - 1);
-        if (m + lane < padded) s_f[m + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (m + tid < padded) s_f[m + tid] = make_float4(0.f, 0.f, 0.f, 0.f);
         unsigned classes = 0;
-        for (unsigned k = lane, u = 0; k < m; k += kWave, ++u) {
+        for (unsigned k = tid, u = 0; k < m; k += nthr, ++u) {
             float4 x;
             const V3 p = place(sc + k, x);
             s_f[k] = pot_bead(inner, outer, p.x, p.y, p.z, lig.mtype[sc + k], x.w, nullptr);
             classes = pack_class<Classes16>(classes, u, nl_cell(nl, p.x, p.y, p.z, lig.type[sc + k]).x);
         }
-        wave_sync();
+        sync();
         // P2: beads with a list, longest lists first.
-        const unsigned qn = class_queue<Classes16, 1, kQueueChunks>(classes, m, s_q, s_cc, lane, wave_sync);
+        const unsigned qn = class_queue<Classes16, WP, LDS::kChunks>(classes, m, L.q, L.cc, tid, sync);
         // P3: one bead per quad of lanes walks its list in the reference's
         // order (NLPotForce); its sums are added to the bead's grid values as
         // outLig[i] += fAcc.
-        for (unsigned q0 = 0; q0 < qn; q0 += kWave / 4) {
-            if (q0 + (lane >> 2) < qn) {
-                const unsigned k = s_q[q0 + (lane >> 2)];
+        for (unsigned q0 = 0, round = 0; q0 < qn; q0 += nthr / 4, ++round) {
+            const unsigned item = q0 + quad_group<WP>(tid, round);
+            if (item < qn) {
+                const unsigned k = L.q[item];
                 float4 x;
                 const V3 p = place(sc + k, x);
                 const unsigned lt = lig.type[sc + k];
@@ -101,22 +110,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
                 }
             }
         }
-        wave_sync();
+        sync();
         // P4: reducePotForce and reduceTorque, in bead order.
-        red = reduce_beads_ref(red, lane, s_f, lig, sc, m);
-        wave_sync();  // the super-chunk's arrays are reused
+        if (wave == 0) red = reduce_beads_ref(red, lane, s_f, lig, sc, m);
+        sync();  // the super-chunk's arrays are reused
     }
+    if (counts) {
+        listed = wave_sum_u(listed);
+        inside = wave_sum_u(inside);
+        if (lane == 0) { L.cnt[wave][0] = listed; L.cnt[wave][1] = inside; }
+        sync();
+    }
+    if (wave != 0) return;
     float o[7];
     finish_ref(red, t, o);
     if (lane == 0) {
         float* r = res + 7 * (size_t)pose;
 #pragma unroll
         for (int q = 0; q < 7; ++q) r[q] = o[q];
-    }
-    if (counts) {
-        listed = wave_sum_u(listed);
-        inside = wave_sum_u(inside);
-        if (lane == 0) counts[pose] = make_uint2(listed, inside);
+        if (counts) {
+            uint2 c = make_uint2(0u, 0u);
+            for (int w = 0; w < WP; ++w) { c.x += L.cnt[w][0]; c.y += L.cnt[w][1]; }
+            counts[pose] = c;
+        }
     }
 }
 
@@ -521,14 +537,23 @@ hipError_t launch_copy(void* dst, const void* src, size_t n16, hipStream_t s) {
 
 hipError_t launch_rigid(const DProt& rec, const DProt& lig, const DGrid& inner, const DGrid& outer,
                         const DNL& nl, const DPar& par, const float* dofs, float* res, unsigned n,
-                        const unsigned* order, uint2* counts, hipStream_t s) {
+                        const unsigned* order, uint2* counts, unsigned numCU, hipStream_t s) {
     if (n == 0) return hipSuccess;
-    const unsigned posesPerBlock = 4;
-    const unsigned blocks = (n + posesPerBlock - 1) / posesPerBlock;
     const unsigned slots = par.T <= kMaxTypesLDS ? par.T * par.T : 0;
-    const size_t lds = rigid_wave_offset(slots) + posesPerBlock * kRigidWaveBytes;
-    hipLaunchKernelGGL(k_rigid, dim3(blocks), dim3(256), lds, s, rec, lig, inner, outer, nl, par,
-                       dofs, res, n, slots, order, counts);
+    const unsigned tab = (unsigned)((sizeof(att_pair_params) * (size_t)slots + 15) & ~(size_t)15);
+#define ATT_LAUNCH_RIGID(WP, POSES)                                                              \
+    hipLaunchKernelGGL(k_rigid<WP>, dim3((n + POSES - 1) / POSES), dim3(kWave * WP * POSES),     \
+                       tab + POSES * sizeof(RigidLDS<WP>), s, rec, lig, inner, outer, nl, par,   \
+                       dofs, res, n, tab, order, counts)
+    // Eight waves per pose while the CUs are not full (512 poses 1000/300: 40
+    // us, 49 on four, 122 on one; 1024: 81, 62, 128), four while they are hardly
+    // (2048: 110 on four, 142 on one; 4096: 208, 212, but 94 -> 120 for 300/80), and for
+    // ligands that are more than one super-chunk of one wave (8192 poses 3000/800:
+    // 955 -> 846).
+    if (n <= 2 * numCU) ATT_LAUNCH_RIGID(8, 1);
+    else if (n <= 8 * numCU || lig.n > RigidLDS<1>::kSuper) ATT_LAUNCH_RIGID(4, 1);
+    else ATT_LAUNCH_RIGID(1, 4);
+#undef ATT_LAUNCH_RIGID
     return hipGetLastError();
 }
 

@@ -417,6 +417,7 @@ bool att_server::step(Job* j) {
         }
         j->finishing = true;
     } else {
+        if (j->rounds > 0) att_minjob_set_running(j->mj, runningPoses);
         const int r = std::min(kRoundsPerChunk, limit - j->rounds);
         if (att_minjob_rounds(ctx, j->mj, r, j->stream) != ATT_OK ||
             att_minjob_running(ctx, j->mj, static_cast<unsigned*>(j->pinned), j->stream) != ATT_OK ||

@@ -404,6 +404,10 @@ att_status att_minjob_start(att_ctx* ctx, att_minjob* job, const float* d_dofs, 
 att_status att_minjob_rounds(att_ctx* ctx, att_minjob* job, int rounds, void* stream);
 int att_minjob_round_limit(const att_minjob* job);
 att_status att_minjob_running(att_ctx* ctx, att_minjob* job, unsigned* h_count, void* stream);
+/* Tells the job that at most `running` poses still run (a count that
+ * att_minjob_running copied): rounds of few poses then get more waves per
+ * pose.  Results do not depend on it. */
+void att_minjob_set_running(att_minjob* job, unsigned running);
 att_status att_minjob_destroy(att_ctx* ctx, att_minjob* job);
 
 /* Library build identification (arch, flags). */

@@ -77,3 +77,22 @@ def test_forward_walk_by_quads_is_the_reference_order(ctx, W, O, nl, mr, ml):
     d6 = np.ascontiguousarray(wl.dofs[:, :6])
     rigid = ctx.score_rigid(hs, d6)
     assert np.array_equal(rigid.view(np.uint32), O.score_rigid(wl, d6, nthreads=8).view(np.uint32))
+
+
+@pytest.mark.parametrize("nl, mr, ml", [(80, 0, 0), (300, 0, 0), (400, 0, 0), (70, 2, 3), (300, 5, 5),
+                                        (400, 4, 0), (600, 8, 10)])
+def test_call_size_changes_no_bit(ctx, W, nl, mr, ml):
+    """Few poses per call get more waves per pose: every pose scores the same
+    bits in one large call and in calls of every width (the widths change
+    between 512 and 2048 poses on 256 CUs, and with the ligand's size)."""
+    n = 4300
+    wl = W.make_workload("call size", 440 + nl + mr, 250, nl, n, mr, ml)
+    hs = ctx.upload_workload(wl)
+    whole = ctx.adjoint(hs, wl.dofs)
+    rigid = np.ascontiguousarray(wl.dofs[:, :6])
+    score = ctx.score_rigid(hs, rigid)
+    for a, b in ((0, 1), (1, 513), (513, 513 + 1024), (1537, 1537 + 2049)):
+        part = ctx.adjoint(hs, wl.dofs[a:b])
+        assert np.array_equal(part.view(np.uint32), whole[a:b].view(np.uint32)), (a, b)
+        part = ctx.score_rigid(hs, rigid[a:b])
+        assert np.array_equal(part.view(np.uint32), score[a:b].view(np.uint32)), (a, b)
