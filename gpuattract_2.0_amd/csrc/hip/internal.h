@@ -111,6 +111,8 @@ struct MinRun {
     unsigned ds, os;   // DOF and result record widths (26/27 or 6/7)
     unsigned* list;    // next round: pose of each request slot
     unsigned* count;   // next round: number of requests
+    unsigned* countNext;   // launch_min_start: the round's after it, set to 0
+    unsigned* countAfter;  // launch_min_step: likewise (three counters take turns)
     float* req;        // next round: requested points as DOF records
     float* dofsOut;    // npose * ds: last evaluated DOFs
     float* eLast;      // npose: their energy

@@ -455,56 +455,61 @@ att_status att_upload_protein(att_ctx* c, const att_protein_desc* d, att_handle*
     o->maxType = *std::max_element(d->type, d->type + n);
     if (o->maxType > 0xFFFFu) return fail(c, ATT_ERR_INVALID, "bead type exceeds 65535");
     o->maxMType = *std::max_element(d->mappedType, d->mappedType + n);
-    float4* dpos;
-    unsigned *dtype, *dmtype;
-    att_status st;
-    if ((st = dev_copy(c, o.get(), pos.data(), n, &dpos)) != ATT_OK) return st;
-    if ((st = dev_copy(c, o.get(), d->type, n, &dtype)) != ATT_OK) return st;
-    if ((st = dev_copy(c, o.get(), d->mappedType, n, &dmtype)) != ATT_OK) return st;
-    // the same coordinates by component, and ones, padded with zeros
+    // One allocation and one copy: the arrays one after the other, 256-byte
+    // aligned.
+    const size_t nM = (size_t)n * M;
     const unsigned ns = (n + 63u) & ~63u;
-    std::vector<float> soa4(4 * (size_t)ns, 0.f);
-    for (unsigned i = 0; i < n; ++i) {
-        for (unsigned k = 0; k < 3; ++k) soa4[(size_t)k * ns + i] = d->xyz[(size_t)k * n + i];
-        soa4[3 * (size_t)ns + i] = 1.f;
-    }
-    float* dsoa4;
-    if ((st = dev_copy(c, o.get(), soa4.data(), soa4.size(), &dsoa4)) != ATT_OK) return st;
-    o->d.soa = dsoa4;
-    o->d.ns = ns;
-    o->d.pos = dpos;
-    o->d.type = dtype;
-    o->d.mtype = dmtype;
-    o->d.n = n;
-    o->d.M = M;
+    const unsigned rowT = (3 * M + 4) / 4;  // float4 per padded row {type, modes}
+    size_t bytes = 0;
+    auto place = [&](size_t b) {
+        const size_t at = bytes;
+        bytes = (bytes + b + 255) & ~(size_t)255;
+        return at;
+    };
+    const size_t oPos = place(sizeof(float4) * n), oType = place(4 * (size_t)n),
+                 oMType = place(4 * (size_t)n), oSoa = place(16 * (size_t)ns),
+                 oRows = place(sizeof(float4) * n * rowT), oModes = place(12 * nM),
+                 oForce = place(4 * (size_t)M);
+    std::vector<float4> host((bytes + 15) / 16, make_float4(0.f, 0.f, 0.f, 0.f));
+    char* h = reinterpret_cast<char*>(host.data());
+    std::memcpy(h + oPos, pos.data(), sizeof(float4) * n);
+    std::memcpy(h + oType, d->type, 4 * (size_t)n);
+    std::memcpy(h + oMType, d->mappedType, 4 * (size_t)n);
+    // the same coordinates by component, and ones, padded with zeros
+    float* soa = reinterpret_cast<float*>(h + oSoa);
+    for (unsigned k = 0; k < 3; ++k) std::memcpy(soa + (size_t)k * ns, d->xyz + (size_t)k * n, 4 * (size_t)n);
+    std::fill_n(soa + 3 * (size_t)ns, n, 1.f);
     // rows {type, modes} for the neighbour-list gathers; without modes too, for
     // a rigid body scored with a flexible one.  A bead with a non-finite mode
     // has no finite distance to anything, so none of its pairs counts: its row
     // is zero (type 0), so that the walks' masked sums stay finite.
-    const size_t nM = (size_t)n * M;
-    const unsigned rowT = (3 * M + 4) / 4;  // float4 per padded row
-    std::vector<float> soa(3 * nM), rows((size_t)n * rowT * 4, 0.f);
+    float* rows = reinterpret_cast<float*>(h + oRows);
+    float* modes = reinterpret_cast<float*>(h + oModes);
     for (unsigned i = 0; i < n; ++i) std::memcpy(&rows[(size_t)i * rowT * 4], &d->type[i], 4);
     std::vector<unsigned> bad;
     for (unsigned cc = 0; cc < 3; ++cc)
         for (unsigned i = 0; i < n; ++i)
             for (unsigned m = 0; m < M; ++m) {
                 const float v = d->modes[cc * nM + (size_t)i * M + m];
-                soa[(cc * M + m) * (size_t)n + i] = v;
+                modes[(cc * M + m) * (size_t)n + i] = v;
                 rows[(size_t)i * rowT * 4 + 1 + 3 * m + cc] = v;
                 if (!std::isfinite(v)) bad.push_back(i);
             }
     for (unsigned i : bad) std::fill_n(&rows[(size_t)i * rowT * 4], (size_t)rowT * 4, 0.f);
-    float *dsoa, *dmf;
-    float4* drows;
-    if ((st = dev_copy(c, o.get(), soa.data(), soa.size(), &dsoa)) != ATT_OK) return st;
-    if ((st = dev_copy(c, o.get(), reinterpret_cast<const float4*>(rows.data()), (size_t)n * rowT,
-                       &drows)) != ATT_OK)
-        return st;
-    if ((st = dev_copy(c, o.get(), d->modeForce, M, &dmf)) != ATT_OK) return st;
-    o->d.modes = dsoa;
-    o->d.modesT = drows;
-    o->d.modeForce = dmf;
+    if (M) std::memcpy(h + oForce, d->modeForce, 4 * (size_t)M);
+    char* dev;
+    att_status st;
+    if ((st = dev_copy(c, o.get(), const_cast<const char*>(h), bytes, &dev)) != ATT_OK) return st;
+    o->d.pos = reinterpret_cast<const float4*>(dev + oPos);
+    o->d.soa = reinterpret_cast<const float*>(dev + oSoa);
+    o->d.type = reinterpret_cast<const unsigned*>(dev + oType);
+    o->d.mtype = reinterpret_cast<const unsigned*>(dev + oMType);
+    o->d.modes = reinterpret_cast<const float*>(dev + oModes);
+    o->d.modesT = reinterpret_cast<const float4*>(dev + oRows);
+    o->d.modeForce = reinterpret_cast<const float*>(dev + oForce);
+    o->d.n = n;
+    o->d.ns = ns;
+    o->d.M = M;
     o->d.rowT = rowT;
     *out = store(c, std::move(o));
     return ATT_OK;
@@ -1616,7 +1621,7 @@ struct att_minjob {
     void* mem = nullptr;
     size_t bytes = 0;
     unsigned* list[2] = {nullptr, nullptr};
-    unsigned* count[2] = {nullptr, nullptr};
+    unsigned* count[3] = {nullptr, nullptr, nullptr};  // of round r: count[r % 3]
     float* req[2] = {nullptr, nullptr};
     float* res = nullptr;
     int cur = 0;
@@ -1630,7 +1635,7 @@ void minjob_layout(size_t n, int dim, unsigned ds, unsigned os, size_t* parts) {
     parts[0] = al256(sizeof(double) * n * va_elements(dim));
     parts[1] = al256(sizeof(VaState) * n);
     parts[2] = al256(sizeof(unsigned) * n);
-    parts[3] = al256(2 * sizeof(unsigned));
+    parts[3] = al256(3 * sizeof(unsigned));
     parts[4] = al256(sizeof(float) * n * ds);
     parts[5] = al256(sizeof(float) * n * os);
 }
@@ -1688,6 +1693,7 @@ att_status att_minjob_create(att_ctx* c, att_handle hr, att_handle hl, att_handl
     j->list[1] = reinterpret_cast<unsigned*>(base + pt[0] + pt[1] + pt[2]);
     j->count[0] = reinterpret_cast<unsigned*>(base + pt[0] + pt[1] + 2 * pt[2]);
     j->count[1] = j->count[0] + 1;
+    j->count[2] = j->count[0] + 2;
     j->req[0] = reinterpret_cast<float*>(base + pt[0] + pt[1] + 2 * pt[2] + pt[3]);
     j->req[1] = reinterpret_cast<float*>(base + pt[0] + pt[1] + 2 * pt[2] + pt[3] + pt[4]);
     j->res = reinterpret_cast<float*>(base + pt[0] + pt[1] + 2 * pt[2] + pt[3] + 2 * pt[4]);
@@ -1723,6 +1729,7 @@ att_status att_minjob_start(att_ctx* c, att_minjob* j, const float* d_dofs, void
     j->rounds = 0;
     j->running = j->R.npose;
     j->R.list = j->list[0]; j->R.count = j->count[0]; j->R.req = j->req[0];
+    j->R.countNext = j->count[1];
     ATT_HIP(c, launch_min_start(j->R, d_dofs, s));
     return ATT_OK;
 }
@@ -1736,10 +1743,13 @@ att_status att_minjob_rounds(att_ctx* c, att_minjob* j, int rounds, void* stream
         const int cur = j->cur, nxt = cur ^ 1;
         const int w = j->running <= j->few ? 1 : 0;
         j->P.dofs = j->req[cur];
-        j->P.nDev = j->count[cur];
+        unsigned* const now = j->count[j->rounds % 3];
+        j->P.nDev = now;
         ATT_HIP(c, launch_adjoint(j->P, j->modes, nullptr, j->blocks[w], j->width[w], j->dyn, s));
-        j->R.list = j->list[nxt]; j->R.count = j->count[nxt]; j->R.req = j->req[nxt];
-        ATT_HIP(c, launch_min_step(j->R, j->list[cur], j->count[cur], j->req[cur], j->res, s));
+        j->R.list = j->list[nxt]; j->R.req = j->req[nxt];
+        j->R.count = j->count[(j->rounds + 1) % 3];
+        j->R.countAfter = j->count[(j->rounds + 2) % 3];
+        ATT_HIP(c, launch_min_step(j->R, j->list[cur], now, j->req[cur], j->res, s));
         j->cur = nxt;
         ++j->rounds;
     }
@@ -1757,7 +1767,7 @@ att_status att_minjob_running(att_ctx* c, att_minjob* j, unsigned* h_count, void
     if (!j || !h_count) return fail(c, ATT_ERR_INVALID, "null argument");
     ATT_HIP(c, hipSetDevice(c->device));
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
-    ATT_HIP(c, hipMemcpyAsync(h_count, j->count[j->cur], sizeof(unsigned), hipMemcpyDeviceToHost, s));
+    ATT_HIP(c, hipMemcpyAsync(h_count, j->count[j->rounds % 3], sizeof(unsigned), hipMemcpyDeviceToHost, s));
     return ATT_OK;
 }
 

@@ -28,7 +28,8 @@ struct VaState {
 enum VaPc : int { kVaFresh = 0, kVaAtStart = 1, kVaInLine = 2, kVaFinished = 3 };
 
 // One pose's vectors: vector v, element k at st[(v * nmax + k) * stride];
-// the packed factors after the vectors.
+// the packed factors after the vectors.  The state machine below takes any view
+// with v() and h().
 struct VaView {
     double* st;
     size_t stride;
@@ -51,7 +52,8 @@ __host__ __device__ inline double va_max(double a, double b) { return b > a ? b 
 // H <- H + sig z z^T on the factors (mc11a): with mk = 1 the vector W holds
 // L^-1 z from the last solve.  `z` and `w` name vectors of the view and may
 // be the same vector.
-__host__ __device__ inline void va_update(const VaView& V, int n, int z, double sig, int w,
+template <class View>
+__host__ __device__ inline void va_update(const View& V, int n, int z, double sig, int w,
                                           int& ir, int mk, double eps) {
     if (n <= 1) {
         V.h(0) = V.h(0) + sig * V.v(z, 0) * V.v(z, 0);
@@ -160,7 +162,8 @@ __host__ __device__ inline void va_update(const VaView& V, int n, int z, double 
 }
 
 // z <- H^-1 z (mc11e); W receives L^-1 z.
-__host__ __device__ inline void va_solve(const VaView& V, int n, int z) {
+template <class View>
+__host__ __device__ inline void va_solve(const View& V, int n, int z) {
     V.v(kVaW, 0) = V.v(z, 0);
     if (n <= 1) {
         V.v(z, 0) = V.v(z, 0) / V.h(0);
@@ -192,8 +195,9 @@ __host__ __device__ inline void va_solve(const VaView& V, int n, int z) {
 // f, g: the objective and its gradient at the point last requested (ignored
 // when fresh).  Returns true with the next point in `req`, or false when the
 // minimizer has finished (the last requested point is then its result).
-__host__ __device__ inline bool va_resume(VaState& s, const VaView& V, int n, int ivmax, double f,
-                                          const double* g, double* req) {
+template <class View, class In, class Out>
+__host__ __device__ inline bool va_advance(VaState& s, const View& V, int n, int ivmax, double f,
+                                           In g, Out req) {
     enum { L110, L135, L170, LEVAL, L240, L270, L280, LEND };
     int at;
     switch (s.pc) {
@@ -356,6 +360,11 @@ __host__ __device__ inline bool va_resume(VaState& s, const VaView& V, int n, in
                 return false;
         }
     }
+}
+
+__host__ __device__ inline bool va_resume(VaState& s, const VaView& V, int n, int ivmax, double f,
+                                          const double* g, double* req) {
+    return va_advance(s, V, n, ivmax, f, g, req);
 }
 
 }  // namespace att

@@ -124,7 +124,7 @@ size_t energy_bytes(size_t nx, size_t ny, size_t nz, size_t numGrids) {
 
 size_t protein_bytes(const as::ProteinData& p) {
     const size_t rowT = (3 * (size_t)p.numModes + 4) / 4;
-    return p.n * (16 + 8 + 16 * rowT + 12 * (size_t)p.numModes) + 4096;
+    return p.n * (16 + 8 + 16 + 16 * rowT + 12 * (size_t)p.numModes) + 4096;
 }
 
 size_t receptor_bytes(const Receptor& r) {

@@ -96,3 +96,16 @@ def test_call_size_changes_no_bit(ctx, W, nl, mr, ml):
         assert np.array_equal(part.view(np.uint32), whole[a:b].view(np.uint32)), (a, b)
         part = ctx.score_rigid(hs, rigid[a:b])
         assert np.array_equal(part.view(np.uint32), score[a:b].view(np.uint32)), (a, b)
+
+
+@pytest.mark.parametrize("n, mr, ml", [(1, 0, 0), (17, 10, 10), (33, 10, 8), (15, 2, 1)])
+def test_minimizer_steps_in_lds(ctx, W, O, n, mr, ml):
+    """Pose counts around the 16 (or, with 25 variables or more, 8) poses whose
+    minimizers a workgroup advances: the oracle's trajectories."""
+    wl = W.make_workload("lds steps", 460 + n, 200, 60, n, mr, ml, with_lig_grid=False)
+    d, el, eb, nf = ctx.minimize(ctx.upload_workload(wl), wl.dofs, 25)
+    od, oel, oeb, onf = O.minimize_kernel_order(wl, ivmax=25)
+    assert np.array_equal(nf, onf)
+    assert np.array_equal(d.view(np.uint32), od.astype(np.float32).view(np.uint32)[:, :d.shape[1]])
+    assert np.array_equal(el.view(np.uint32), oel.astype(np.float32).view(np.uint32))
+    assert np.array_equal(eb.view(np.uint32), oeb.astype(np.float32).view(np.uint32))
