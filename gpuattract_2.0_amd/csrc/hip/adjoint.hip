@@ -88,8 +88,7 @@ struct PGrad {
     unsigned* key;                // kPgRecords: per (slot, bead) grid-cell record
     float4* pos4;                 //   {x, y, z, w}, or
     float3* pos3;                 //   {x, y, z} when the call has no weights
-    unsigned cellsIn;             //   key = (cell, inner cells first) * T + type - 1
-    unsigned invalid;             //   key of a bead without a grid term
+    PgKeys keys;
 };
 
 
@@ -128,13 +127,13 @@ __device__ __forceinline__ float grid_adj_one(const DGrid& g, const DBasis& b, f
     if (PG == kPgRecords) {
         if (type - 1u < pg.T) {
             const unsigned o = (iz * (g.ny - 1) + iy) * (g.nx - 1) + ix;
-            pg.key[rec] = (cellBase + o) * pg.T + (type - 1);
+            pg.key[rec] = pg.keys.key(cellBase + o, type);
             if (pg.pos3)
                 pg.pos3[rec] = make_float3(px, py, pz);
             else
                 pg.pos4[rec] = make_float4(px, py, pz, pg.w);
         } else {
-            pg.key[rec] = pg.invalid;
+            pg.key[rec] = pg.keys.invalid;
         }
     }
     if (PG == kPgFused && b.oct && type - 1u < pg.T) {
@@ -187,12 +186,12 @@ __device__ __forceinline__ float grid_adj(const DGrid& inner, const DGrid& outer
                                           size_t rec) {
     G = make_float3(0.f, 0.f, 0.f);
     if (mtype == 0) {
-        if (PG == kPgRecords) pg.key[rec] = pg.invalid;
+        if (PG == kPgRecords) pg.key[rec] = pg.keys.invalid;
         return 0.f;
     }
     const bool in = !grid_out(inner, px, py, pz);
     if (!in && grid_out(outer, px, py, pz)) {
-        if (PG == kPgRecords) pg.key[rec] = pg.invalid;
+        if (PG == kPgRecords) pg.key[rec] = pg.keys.invalid;
         return 0.f;
     }
     DGrid g{};
@@ -210,7 +209,7 @@ __device__ __forceinline__ float grid_adj(const DGrid& inner, const DGrid& outer
     DBasis b{};
     b.oct = in ? bin.oct : bout.oct;
     b.nb = in ? bin.nb : bout.nb;
-    return grid_adj_one<PG>(g, b, px, py, pz, mtype, type, charge, G, pg, in ? 0u : pg.cellsIn,
+    return grid_adj_one<PG>(g, b, px, py, pz, mtype, type, charge, G, pg, in ? 0u : pg.keys.cellsIn,
                             rec, inner.octE != nullptr);
 }
 
@@ -381,7 +380,7 @@ __device__ __forceinline__ void adjoint_pose(const PairDesc& P, unsigned pose, P
     const float tx = uniform(d[0]), ty = uniform(d[1]), tz = uniform(d[2]);
     const float wp = P.wts ? P.wts[pose] : 1.f;
     const PGrad pg{PG != kPgNone ? s_pg + wave * 3 * par.T * par.T : nullptr, tab, par.T, wp,
-                   P.recKey, P.recPos4, P.recPos3, P.recCellsIn, P.recInvalid};
+                   P.recKey, P.recPos4, P.recPos3, P.recKeys};
     float ampR[MA], ampL[MA];
 #pragma unroll
     for (int m = 0; m < MA; ++m) {

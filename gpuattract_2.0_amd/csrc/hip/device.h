@@ -691,6 +691,16 @@ __host__ __device__ constexpr size_t adjoint_pg_offset(unsigned tabSlots) {
     return (sizeof(att_pair_params) * (size_t)tabSlots + 15) & ~(size_t)15;
 }
 
+// Key of a grid-cell record: cells (inner grid first) in buckets of 2^cellBits,
+// key = bucket << lowBits | (type - 1) << cellBits | cell in its bucket.
+struct PgKeys {
+    unsigned cellsIn, cellBits, lowBits;
+    unsigned invalid;  // number of buckets << lowBits: no grid term
+    __host__ __device__ unsigned key(unsigned cell, unsigned type) const {
+        return (cell >> cellBits) << lowBits | (type - 1u) << cellBits | (cell & ((1u << cellBits) - 1u));
+    }
+};
+
 // Everything the adjoint of one pose needs about its receptor-ligand pair.
 struct PairDesc {
     DProt rec, lig;
@@ -705,14 +715,14 @@ struct PairDesc {
     const unsigned* nDev;  // when set, the number of poses is read here at launch (<= n)
     const unsigned* order; // when set, a spatial permutation of the poses (XCD ranges)
     // Grid part of the parameter gradient as records (when set): slot i's bead
-    // k writes recKey/recPos[i * lig.n + k]; keys (cell * T + type - 1, inner
-    // cells first) below recInvalid, recInvalid for beads without a grid term.
+    // k writes recKey/recPos[i * lig.n + k]; keys as PgKeys packs them, below
+    // recKeys.invalid, that value for beads without a grid term.
     // Positions as {x, y, z, w} (recPos4), or {x, y, z} when the call has no
     // weights (recPos3; w = 1).
     unsigned* recKey;
     float4* recPos4;
     float3* recPos3;
-    unsigned recCellsIn, recInvalid;
+    PgKeys recKeys;
     // when set, per pose {listed neighbours of the beads walked, pairs inside
     // the plateau}
     uint2* counts;

@@ -66,6 +66,11 @@ unsigned adjoint_blocks_per_cu(unsigned mm, AdjWidth w, bool batch, size_t lds, 
 // (cell, type) after sorting (kPgRecords; PairDesc.recKey set).
 constexpr int kPgNone = 0, kPgFused = 1, kPgRecords = 2;
 
+// The keys of a call's records (false: they do not fit 32 bits).
+bool pg_keys(size_t cellsIn, size_t cellsOut, unsigned T, PgKeys* keys);
+// Tables up to this many types take the bucket pass, larger ones the run pass.
+constexpr unsigned kPgBucketTypes = 32;
+
 // Scratch of the cell pass for `records` records: the adjoint's records
 // (keys, then positions) at the front, sort and reduction buffers after.
 struct PgCellBufs {
@@ -74,6 +79,7 @@ struct PgCellBufs {
     unsigned* keySorted;
     void* posSorted;
     bool weights;
+    // run pass only:
     unsigned* cellKey;   // runs of equal keys (per group of 64 sorted records), in order
     float* cellW;        // their summed corner weights, 8 per run
     unsigned* groupRuns; // runs per group of 64 records
@@ -81,14 +87,15 @@ struct PgCellBufs {
     void* temp;
     size_t tempBytes;
 };
-size_t pg_cells_bytes(size_t records, unsigned endBit, bool weights);
-PgCellBufs pg_cells_layout(void* scratch, size_t records, unsigned endBit, bool weights);
-// Cell pass over the records of P's k_adjoint launch: sort by key, sum the
-// corner weights of each run of equal keys (fixed order), then `blocks`
-// one-wave workgroups contract every run with its cell's basis values and
-// write one parameter row each to rows[0 .. blocks).
-hipError_t launch_pg_cells(const PairDesc& P, const PgCellBufs& B, size_t records, unsigned endBit,
-                           float* rows, unsigned blocks, hipStream_t s);
+size_t pg_cells_bytes(size_t records, const PgKeys& keys, unsigned T, bool weights);
+PgCellBufs pg_cells_layout(void* scratch, size_t records, const PgKeys& keys, unsigned T, bool weights);
+unsigned pg_cells_blocks(unsigned T, unsigned numCU);
+// Cell pass over the records of P's k_adjoint launch: the records sorted (by
+// bucket, or by key), the corner weights of each (cell, type) summed in a fixed
+// order and contracted with the cell's basis values by `blocks` one-wave
+// workgroups (pg_cells_blocks), one parameter row each in rows[0 .. blocks).
+hipError_t launch_pg_cells(const PairDesc& P, const PgCellBufs& B, size_t records, float* rows,
+                           unsigned blocks, hipStream_t s);
 
 // One pair: persistent grid of `blocks` workgroups of 64 * w.work threads.
 hipError_t launch_adjoint(const PairDesc& P, bool modes, float* pgPartial, unsigned blocks,

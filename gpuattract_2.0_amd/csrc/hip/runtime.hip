@@ -319,11 +319,10 @@ AdjWidth adjoint_width(const att_ctx* c, const DProt& rec, const DProt& lig, con
     return AdjWidth{order, order};
 }
 // Parameter-gradient records per call up to which the cell pass takes the
-// grid part (68 B of scratch per record without pose weights, 76 B with:
-// 9-10 GB at the cap), and the workgroups of that pass (one parameter row
-// each).
+// grid part (32 B of scratch per record, 40 with pose weights, and the sort's
+// own: 4-5 GB and that at the cap; 36 B more for tables of over kPgBucketTypes
+// types).
 constexpr size_t kPgRecordCap = (size_t)1 << 27;
-constexpr unsigned kPgCellBlocks = 2048;
 // Waves per pose of the flexible forward kernel (k_modes): with 384 ligand
 // beads or more, four (3000/800 beads, 5 + 5 modes: 100,000 poses 3% slower
 // than with two, a call of 100 poses 1.6x faster).  A function of the pair
@@ -821,24 +820,23 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
     const size_t records = pgrad ? n * (size_t)lig->d.n : 0;
     const size_t cellsIn = (size_t)(g->inner.nx - 1) * (g->inner.ny - 1) * (g->inner.nz - 1);
     const size_t cellsOut = (size_t)(g->outer.nx - 1) * (g->outer.ny - 1) * (g->outer.nz - 1);
-    const size_t invalid = (cellsIn + cellsOut) * p->d.T;
-    const bool useRec = records > 0 && records <= kPgRecordCap && invalid < 0xFFFFFFFFull &&
+    PgKeys keys{};
+    const bool useRec = records > 0 && records <= kPgRecordCap &&
+                        pg_keys(cellsIn, cellsOut, p->d.T, &keys) &&
                         sizeof(float) * cols <= c->maxLdsPerBlock;
     const int pgMode = !pgrad ? kPgNone : useRec ? kPgRecords : kPgFused;
     // persistent grid: as many workgroups as the device holds at once
     const size_t resident = (size_t)c->numCU * adjoint_blocks_per_cu(mm, width, false, dyn, pgMode);
     const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(n, resident));
-    const unsigned cellBlocks = useRec ? kPgCellBlocks : 0;
+    const unsigned cellBlocks = useRec ? pg_cells_blocks(p->d.T, c->numCU) : 0;
     // per-workgroup rows (the adjoint's, then the cell pass's), then the
     // reduction's group sums (8-byte aligned)
     const size_t rowBytes = (sizeof(float) * ((size_t)blocks + cellBlocks) * cols + 255) & ~(size_t)255;
     if (pgrad && (st = grow(c, &c->d_pg, &c->d_pg_cap, rowBytes + pgrad_group_bytes(cols))) != ATT_OK)
         return st;
-    unsigned endBit = 0;
-    while (endBit < 32 && (invalid >> endBit) != 0) ++endBit;
     const bool recW = d_w != nullptr;
     if (useRec &&
-        (st = grow(c, &c->d_rec, &c->d_rec_cap, pg_cells_bytes(records, endBit, recW))) != ATT_OK)
+        (st = grow(c, &c->d_rec, &c->d_rec_cap, pg_cells_bytes(records, keys, p->d.T, recW))) != ATT_OK)
         return st;
     if (n == 0) {
         if (pgrad) ATT_HIP(c, launch_fill_zero(d_pgrad, cols, s));
@@ -855,14 +853,13 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
     if ((st = pair_counts(c, n, &P.counts)) != ATT_OK) return st;
     PgCellBufs B{};
     if (useRec) {
-        B = pg_cells_layout(c->d_rec, records, endBit, recW);
+        B = pg_cells_layout(c->d_rec, records, keys, p->d.T, recW);
         P.recKey = B.key;
         if (recW)
             P.recPos4 = static_cast<float4*>(B.pos);
         else
             P.recPos3 = static_cast<float3*>(B.pos);
-        P.recCellsIn = (unsigned)cellsIn;
-        P.recInvalid = (unsigned)invalid;
+        P.recKeys = keys;
     }
     if (blocks >= 8 && (st = pose_order(c, d_dofs, P.dofStride, n, 4 * (size_t)blocks, s, &P.order)) != ATT_OK)
         return st;
@@ -871,7 +868,7 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
     float* rows = pgrad ? static_cast<float*>(c->d_pg) : nullptr;
     ATT_HIP(c, launch_adjoint(P, modes != 0, rows, blocks, width, dyn, s));
     if (useRec)
-        ATT_HIP(c, launch_pg_cells(P, B, records, endBit, rows + (size_t)blocks * cols, cellBlocks, s));
+        ATT_HIP(c, launch_pg_cells(P, B, records, rows + (size_t)blocks * cols, cellBlocks, s));
     if (pgrad)
         ATT_HIP(c, launch_pgrad_reduce(rows, blocks + cellBlocks, cols,
                                        reinterpret_cast<double*>(static_cast<char*>(c->d_pg) + rowBytes),

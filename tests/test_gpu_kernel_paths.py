@@ -109,3 +109,63 @@ def test_minimizer_steps_in_lds(ctx, W, O, n, mr, ml):
     assert np.array_equal(d.view(np.uint32), od.astype(np.float32).view(np.uint32)[:, :d.shape[1]])
     assert np.array_equal(el.view(np.uint32), oel.astype(np.float32).view(np.uint32))
     assert np.array_equal(eb.view(np.uint32), oeb.astype(np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("types, n, weights", [(1, 40, False), (2, 1, True), (12, 700, True),
+                                               (16, 90, False), (17, 90, True), (32, 90, False),
+                                               (33, 60, True), (40, 60, False)])
+def test_parameter_gradient_cell_pass(ctx, W, O, types, n, weights):
+    """One and two matrix tiles of types, full and not, and the run pass above
+    them; one workgroup's share from nothing to many buckets.  FP64 oracle to
+    1e-4 of the largest entry, the per-bead basis path (16 types at most) to
+    FP32 rounding (1e-5), and the same bits in a second call."""
+    wl = W.make_workload("cells", 500 + types, 300, 130, n, 0, 0, num_types=types,
+                         with_basis=True, shell=(8.0, 45.0), type0_frac=0.05)
+    hs = ctx.upload_workload(wl)
+    ctx.upload_basis(hs["grid"], wl)
+    w = np.linspace(-1.0, 2.0, n).astype(np.float32) if weights else None
+    T = wl.params.T
+    _, pg = ctx.adjoint(hs, wl.dofs, w=w, pgrad=True, T=T)
+    _, again = ctx.adjoint(hs, wl.dofs, w=w, pgrad=True, T=T)
+    assert np.array_equal(pg.view(np.uint32), again.view(np.uint32))
+    ref = O.adjoint(wl, w=None if w is None else w.astype(np.float64), pgrad=True)[1].reshape(-1)
+    assert np.abs(pg.reshape(-1) - ref).max() <= 1e-4 * np.abs(ref).max()
+    if T > 16:
+        return
+    d_in, d_w = ctx.to_device(wl.dofs), None if w is None else ctx.to_device(w)
+    d_out, d_pg = ctx.dev_alloc(n * 7 * 4), ctx.dev_alloc(3 * T * T * 4)
+    ctx.adjoint_dev_noalloc(hs, d_in.ptr, False, n, d_w and d_w.ptr, d_out.ptr, d_pg.ptr)
+    ctx.sync()
+    beads = ctx.to_host(d_pg, (3 * T * T,))
+    assert np.abs(pg.reshape(-1) - beads).max() <= 1e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("types", [12, 20])
+def test_parameter_gradient_basis_value_not_finite(ctx, W, types):
+    """It reaches the types of the beads beside it and no others: everything
+    that stays finite is what the finite basis gives (and, with 16 types or
+    fewer, finite in the per-bead basis path too)."""
+    wl = W.make_workload("cells inf", 540 + types, 300, 130, 12, 0, 0, num_types=types,
+                         with_basis=True, shell=(8.0, 30.0))
+    n, T = wl.dofs.shape[0], wl.params.T
+    hs = ctx.upload_workload(wl)
+    ctx.upload_basis(hs["grid"], wl)
+    clean = ctx.adjoint(hs, wl.dofs, pgrad=True, T=T)[1]
+    # receptor type 1: some points of both grids; infinite in the inner, NaN in the outer
+    nv = wl.rec_inner_basis.size // (2 * types)
+    wl.rec_inner_basis[0:nv:97] = np.inf
+    nv = wl.rec_outer_basis.size // (2 * types)
+    wl.rec_outer_basis[nv:2 * nv:151] = np.nan
+    hs = ctx.upload_workload(wl)
+    ctx.upload_basis(hs["grid"], wl)
+    pg = ctx.adjoint(hs, wl.dofs, pgrad=True, T=T)[1]
+    ok = np.isfinite(pg)
+    assert ok[T:].all() and ok[:, 2].all()
+    assert not ok[:T, :2].all() and ok[:T, :2].any()
+    assert np.abs(pg - clean)[ok].max() <= 1e-5 * np.abs(clean).max()
+    if T > 16:
+        return
+    d_in, d_out, d_pg = ctx.to_device(wl.dofs), ctx.dev_alloc(n * 28), ctx.dev_alloc(12 * T * T)
+    ctx.adjoint_dev_noalloc(hs, d_in.ptr, False, n, None, d_out.ptr, d_pg.ptr)
+    ctx.sync()
+    assert np.array_equal(np.isfinite(ctx.to_host(d_pg, (T * T, 3))), ok)
