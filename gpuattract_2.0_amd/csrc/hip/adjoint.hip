@@ -603,6 +603,37 @@ __global__ __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(adjoint
         first = (unsigned)(((unsigned long long)n * x) >> 3) + (blockIdx.x >> 3);
         end = (unsigned)(((unsigned long long)n * (x + 1)) >> 3);
     }
+    if (PG == kPgNone && ordered && P.queues) {
+        // After its first pose a workgroup draws from its eighth's queue, then
+        // from the others': such a call has few rounds of poses (four or more)
+        // of unequal work, and with fixed shares the last rounds leave part of
+        // the chip idle.  30001 rigid poses (1000/300 beads, 7 rounds) 668 ->
+        // 625 us, 10007 poses with 10 + 10 modes (6 rounds) 1753 -> 1708 us; one
+        // loop for both kinds of share, of more live registers, 645 and 1744.
+        // Which workgroup takes a pose changes no result of it; the sums of the
+        // parameter gradient would change, so there the shares are fixed.
+        __shared__ unsigned s_next[2];
+        unsigned i = first, x = blockIdx.x & 7u, parity = 0;
+        for (unsigned helped = 0;;) {
+            const bool have = i < end;
+            if (!have) {
+                if (++helped == 8) break;
+                x = (x + 1) & 7u;
+                end = (unsigned)(((unsigned long long)n * (x + 1)) >> 3);
+            }
+            unsigned drawn = 0;  // in flight while the pose is scored
+            if (threadIdx.x == 0)
+                drawn = (unsigned)(((unsigned long long)n * x) >> 3) + ((gridDim.x - x + 7u) >> 3) +
+                        atomicAdd(&P.queues[x * kQueueStride], 1u);
+            if (have) adjoint_pose<MM, VW, PW, PG>(P, P.order[i], S, tab, s_pg, 0);
+            // two slots in turn: one is read while the other is written
+            if (threadIdx.x == 0) s_next[parity] = drawn;
+            __syncthreads();
+            i = (unsigned)__builtin_amdgcn_readfirstlane((int)s_next[parity]);
+            parity ^= 1u;
+        }
+        return;
+    }
     // grid-cell records of slot i (kPgRecords) start at i * ligand beads
     for (unsigned i = first; i < end; i += step)
         adjoint_pose<MM, VW, PW, PG>(P, P.order ? P.order[i] : i, S, tab, s_pg, (size_t)i * P.lig.n);

@@ -148,7 +148,8 @@ __device__ __forceinline__ void torque_reduce(float cSSI, float cPHI, float sSSI
 
 // A value that is the same on every lane, in a scalar register: a pose's
 // rotation, translation and amplitudes would otherwise hold some 30 vector
-// registers through the walks (and spill: 96 -> 0 B per lane in the 5-mode adjoint).
+// registers through the walks (the 10-mode adjoint spilled 84 B per lane with
+// them there and spills none now).
 __device__ __forceinline__ float uniform(float v) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
@@ -701,6 +702,8 @@ struct PgKeys {
     }
 };
 
+constexpr unsigned kQueueStride = 64;  // words: counters lie in cache lines of their own
+
 // Everything the adjoint of one pose needs about its receptor-ligand pair.
 struct PairDesc {
     DProt rec, lig;
@@ -714,6 +717,7 @@ struct PairDesc {
     unsigned dofStride, outStride, n, tabSlots;
     const unsigned* nDev;  // when set, the number of poses is read here at launch (<= n)
     const unsigned* order; // when set, a spatial permutation of the poses (XCD ranges)
+    unsigned* queues;      // and, when set, zeroed counters of the ranges, kQueueStride apart
     // Grid part of the parameter gradient as records (when set): slot i's bead
     // k writes recKey/recPos[i * lig.n + k]; keys as PgKeys packs them, below
     // recKeys.invalid, that value for beads without a grid term.

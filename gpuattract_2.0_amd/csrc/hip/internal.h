@@ -147,6 +147,7 @@ hipError_t launch_basis_octets(const float* b, float4* oct, unsigned nx, unsigne
 // Spatial pose order (order.hip): scratch bytes for n poses, and the launch
 // writing the permutation to `order`.
 size_t pose_order_scratch(unsigned n);
+unsigned* pose_order_queues(void* scratch);  // 8 counters (PairDesc::queues), zeroed by the launch
 hipError_t launch_pose_order(const float* dofs, unsigned stride, unsigned n, void* scratch,
                              size_t scratchBytes, unsigned* order, hipStream_t s);
 

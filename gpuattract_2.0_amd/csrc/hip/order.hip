@@ -3,7 +3,8 @@
 // Poses are sorted by the Morton code of their translation inside the poses'
 // bounding box (stable radix sort: a deterministic order).  The adjoint kernel
 // gives each XCD a contiguous range of that order, so the poses one XCD holds
-// at a time lie close together and share the grid lines in its L2; results are
+// at a time lie close together and share the grid lines in its L2 (and, without
+// parameter gradients, its workgroups draw them from the range's queue); results are
 // written to each pose's own slot, so the order changes no per-pose result.
 #include <rocprim/device/device_radix_sort.hpp>
 
@@ -27,6 +28,8 @@ __device__ inline unsigned spread10(unsigned v) {
 
 constexpr unsigned kBoxBlocks = 64;  // workgroups of the bounding-box pass
 constexpr size_t kBoxBytes = 2048;   // their partial boxes, at the front of the scratch
+constexpr size_t kQueueBytes = 8 * kQueueStride * sizeof(unsigned);  // the ranges' counters
+constexpr size_t kFrontBytes = kBoxBytes + kQueueBytes;
 static_assert(kBoxBlocks <= 64 && kBoxBlocks * 6 * sizeof(float) <= kBoxBytes, "box scratch");
 
 // Partial bounding boxes of the translations (dofs[i*stride + 0..2]): block b
@@ -67,8 +70,10 @@ __global__ __launch_bounds__(256) void k_pose_bbox(const float* __restrict__ dof
 __global__ __launch_bounds__(256) void k_pose_keys(const float* __restrict__ dofs, unsigned stride,
                                                    unsigned n, const float* __restrict__ part,
                                                    unsigned* __restrict__ keys,
-                                                   unsigned* __restrict__ idx) {
+                                                   unsigned* __restrict__ idx,
+                                                   unsigned* __restrict__ queues) {
     __shared__ float box[6];
+    if (blockIdx.x == 0 && threadIdx.x < 8) queues[threadIdx.x * kQueueStride] = 0u;
     if (threadIdx.x < 64) {
         float v[6];
         for (int k = 0; k < 6; ++k) v[k] = threadIdx.x < kBoxBlocks ? part[threadIdx.x * 6 + k]
@@ -99,7 +104,11 @@ size_t pose_order_scratch(unsigned n) {
     size_t temp = 0;
     (void)rocprim::radix_sort_pairs(nullptr, temp, (unsigned*)nullptr, (unsigned*)nullptr,
                                     (unsigned*)nullptr, (unsigned*)nullptr, n, 0, 30);
-    return kBoxBytes + 3 * sizeof(unsigned) * (size_t)n + ((temp + 255) & ~(size_t)255);
+    return kFrontBytes + 3 * sizeof(unsigned) * (size_t)n + ((temp + 255) & ~(size_t)255);
+}
+
+unsigned* pose_order_queues(void* scratch) {
+    return reinterpret_cast<unsigned*>(static_cast<char*>(scratch) + kBoxBytes);
 }
 
 hipError_t launch_pose_order(const float* dofs, unsigned stride, unsigned n, void* scratch,
@@ -107,14 +116,14 @@ hipError_t launch_pose_order(const float* dofs, unsigned stride, unsigned n, voi
     if (n == 0) return hipSuccess;
     char* p = static_cast<char*>(scratch);
     float* part = reinterpret_cast<float*>(p);
-    unsigned* keysIn = reinterpret_cast<unsigned*>(p + kBoxBytes);
+    unsigned* keysIn = reinterpret_cast<unsigned*>(p + kFrontBytes);
     unsigned* keysOut = keysIn + n;
     unsigned* idxIn = keysOut + n;
-    void* temp = p + kBoxBytes + 3 * sizeof(unsigned) * (size_t)n;
-    size_t tempBytes = scratchBytes - (kBoxBytes + 3 * sizeof(unsigned) * (size_t)n);
+    void* temp = p + kFrontBytes + 3 * sizeof(unsigned) * (size_t)n;
+    size_t tempBytes = scratchBytes - (kFrontBytes + 3 * sizeof(unsigned) * (size_t)n);
     hipLaunchKernelGGL(k_pose_bbox, dim3(kBoxBlocks), dim3(256), 0, s, dofs, stride, n, part);
     hipLaunchKernelGGL(k_pose_keys, dim3((n + 255) / 256), dim3(256), 0, s, dofs, stride, n, part,
-                       keysIn, idxIn);
+                       keysIn, idxIn, pose_order_queues(scratch));
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     return rocprim::radix_sort_pairs(temp, tempBytes, keysIn, keysOut, idxIn, order, n, 0, 30, s);

@@ -619,7 +619,8 @@ static att_status grow(att_ctx* c, void** p, size_t* cap, size_t bytes) {
 // user; *order stays null when the order is off or n is below minPoses.  The
 // caller records scratchEv on s after its last kernel that reads the order.
 static att_status pose_order(att_ctx* c, const float* d_dofs, unsigned stride, size_t n,
-                             size_t minPoses, hipStream_t s, const unsigned** order) {
+                             size_t minPoses, hipStream_t s, const unsigned** order,
+                             unsigned** queues = nullptr) {
     *order = nullptr;
     if (!c->poseOrder || n < minPoses || n == 0) return ATT_OK;
     const size_t scratch = pose_order_scratch((unsigned)n);
@@ -629,6 +630,7 @@ static att_status pose_order(att_ctx* c, const float* d_dofs, unsigned stride, s
     ATT_HIP(c, hipStreamWaitEvent(s, c->scratchEv, 0));
     ATT_HIP(c, launch_pose_order(d_dofs, stride, (unsigned)n, c->d_ord, scratch, o, s));
     *order = o;
+    if (queues) *queues = pose_order_queues(c->d_ord);
     return ATT_OK;
 }
 
@@ -861,7 +863,8 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
             P.recPos3 = static_cast<float3*>(B.pos);
         P.recKeys = keys;
     }
-    if (blocks >= 8 && (st = pose_order(c, d_dofs, P.dofStride, n, 4 * (size_t)blocks, s, &P.order)) != ATT_OK)
+    if (blocks >= 8 && (st = pose_order(c, d_dofs, P.dofStride, n, 4 * (size_t)blocks, s, &P.order,
+                                        &P.queues)) != ATT_OK)
         return st;
     const bool scratch = pgrad || P.order;
     if (pgrad && !P.order) ATT_HIP(c, hipStreamWaitEvent(s, c->scratchEv, 0));

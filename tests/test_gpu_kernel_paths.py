@@ -169,3 +169,23 @@ def test_parameter_gradient_basis_value_not_finite(ctx, W, types):
     ctx.adjoint_dev_noalloc(hs, d_in.ptr, False, n, None, d_out.ptr, d_pg.ptr)
     ctx.sync()
     assert np.array_equal(np.isfinite(ctx.to_host(d_pg, (T * T, 3))), ok)
+
+
+@pytest.mark.parametrize("nl, mr, ml, n", [(20, 0, 0, 16391), (20, 0, 0, 33001), (400, 0, 0, 8501),
+                                           (70, 5, 3, 16385), (40, 10, 10, 12300), (390, 2, 9, 6203)])
+def test_poses_drawn_from_queues(ctx, W, nl, mr, ml, n):
+    """Calls of a few rounds of poses, no multiple of the eight ranges: every
+    pose is scored, with the bits of the input order."""
+    wl = W.make_workload("queues", 600 + nl, 120, nl, n, mr, ml, shell=(5.0, 60.0),
+                         with_lig_grid=False)
+    hs = ctx.upload_workload(wl)
+    w = np.linspace(0.5, 1.5, n).astype(np.float32)
+    got = ctx.adjoint(hs, wl.dofs, w=w)
+    again = ctx.adjoint(hs, wl.dofs, w=w)
+    ctx.set_pose_order(False)
+    try:
+        ref = ctx.adjoint(hs, wl.dofs, w=w)
+    finally:
+        ctx.set_pose_order(True)
+    assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
+    assert np.array_equal(again.view(np.uint32), ref.view(np.uint32))
