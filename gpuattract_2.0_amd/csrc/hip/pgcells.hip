@@ -224,7 +224,7 @@ __global__ __launch_bounds__(64) void k_pgrad_cells(const unsigned* __restrict__
 // / 16 holds corners 2 g and 2 g + 1, one per product), and the accumulators run
 // over every cell of the workgroup.  Bound by the instructions of the turns (a
 // step's lanes of one cell and type add one after the other, four 16-byte LDS
-// operations each) and their latency: 30 million records of 12 types 1.46 ms
+// operations each) and their latency: 80 million records of 12 types 1.46 ms
 // with 16 workgroups per CU, 1.71 with 12, 1.78 with 8; LDS float atomics in
 // their place 3.7 (a wave's takes about 400 cycles).  The contraction, 2 MT NT
 // products and one read of 64 T bytes of basis per cell, kFlight cells in
