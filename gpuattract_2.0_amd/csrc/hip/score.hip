@@ -535,6 +535,24 @@ hipError_t launch_copy(void* dst, const void* src, size_t n16, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Calls launch(order, dofs, res, counts, m) for consecutive slices of a call's n
+// poses.  A launch has fewer than 2^32 threads, and a larger one runs short
+// without an error: calls of more poses (2^23 of four waves each) are several
+// launches.
+template <class Launch>
+static void pose_slices(unsigned n, unsigned threadsPerPose, const unsigned* order, const float* dofs,
+                        unsigned dofStride, float* res, unsigned resStride, uint2* counts, Launch launch) {
+    const unsigned most = (1u << 31) / threadsPerPose;
+    for (unsigned first = 0, m; first < n; first += m) {
+        m = std::min(most, n - first);
+        if (order)  // indices into the whole call's arrays
+            launch(order + first, dofs, res, counts, m);
+        else
+            launch(order, dofs + (size_t)dofStride * first, res + (size_t)resStride * first,
+                   counts ? counts + first : nullptr, m);
+    }
+}
+
 hipError_t launch_rigid(const DProt& rec, const DProt& lig, const DGrid& inner, const DGrid& outer,
                         const DNL& nl, const DPar& par, const float* dofs, float* res, unsigned n,
                         const unsigned* order, uint2* counts, unsigned numCU, hipStream_t s) {
@@ -542,9 +560,12 @@ hipError_t launch_rigid(const DProt& rec, const DProt& lig, const DGrid& inner, 
     const unsigned slots = par.T <= kMaxTypesLDS ? par.T * par.T : 0;
     const unsigned tab = (unsigned)((sizeof(att_pair_params) * (size_t)slots + 15) & ~(size_t)15);
 #define ATT_LAUNCH_RIGID(WP, POSES)                                                              \
-    hipLaunchKernelGGL(k_rigid<WP>, dim3((n + POSES - 1) / POSES), dim3(kWave * WP * POSES),     \
-                       tab + POSES * sizeof(RigidLDS<WP>), s, rec, lig, inner, outer, nl, par,   \
-                       dofs, res, n, tab, order, counts)
+    pose_slices(n, kWave * WP, order, dofs, 6, res, 7, counts,                                    \
+                [&](const unsigned* o, const float* d, float* r, uint2* c, unsigned m) {          \
+        hipLaunchKernelGGL(k_rigid<WP>, dim3((m + POSES - 1) / POSES), dim3(kWave * WP * POSES), \
+                           tab + POSES * sizeof(RigidLDS<WP>), s, rec, lig, inner, outer, nl,    \
+                           par, d, r, m, tab, o, c);                                             \
+    })
     // Eight waves per pose while the CUs are not full (512 poses 1000/300: 40
     // us, 49 on four, 122 on one; 1024: 81, 62, 128), four while they are hardly
     // (2048: 110 on four, 142 on one; 4096: 208, 212, but 94 -> 120 for 300/80), and for
@@ -574,8 +595,11 @@ hipError_t launch_modes(const DProt& rec, const DProt& lig, const DGrid& rInner,
     const size_t lds = modes_lds_bytes(rec, lig, par, nullptr);
     const unsigned mm = rec.M > lig.M ? rec.M : lig.M;
 #define ATT_LAUNCH_MODES(MMV, WV)                                                                 \
-    hipLaunchKernelGGL((k_modes<MMV, WV>), dim3(n), dim3(64 * WV), lds, s, rec, lig, rInner, rOuter, \
-                       nl, lInner, lOuter, par, dofs, res, n, order, counts)
+    pose_slices(n, kWave * WV, order, dofs, 26, res, 27, counts,                                  \
+                [&](const unsigned* o, const float* d, float* r, uint2* c, unsigned m) {          \
+        hipLaunchKernelGGL((k_modes<MMV, WV>), dim3(m), dim3(kWave * WV), lds, s, rec, lig,       \
+                           rInner, rOuter, nl, lInner, lOuter, par, d, r, m, o, c);               \
+    })
 #define ATT_LAUNCH_MODES_W(MMV)                                                                  \
     switch (waves) {                                                                              \
     case 8: ATT_LAUNCH_MODES(MMV, 8); break;                                                      \

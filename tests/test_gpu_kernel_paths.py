@@ -189,3 +189,25 @@ def test_poses_drawn_from_queues(ctx, W, nl, mr, ml, n):
         ctx.set_pose_order(True)
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
     assert np.array_equal(again.view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("kind, width, waves, n", [("rigid", 7, 4, (1 << 24) + 4096),
+                                                   ("modes", 27, 8, (1 << 23) + 4096)])
+def test_call_of_more_poses_than_one_launch_holds(ctx, W, kind, width, waves, n):
+    """A launch has fewer than 2^32 threads: with a ligand of over 384 beads
+    and four waves per pose, fewer than 2^24 poses (and with eight, which
+    flexible calls can ask for, 2^23).  Every pose of a larger call is scored,
+    with the bits of a small call."""
+    wl = W.make_workload("many poses", 620, 30, 385, 64, 1, 1, spacing=2.0)
+    hs = ctx.upload_workload(wl)
+    dofs = wl.dofs if kind == "modes" else np.ascontiguousarray(wl.dofs[:, :6])
+    ctx.set_modes_waves(waves if kind == "modes" else 0)
+    try:
+        ref = (ctx.score_modes if kind == "modes" else ctx.score_rigid)(hs, dofs)
+        d_in, d_out = ctx.to_device(np.tile(dofs, (n // 64, 1))), ctx.dev_alloc(n * width * 4)
+        (ctx.score_modes_dev if kind == "modes" else ctx.score_rigid_dev)(hs, d_in.ptr, n, d_out.ptr)
+        ctx.sync()
+    finally:
+        ctx.set_modes_waves(0)
+    got = ctx.to_host(d_out, (n // 64, 64 * width)).view(np.uint32)
+    assert (got == ref.reshape(-1).view(np.uint32)).all()
