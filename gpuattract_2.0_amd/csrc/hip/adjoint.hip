@@ -763,14 +763,14 @@ size_t adjoint_lds_bytes(const DProt& rec, const DProt& lig, const DPar& par, bo
            (pgrad ? sizeof(float) * 3 * (size_t)par.T * par.T * (size_t)waves : 0);
 }
 
-size_t adjoint_static_lds(AdjWidth w) {
+size_t adjoint_static_lds(unsigned mm, AdjWidth w) {
     constexpr int M = ATT_MODES_MAX;
     if (w.work != w.order)
         return (w.order == 1 ? sizeof(PoseLDS<1, 4, M>) : sizeof(PoseLDS<2, 8, M>)) + 16;
     switch (w.order) {
-        case 1: return std::max(sizeof(PoseLDS<1, 1, 0>), sizeof(PoseLDS<1, 1, M>)) + 16;
-        case 2: return std::max(sizeof(PoseLDS<2, 2, 0>), sizeof(PoseLDS<2, 2, M>)) + 16;
-        default: return std::max(sizeof(PoseLDS<4, 4, 0>), sizeof(PoseLDS<4, 4, M>)) + 16;
+        case 1: return (mm == 0 ? sizeof(PoseLDS<1, 1, 0>) : sizeof(PoseLDS<1, 1, M>)) + 16;
+        case 2: return (mm == 0 ? sizeof(PoseLDS<2, 2, 0>) : sizeof(PoseLDS<2, 2, M>)) + 16;
+        default: return (mm == 0 ? sizeof(PoseLDS<4, 4, 0>) : sizeof(PoseLDS<4, 4, M>)) + 16;
     }
 }
 

@@ -54,9 +54,9 @@ size_t adjoint_lds_bytes(const DProt& rec, const DProt& lig, const DPar& par, bo
 struct AdjWidth {
     int order, work;
 };
-// Static LDS of the adjoint kernels of a width, and how many of their workgroups
-// one CU holds with `lds` bytes of dynamic LDS.
-size_t adjoint_static_lds(AdjWidth w);
+// Static LDS of the adjoint kernels of a width (mm: the pair's modes), and how
+// many of their workgroups one CU holds with `lds` bytes of dynamic LDS.
+size_t adjoint_static_lds(unsigned mm, AdjWidth w);
 unsigned adjoint_blocks_per_cu(unsigned mm, AdjWidth w, bool batch, size_t lds, int pg = 0);
 
 // How k_adjoint takes the grid part of the parameter gradient: not at all (no

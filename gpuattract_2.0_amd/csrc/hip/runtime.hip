@@ -312,11 +312,17 @@ AdjWidth adjoint_width(const att_ctx* c, const DProt& rec, const DProt& lig, con
                        unsigned mm, size_t n, bool pgrad) {
     const int order = pair_waves(lig.n);
     const AdjWidth few = mm == 0 ? AdjWidth{4, 4} : AdjWidth{order, 4 * order};
-    if (n * (size_t)few.work <= 16 * (size_t)c->numCU &&
-        adjoint_lds_bytes(rec, lig, par, pgrad, few.work, nullptr) + adjoint_static_lds(few) <=
-            c->maxLdsPerBlock)
-        return few;
-    return AdjWidth{order, order};
+    auto fits = [&](unsigned m, AdjWidth w) {
+        return adjoint_lds_bytes(rec, lig, par, pgrad, w.work, nullptr) + adjoint_static_lds(m, w) <=
+               c->maxLdsPerBlock;
+    };
+    if (n * (size_t)few.work <= 16 * (size_t)c->numCU && fits(mm, few)) return few;
+    // The super-chunk of two waves is 1 KB larger without modes than with.  A
+    // rigid call whose parameter sums leave room for the smaller one only (79
+    // types) takes one wave.
+    const AdjWidth own{order, order};
+    if (mm == 0 && order == 2 && !fits(0, own) && fits(ATT_MODES_MAX, own)) return AdjWidth{1, 1};
+    return own;
 }
 // Parameter-gradient records per call up to which the cell pass takes the
 // grid part (32 B of scratch per record, 40 with pose weights, and the sort's
@@ -812,7 +818,7 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
     const unsigned mm = modes ? std::max(rec->d.M, lig->d.M) : 0;
     const AdjWidth width = adjoint_width(c, rec->d, lig->d, p->d, mm, n, pgrad);
     const size_t dyn = adjoint_lds_bytes(rec->d, lig->d, p->d, pgrad, width.work, &slots);
-    if (dyn + adjoint_static_lds(width) > c->maxLdsPerBlock)
+    if (dyn + adjoint_static_lds(mm, width) > c->maxLdsPerBlock)
         return fail(c, ATT_ERR_UNSUPPORTED, "ligand too large for the LDS of the adjoint kernel");
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     const unsigned cols = 3 * p->d.T * p->d.T;
@@ -905,7 +911,7 @@ att_status att_score_adjoint_dev_noalloc(att_ctx* c, att_handle hr, att_handle h
     const unsigned mm = modes ? std::max(rec->d.M, lig->d.M) : 0;
     const AdjWidth width = adjoint_width(c, rec->d, lig->d, p->d, mm, n, pgrad);
     const size_t dyn = adjoint_lds_bytes(rec->d, lig->d, p->d, pgrad, width.work, &slots);
-    if (dyn + adjoint_static_lds(width) > c->maxLdsPerBlock)
+    if (dyn + adjoint_static_lds(mm, width) > c->maxLdsPerBlock)
         return fail(c, ATT_ERR_UNSUPPORTED, "pair table too large for the LDS of the adjoint kernel");
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     const size_t resident =
@@ -1408,7 +1414,7 @@ att_status batch_fill(att_ctx* c, att_batch* b, const att_batch_pair* in, unsign
         if (q.n && (!q.d_dofs || !q.d_out)) return fail(c, ATT_ERR_INVALID, "null buffer");
         unsigned slots = 0;
         const size_t dyn = adjoint_lds_bytes(rec->d, lig->d, p->d, false, 1, &slots);
-        if (dyn + adjoint_static_lds(AdjWidth{4, 4}) > c->maxLdsPerBlock)
+        if (dyn + adjoint_static_lds(0, AdjWidth{4, 4}) > c->maxLdsPerBlock)
             return fail(c, ATT_ERR_UNSUPPORTED, "ligand too large for the LDS of the adjoint kernel");
         PairDesc P{};
         P.rec = rec->d; P.lig = lig->d;
@@ -1516,7 +1522,7 @@ att_status att_batch_set_shape(att_ctx* c, att_batch* b, unsigned bucket, int wa
         return fail(c, ATT_ERR_INVALID, "waves per pose must be 1, 2 or 4 and tiles non-empty");
     ATT_HIP(c, hipSetDevice(c->device));
     att_batch::Bucket& k = b->buckets[bucket];
-    if (k.lds + adjoint_static_lds(AdjWidth{wavesPerPose, wavesPerPose}) > c->maxLdsPerBlock)
+    if (k.lds + adjoint_static_lds(k.mm, AdjWidth{wavesPerPose, wavesPerPose}) > c->maxLdsPerBlock)
         return fail(c, ATT_ERR_UNSUPPORTED, "shape does not fit the LDS");
     k.waves = wavesPerPose;
     k.ms = -1.f;
@@ -1546,7 +1552,7 @@ att_status att_batch_tune(att_ctx* c, att_batch* b, void* stream) {
         int bw = 4;
         unsigned bt = 16;
         for (int w : kWaves) {
-            if (k.lds + adjoint_static_lds(AdjWidth{w, w}) > c->maxLdsPerBlock) continue;
+            if (k.lds + adjoint_static_lds(k.mm, AdjWidth{w, w}) > c->maxLdsPerBlock) continue;
             for (unsigned tl : kTiles) {
                 if ((st = att_batch_set_shape(c, b, (unsigned)i, w, tl)) != ATT_OK) break;
                 hipError_t e = batch_launch(c, b, i, s);  // warm-up
@@ -1671,7 +1677,7 @@ att_status att_minjob_create(att_ctx* c, att_handle hr, att_handle hl, att_handl
     // the single-pair adjoint's shapes: same results
     j->width[0] = AdjWidth{pair_waves(lig->d.n), pair_waves(lig->d.n)};
     j->width[1] = adjoint_width(c, rec->d, lig->d, p->d, mm, 1, false);
-    if (j->dyn + adjoint_static_lds(j->width[0]) > c->maxLdsPerBlock)
+    if (j->dyn + adjoint_static_lds(mm, j->width[0]) > c->maxLdsPerBlock)
         return fail(c, ATT_ERR_UNSUPPORTED, "ligand too large for the LDS of the adjoint kernel");
     MinRun& R = j->R;
     R.npose = (unsigned)n;

@@ -211,3 +211,18 @@ def test_call_of_more_poses_than_one_launch_holds(ctx, W, kind, width, waves, n)
         ctx.set_modes_waves(0)
     got = ctx.to_host(d_out, (n // 64, 64 * width)).view(np.uint32)
     assert (got == ref.reshape(-1).view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("nl, mr", [(390, 0), (390, 2), (300, 0)])
+def test_parameter_gradient_of_the_widest_tables(ctx, W, O, nl, mr):
+    """The parameter sums of 79 types and a ligand of two waves nearly fill a
+    workgroup's LDS: accepted with and without modes, and with one wave."""
+    wl = W.make_workload("wide table", 579 + nl, 40, nl, 6, mr, 0, num_types=79, with_basis=True,
+                         shell=(8.0, 30.0), with_lig_grid=False)
+    hs = ctx.upload_workload(wl)
+    ctx.upload_basis(hs["grid"], wl)
+    out, pg = ctx.adjoint(hs, wl.dofs, pgrad=True, T=79)
+    plain = ctx.adjoint(hs, wl.dofs)
+    assert np.array_equal(out.view(np.uint32), plain.view(np.uint32))
+    ref = O.adjoint(wl, pgrad=True)[1].reshape(-1)
+    assert np.abs(pg.reshape(-1) - ref).max() <= 1e-4 * np.abs(ref).max()
