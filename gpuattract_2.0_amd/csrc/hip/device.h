@@ -24,7 +24,8 @@ constexpr unsigned kMaxTypesLDS = 32;  // pair table staged in LDS up to 32x32 t
 // 110, 111), contiguous and 128-byte aligned — one cache line per lookup.
 // octE holds the energy channel of the same octets (8 floats, 32 bytes per
 // voxel) for the adjoint, which reads no other channel; null for grids without
-// a neighbour list (the adjoint never reads those) and where memory is short.
+// a neighbour list (the adjoint never reads those) and where their memory was
+// needed elsewhere.
 struct DGrid {
     const float4* oct;
     const float4* octE;

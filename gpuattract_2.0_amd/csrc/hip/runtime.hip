@@ -46,9 +46,21 @@ struct ProtObj : Obj {
     unsigned maxType = 0, maxMType = 0;
 };
 
+// The energy octets of a grid's two levels.  Shared with the plans whose
+// descriptors hold their pointers (batches, minimizer jobs).
+struct EnergyOctets {
+    float4* level[2] = {nullptr, nullptr};
+    ~EnergyOctets() {
+        for (float4* p : level)
+            if (p) (void)hipFree(p);
+    }
+};
+
 struct GridObj : Obj {
     GridObj() : Obj(Kind::Grid) {}
     DGrid inner{}, outer{};
+    std::shared_ptr<EnergyOctets> energy;  // or null
+    bool captured = false;  // a captured call may hold their pointers
     DBasis bin{}, bout{};
     DNL nl{};
     bool hasNL = false;
@@ -146,12 +158,38 @@ att_status fail(att_ctx* c, att_status code, const std::string& msg) {
                         std::string(#expr) + ": " + hipGetErrorString(e_));                  \
     } while (0)
 
+// Frees the energy octets of the context's grids, except those that a plan or
+// a captured call may still read; false when there were none.
+bool reclaim(att_ctx* c) {
+    std::vector<GridObj*> from;
+    for (auto& kv : c->objs)
+        if (kv.second->kind == Kind::Grid) {
+            GridObj* g = static_cast<GridObj*>(kv.second.get());
+            if (g->energy && !g->captured && g->energy.use_count() == 1) from.push_back(g);
+        }
+    if (from.empty() || hipDeviceSynchronize() != hipSuccess) return false;
+    for (GridObj* g : from) {
+        g->energy.reset();
+        g->inner.octE = g->outer.octE = nullptr;
+    }
+    return true;
+}
+
+// Device memory for a required buffer of the context.  A failure is the
+// caller's to report: it is cleared, or the next launch would report it again.
+hipError_t dev_malloc(att_ctx* c, void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && reclaim(c)) e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 template <class T>
 att_status dev_copy(att_ctx* c, Obj* o, const T* host, size_t count, T** out) {
     *out = nullptr;
     if (count == 0) return ATT_OK;
     void* p = nullptr;
-    ATT_HIP(c, hipMalloc(&p, sizeof(T) * count));
+    ATT_HIP(c, dev_malloc(c, &p, sizeof(T) * count));
     o->allocs.push_back(p);
     ATT_HIP(c, hipMemcpy(p, host, sizeof(T) * count, hipMemcpyHostToDevice));
     *out = static_cast<T*>(p);
@@ -171,16 +209,10 @@ att_handle store(att_ctx* c, std::unique_ptr<Obj> o) {
     return h;
 }
 
-// Both levels of a grid have energy octets, or neither.
-void pair_octets(float4** inner, float4** outer) {
-    if (!*inner || !*outer) *inner = *outer = nullptr;
-}
-
 // Grid constants as IntrplGrid's constructor computes them (float arithmetic).
-DGrid make_dgrid(const att_grid_desc& g, const float4* oct, const float4* octE) {
+DGrid make_dgrid(const att_grid_desc& g, const float4* oct) {
     DGrid d{};
     d.oct = oct;
-    d.octE = octE;
     d.nx = g.nx; d.ny = g.ny; d.nz = g.nz;
     d.nxy = g.nx * g.ny;
     d.nvox = g.nx * g.ny * g.nz;
@@ -197,47 +229,69 @@ DGrid make_dgrid(const att_grid_desc& g, const float4* oct, const float4* octE) 
 }
 
 // Expands a device-resident point grid into voxel octets (owned by o) on the
-// context's stream; *octE (the energy octets) stays null unless `energy`, and
-// where memory is too short for them.
+// context's stream.
 att_status expand_octets(att_ctx* c, Obj* o, const att_grid_desc& g, const float4* d_points,
-                         bool energy, float4** out, float4** octE) {
+                         float4** out) {
     const size_t cells = (size_t)(g.nx - 1) * (g.ny - 1) * (g.nz - 1) * g.numGrids;
     void* oct = nullptr;
-    void* e = nullptr;
-    ATT_HIP(c, hipMalloc(&oct, sizeof(float4) * 8 * cells));
+    ATT_HIP(c, dev_malloc(c, &oct, sizeof(float4) * 8 * cells));
     o->allocs.push_back(oct);
-    if (energy && c->energyOctets) {
-        if (hipMalloc(&e, sizeof(float4) * 2 * cells) == hipSuccess) {
-            o->allocs.push_back(e);
-        } else {
-            (void)hipGetLastError();  // done without
-            e = nullptr;
-        }
-    }
-    ATT_HIP(c, launch_octets(d_points, static_cast<float4*>(oct), static_cast<float4*>(e), g.nx, g.ny,
-                             g.nz, g.numGrids, c->stream));
+    ATT_HIP(c, launch_octets(d_points, static_cast<float4*>(oct), g.nx, g.ny, g.nz, g.numGrids,
+                             c->stream));
     *out = static_cast<float4*>(oct);
-    *octE = static_cast<float4*>(e);
     return ATT_OK;
 }
 
 // Upload a [grid][z][y][x] float4 grid and expand it on the device into voxel
-// octets (8x the memory, one 128-byte line per lookup; 10x with the energy
-// octets); the compact copy is freed once expanded.
-att_status upload_octets(att_ctx* c, Obj* o, const att_grid_desc& g, bool energy, float4** out,
-                         float4** octE) {
+// octets (8x the memory, one 128-byte line per lookup); the compact copy is
+// freed once expanded.
+att_status upload_octets(att_ctx* c, Obj* o, const att_grid_desc& g, float4** out) {
     const size_t n = (size_t)g.nx * g.ny * g.nz * g.numGrids;
     void* tmp = nullptr;
-    ATT_HIP(c, hipMalloc(&tmp, sizeof(float4) * n));
+    ATT_HIP(c, dev_malloc(c, &tmp, sizeof(float4) * n));
     hipError_t e = hipMemcpy(tmp, g.data, sizeof(float4) * n, hipMemcpyHostToDevice);
     att_status st = ATT_OK;
-    if (e == hipSuccess) st = expand_octets(c, o, g, static_cast<const float4*>(tmp), energy, out, octE);
+    if (e == hipSuccess) st = expand_octets(c, o, g, static_cast<const float4*>(tmp), out);
     if (e == hipSuccess && st == ATT_OK) e = hipStreamSynchronize(c->stream);
     (void)hipFree(tmp);
     if (e != hipSuccess)
         return fail(c, e == hipErrorOutOfMemory ? ATT_ERR_NOMEM : ATT_ERR_HIP,
                     std::string("grid upload: ") + hipGetErrorString(e));
     return st;
+}
+
+// The energy octets of a grid that is complete otherwise: both levels, or
+// neither.  A quarter of the device's memory stays free after them, and the
+// context's later buffers take them back (dev_malloc), so they cost no call
+// its memory.
+att_status add_energy_octets(att_ctx* c, GridObj* o) {
+    if (!c->energyOctets) return ATT_OK;
+    DGrid* levels[2] = {&o->inner, &o->outer};
+    size_t cells[2], fr = 0, total = 0;
+    for (int k = 0; k < 2; ++k)
+        cells[k] = (size_t)(levels[k]->nx - 1) * (levels[k]->ny - 1) * (levels[k]->nz - 1) * levels[k]->ngrids;
+    const size_t bytes = sizeof(float4) * 2 * (cells[0] + cells[1]);
+    ATT_HIP(c, hipMemGetInfo(&fr, &total));
+    if (fr < bytes || fr - bytes < total / 4) return ATT_OK;
+    auto e = std::make_shared<EnergyOctets>();
+    for (int k = 0; k < 2; ++k)
+        if (hipMalloc(reinterpret_cast<void**>(&e->level[k]), sizeof(float4) * 2 * cells[k]) != hipSuccess) {
+            (void)hipGetLastError();
+            return ATT_OK;  // done without
+        }
+    for (int k = 0; k < 2; ++k)
+        ATT_HIP(c, launch_energy_octets(levels[k]->oct, e->level[k], cells[k], c->stream));
+    ATT_HIP(c, hipStreamSynchronize(c->stream));
+    o->energy = std::move(e);
+    for (int k = 0; k < 2; ++k) levels[k]->octE = o->energy->level[k];
+    return ATT_OK;
+}
+
+// Marks a grid whose pointers a captured call on stream s keeps.
+void note_capture(GridObj* g, hipStream_t s) {
+    if (!g->energy || g->captured) return;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) g->captured = true;
 }
 
 // Neighbour-list constants of a grid whose desc/list are already on the
@@ -337,6 +391,8 @@ int modes_waves(unsigned ligN) { return ligN < 384 ? 1 : 4; }
 
 // Scoped device buffers for the diagnostic entry points.
 struct Tmp {
+    explicit Tmp(att_ctx* ctx) : c(ctx) {}
+    att_ctx* c;
     std::vector<void*> p;
     ~Tmp() {
         for (void* q : p) (void)hipFree(q);
@@ -344,7 +400,7 @@ struct Tmp {
     template <class T>
     hipError_t alloc(T** out, size_t count) {
         void* q = nullptr;
-        hipError_t e = hipMalloc(&q, sizeof(T) * std::max<size_t>(count, 1));
+        hipError_t e = dev_malloc(c, &q, sizeof(T) * std::max<size_t>(count, 1));
         if (e == hipSuccess) p.push_back(q);
         *out = static_cast<T*>(q);
         return e;
@@ -530,12 +586,11 @@ att_status att_upload_grid(att_ctx* c, const att_grid_desc* inner, const att_gri
     if (inner->numGrids != outer->numGrids)
         return fail(c, ATT_ERR_INVALID, "inner and outer grids differ in the number of types");
     auto o = std::make_unique<GridObj>();
-    float4 *din, *dout, *ein, *eout;
-    if ((st = upload_octets(c, o.get(), *inner, nl != nullptr, &din, &ein)) != ATT_OK) return st;
-    if ((st = upload_octets(c, o.get(), *outer, nl != nullptr, &dout, &eout)) != ATT_OK) return st;
-    pair_octets(&ein, &eout);
-    o->inner = make_dgrid(*inner, din, ein);
-    o->outer = make_dgrid(*outer, dout, eout);
+    float4 *din, *dout;
+    if ((st = upload_octets(c, o.get(), *inner, &din)) != ATT_OK) return st;
+    if ((st = upload_octets(c, o.get(), *outer, &dout)) != ATT_OK) return st;
+    o->inner = make_dgrid(*inner, din);
+    o->outer = make_dgrid(*outer, dout);
     if (nl) {
         if (!nl->desc) return fail(c, ATT_ERR_INVALID, "neighbour grid descriptors missing");
         if (nl->nx < 1 || nl->ny < 1 || nl->nz < 1) return fail(c, ATT_ERR_INVALID, "empty neighbour grid");
@@ -562,6 +617,7 @@ att_status att_upload_grid(att_ctx* c, const att_grid_desc* inner, const att_gri
         if ((st = attach_nl(c, o.get(), nl->nx, nl->ny, nl->nz, nl->ox, nl->oy, nl->oz, nl->spacing,
                             nl->plateau, ddesc, dlist)) != ATT_OK)
             return st;
+        if ((st = add_energy_octets(c, o.get())) != ATT_OK) return st;
     }
     *out = store(c, std::move(o));
     return ATT_OK;
@@ -615,7 +671,7 @@ static att_status grow(att_ctx* c, void** p, size_t* cap, size_t bytes) {
     if (*p) ATT_HIP(c, hipFree(*p));
     *p = nullptr;
     *cap = 0;
-    ATT_HIP(c, hipMalloc(p, bytes));
+    ATT_HIP(c, dev_malloc(c, p, bytes));
     *cap = bytes;
     return ATT_OK;
 }
@@ -648,14 +704,14 @@ static att_status ensure_staging(att_ctx* c, size_t inBytes, size_t outBytes) {
         if (c->d_in) ATT_HIP(c, hipFree(c->d_in));
         c->d_in = nullptr;
         c->d_in_cap = 0;
-        ATT_HIP(c, hipMalloc(&c->d_in, inBytes));
+        ATT_HIP(c, dev_malloc(c, &c->d_in, inBytes));
         c->d_in_cap = inBytes;
     }
     if (outBytes > c->d_out_cap) {
         if (c->d_out) ATT_HIP(c, hipFree(c->d_out));
         c->d_out = nullptr;
         c->d_out_cap = 0;
-        ATT_HIP(c, hipMalloc(&c->d_out, outBytes));
+        ATT_HIP(c, dev_malloc(c, &c->d_out, outBytes));
         c->d_out_cap = outBytes;
     }
     return ATT_OK;
@@ -781,9 +837,9 @@ att_status att_upload_basis(att_ctx* c, att_handle hg, unsigned T, const float* 
         const size_t nvo = (size_t)(G.nx - 1) * (G.ny - 1) * (G.nz - 1);
         void* tmp = nullptr;
         void* oct = nullptr;
-        ATT_HIP(c, hipMalloc(&oct, sizeof(float4) * 2 * nvo * 2 * T));
+        ATT_HIP(c, dev_malloc(c, &oct, sizeof(float4) * 2 * nvo * 2 * T));
         g->allocs.push_back(oct);
-        hipError_t e = hipMalloc(&tmp, sizeof(float) * nv * 2 * T);
+        hipError_t e = dev_malloc(c, &tmp, sizeof(float) * nv * 2 * T);
         if (e == hipSuccess) e = hipMemcpy(tmp, src[k], sizeof(float) * nv * 2 * T, hipMemcpyHostToDevice);
         if (e == hipSuccess)
             e = launch_basis_octets(static_cast<const float*>(tmp), static_cast<float4*>(oct), G.nx,
@@ -852,7 +908,7 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
     }
     PairDesc P{};
     P.rec = rec->d; P.lig = lig->d;
-    P.inner = g->inner; P.outer = g->outer; P.nl = g->nl;
+    P.nl = g->nl;
     P.par = p->d;
     P.bin = g->bin; P.bout = g->bout;
     P.dofs = d_dofs; P.wts = d_w; P.out = d_out;
@@ -875,6 +931,8 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
     const bool scratch = pgrad || P.order;
     if (pgrad && !P.order) ATT_HIP(c, hipStreamWaitEvent(s, c->scratchEv, 0));
     float* rows = pgrad ? static_cast<float*>(c->d_pg) : nullptr;
+    note_capture(g, s);
+    P.inner = g->inner; P.outer = g->outer;  // after the last allocation (reclaim)
     ATT_HIP(c, launch_adjoint(P, modes != 0, rows, blocks, width, dyn, s));
     if (useRec)
         ATT_HIP(c, launch_pg_cells(P, B, records, rows + (size_t)blocks * cols, cellBlocks, s));
@@ -937,6 +995,7 @@ att_status att_score_adjoint_dev_noalloc(att_ctx* c, att_handle hr, att_handle h
     // so the scratch needs no clearing between calls.
     float* rows = static_cast<float*>(c->noallocScratch);
     double* groups = reinterpret_cast<double*>(static_cast<char*>(c->noallocScratch) + kNoAllocRowBytes);
+    note_capture(g, s);
     ATT_HIP(c, launch_adjoint(P, modes != 0, pgrad ? rows : nullptr, blocks, width, dyn, s));
     if (pgrad) ATT_HIP(c, launch_pgrad_reduce(rows, blocks, cols, groups, d_pgrad, s));
     return ATT_OK;
@@ -1003,7 +1062,7 @@ att_status att_debug_beads_rigid(att_ctx* c, att_handle hr, att_handle hl, att_h
     if ((st = resolve(c, hr, hl, hg, hp, &rec, &lig, &g, &p)) != ATT_OK) return st;
     if ((st = check_pair(c, rec, lig, g, p)) != ATT_OK) return st;
     const unsigned n = lig->d.n;
-    Tmp t;
+    Tmp t(c);
     float *ddof, *dxyz, *dpot;
     int* dcell;
     unsigned* dnp;
@@ -1041,7 +1100,7 @@ att_status att_debug_beads_modes(att_ctx* c, att_handle hr, att_handle hl, att_h
     if (rec->maxMType >= gl->inner.ngrids || rec->maxMType >= gl->outer.ngrids)
         return fail(c, ATT_ERR_INVALID, "receptor mapped type has no ligand grid");
     const unsigned n = lig->d.n, nr = rec->d.n;
-    Tmp t;
+    Tmp t(c);
     float *ddof, *dxyz, *dpot, *drpot, *drxyz, *drdefo;
     int* dcell;
     unsigned* dnp;
@@ -1071,7 +1130,7 @@ att_status att_debug_rotmats(att_ctx* c, const float* angles, size_t n, float* R
     if (n == 0) return ATT_OK;
     if (n > (1u << 30)) return fail(c, ATT_ERR_UNSUPPORTED, "too many angle triples");
     ATT_HIP(c, hipSetDevice(c->device));
-    Tmp t;
+    Tmp t(c);
     float *da, *dR;
     ATT_HIP(c, t.alloc(&da, 3 * n));
     ATT_HIP(c, t.alloc(&dR, 9 * n));
@@ -1087,7 +1146,7 @@ att_status att_debug_sincosf(att_ctx* c, const float* x, size_t n, float* sn, fl
     if (n == 0) return ATT_OK;
     if (n > (1u << 30)) return fail(c, ATT_ERR_UNSUPPORTED, "too many arguments");
     ATT_HIP(c, hipSetDevice(c->device));
-    Tmp t;
+    Tmp t(c);
     float *dx, *ds, *dc;
     ATT_HIP(c, t.alloc(&dx, n));
     ATT_HIP(c, t.alloc(&ds, n));
@@ -1105,7 +1164,7 @@ att_status att_debug_plateau_ratio(att_ctx* c, float P2, size_t n, float* ratio)
     if (n == 0) return ATT_OK;
     if (n > (1u << 30)) return fail(c, ATT_ERR_UNSUPPORTED, "too many entries");
     ATT_HIP(c, hipSetDevice(c->device));
-    Tmp t;
+    Tmp t(c);
     float* dr;
     ATT_HIP(c, t.alloc(&dr, n));
     ATT_HIP(c, launch_debug_plateau_ratio(P2, (unsigned)n, dr, c->stream));
@@ -1134,7 +1193,7 @@ att_status att_dev_alloc(att_ctx* c, size_t bytes, void** d_ptr) {
     if (!c || !d_ptr) return fail(c, ATT_ERR_INVALID, "null argument");
     *d_ptr = nullptr;
     ATT_HIP(c, hipSetDevice(c->device));
-    ATT_HIP(c, hipMalloc(d_ptr, bytes ? bytes : 1));
+    ATT_HIP(c, dev_malloc(c, d_ptr, bytes ? bytes : 1));
     return ATT_OK;
 }
 
@@ -1292,6 +1351,7 @@ struct att_batch {
         float ms = -1.f;              // time of the chosen shape when tuned
     };
     std::vector<PairDesc> pairs;
+    std::vector<std::shared_ptr<EnergyOctets>> energy;  // that the pairs read
     std::vector<double> cost;         // per pair, relative cost of one pose
     PairDesc* d_pairs = nullptr;
     std::vector<Bucket> buckets;
@@ -1365,9 +1425,9 @@ att_status batch_order(att_ctx* c, att_batch* b) {
             scratch = std::max(scratch, pose_order_scratch(P.n));
         }
     if (total == 0) return ATT_OK;
-    ATT_HIP(c, hipMalloc(&b->d_order, sizeof(unsigned) * total));
+    ATT_HIP(c, dev_malloc(c, reinterpret_cast<void**>(&b->d_order), sizeof(unsigned) * total));
     void* tmp = nullptr;
-    ATT_HIP(c, hipMalloc(&tmp, scratch));
+    ATT_HIP(c, dev_malloc(c, &tmp, scratch));
     hipError_t e = hipSuccess;
     unsigned* o = b->d_order;
     for (PairDesc& P : b->pairs)
@@ -1438,16 +1498,17 @@ att_status batch_fill(att_ctx* c, att_batch* b, const att_batch_pair* in, unsign
         k.pairs.push_back(i);
         k.lds = std::max(k.lds, dyn);
         b->pairs.push_back(P);
+        if (g->energy) b->energy.push_back(g->energy);
         b->cost.push_back((double)lig->d.n * (1.0 + 0.25 * m) + 0.05 * rec->d.n);
     }
     att_status st;
     if ((st = batch_order(c, b)) != ATT_OK) return st;
     if (npairs) {
-        ATT_HIP(c, hipMalloc(&b->d_pairs, sizeof(PairDesc) * npairs));
+        ATT_HIP(c, dev_malloc(c, reinterpret_cast<void**>(&b->d_pairs), sizeof(PairDesc) * npairs));
         ATT_HIP(c, hipMemcpy(b->d_pairs, b->pairs.data(), sizeof(PairDesc) * npairs, hipMemcpyHostToDevice));
     }
-    ATT_HIP(c, hipMalloc(&b->d_counters,
-                         sizeof(unsigned) * kBatchQueues * std::max<size_t>(b->buckets.size(), 1)));
+    ATT_HIP(c, dev_malloc(c, reinterpret_cast<void**>(&b->d_counters),
+                          sizeof(unsigned) * kBatchQueues * std::max<size_t>(b->buckets.size(), 1)));
     for (auto& k : b->buckets)
         if ((st = batch_tiles(c, b, k)) != ATT_OK) return st;
     ATT_HIP(c, hipStreamCreateWithFlags(&b->capture, hipStreamNonBlocking));
@@ -1618,6 +1679,7 @@ att_status att_batch_run(att_ctx* c, att_batch* b, void* stream) {
 struct att_minjob {
     MinRun R{};
     PairDesc P{};
+    std::shared_ptr<EnergyOctets> energy;  // that P reads
     bool modes = false;
     size_t dyn = 0;
     unsigned blocks[2] = {1, 1};      // of a round of many poses, of few
@@ -1691,7 +1753,7 @@ att_status att_minjob_create(att_ctx* c, att_handle hr, att_handle hl, att_handl
     size_t pt[6];
     minjob_layout(n, R.dim, R.ds, R.os, pt);
     j->bytes = pt[0] + pt[1] + 2 * pt[2] + pt[3] + 2 * pt[4] + pt[5];
-    ATT_HIP(c, hipMalloc(&j->mem, j->bytes));
+    ATT_HIP(c, dev_malloc(c, &j->mem, j->bytes));
     char* base = static_cast<char*>(j->mem);
     R.st = reinterpret_cast<double*>(base);
     R.sc = reinterpret_cast<VaState*>(base + pt[0]);
@@ -1710,6 +1772,7 @@ att_status att_minjob_create(att_ctx* c, att_handle hr, att_handle hl, att_handl
     PairDesc& P = j->P;
     P.rec = rec->d; P.lig = lig->d;
     P.inner = g->inner; P.outer = g->outer; P.nl = g->nl;
+    j->energy = g->energy;
     P.par = p->d;
     P.bin = g->bin; P.bout = g->bout;
     P.out = j->res;
@@ -1835,7 +1898,7 @@ att_status att_minimize(att_ctx* c, att_handle hr, att_handle hl, att_handle hg,
     ATT_HIP(c, hipSetDevice(c->device));
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     const size_t ds = modes ? 26 : 6;
-    Tmp tmp;
+    Tmp tmp(c);
     float *d_in, *d_out, *d_e, *d_eb = nullptr;
     int* d_nf = nullptr;
     ATT_HIP(c, tmp.alloc(&d_in, n * ds));
@@ -1864,6 +1927,7 @@ namespace {
 // Device copies of a body's beads and of the pair table, arranged for the
 // generator kernels (gridgen.hip).
 struct GenInputs {
+    explicit GenInputs(att_ctx* c) : tmp(c) {}
     Tmp tmp;
     GenSrc src{};
     float4* nlBeads = nullptr;
@@ -1987,7 +2051,7 @@ att_status gen_nl(att_ctx* c, const GenInputs& in, const att_grid_geom& g, float
     const double nd2 = nd * nd;
     const double cr = nd + 0.01;
     const float cullR2 = (float)(cr * cr);
-    Tmp tmp;
+    Tmp tmp(c);
     uint32_t* cnt;
     unsigned long long* scratch;
     ATT_HIP(c, tmp.alloc(&cnt, npts));
@@ -2037,10 +2101,10 @@ att_status att_generate_grid(att_ctx* c, const att_protein_desc* body, const att
     att_status st;
     if ((st = check_gen_args(c, body, table, numTypes, potShape, dielec, plateau)) != ATT_OK) return st;
     if ((st = check_geom(c, geom, numTypes + 1, "grid")) != ATT_OK) return st;
-    GenInputs in;
+    GenInputs in(c);
     if ((st = gen_prepare(c, body, table, numTypes, srcIsLigand, plateau, in)) != ATT_OK) return st;
     const size_t n4 = (size_t)geom->nx * geom->ny * geom->nz * (numTypes + 1);
-    Tmp tmp;
+    Tmp tmp(c);
     float4* d;
     ATT_HIP(c, tmp.alloc(&d, n4));
     if ((st = gen_grid(c, in, *geom, numTypes, potShape, dielec, ffelec, d)) != ATT_OK) return st;
@@ -2060,9 +2124,9 @@ att_status att_generate_nl(att_ctx* c, const att_protein_desc* body, const att_g
     if ((st = check_geom(c, geom, 1, "neighbour grid")) != ATT_OK) return st;
     if (!(neighbourdis > 0.f) || !std::isfinite(neighbourdis))
         return fail(c, ATT_ERR_INVALID, "neighbour distance must be positive");
-    GenInputs in;
+    GenInputs in(c);
     if ((st = gen_prepare(c, body, nullptr, 0, 0, 1.f, in)) != ATT_OK) return st;
-    Tmp tmp;
+    Tmp tmp(c);
     auto alloc = [&](void** p, size_t bytes) { return tmp.alloc(reinterpret_cast<char**>(p), bytes); };
     uint2* d_desc;
     uint32_t* d_list;
@@ -2091,27 +2155,26 @@ att_status att_build_grid(att_ctx* c, const att_protein_desc* body, const att_pa
     if ((st = check_geom(c, outer, numTypes + 1, "outer")) != ATT_OK) return st;
     if (neighbourdis > 0.f && !std::isfinite(neighbourdis))
         return fail(c, ATT_ERR_INVALID, "neighbour distance must be finite");
-    GenInputs in;
+    GenInputs in(c);
     if ((st = gen_prepare(c, body, table, numTypes, srcIsLigand, plateau, in)) != ATT_OK) return st;
     auto o = std::make_unique<GridObj>();
     const att_grid_geom* geoms[2] = {inner, outer};
-    float4 *oct[2], *octE[2];
+    float4* oct[2];
     for (int k = 0; k < 2; ++k) {
         const att_grid_desc gd = grid_of(*geoms[k], numTypes + 1);
-        Tmp tmp;
+        Tmp tmp(c);
         float4* d;
         ATT_HIP(c, tmp.alloc(&d, (size_t)gd.nx * gd.ny * gd.nz * gd.numGrids));
         if ((st = gen_grid(c, in, *geoms[k], numTypes, potShape, dielec, ffelec, d)) != ATT_OK) return st;
-        if ((st = expand_octets(c, o.get(), gd, d, neighbourdis > 0.f, &oct[k], &octE[k])) != ATT_OK) return st;
+        if ((st = expand_octets(c, o.get(), gd, d, &oct[k])) != ATT_OK) return st;
         ATT_HIP(c, hipStreamSynchronize(c->stream));
     }
-    pair_octets(&octE[0], &octE[1]);
-    o->inner = make_dgrid(grid_of(*inner, numTypes + 1), oct[0], octE[0]);
-    o->outer = make_dgrid(grid_of(*outer, numTypes + 1), oct[1], octE[1]);
+    o->inner = make_dgrid(grid_of(*inner, numTypes + 1), oct[0]);
+    o->outer = make_dgrid(grid_of(*outer, numTypes + 1), oct[1]);
     if (neighbourdis > 0.f) {
         Obj* owner = o.get();
         auto alloc = [&](void** p, size_t bytes) {
-            hipError_t e = hipMalloc(p, bytes);
+            hipError_t e = dev_malloc(c, p, bytes);
             if (e == hipSuccess) owner->allocs.push_back(*p);
             return e;
         };
@@ -2124,6 +2187,7 @@ att_status att_build_grid(att_ctx* c, const att_protein_desc* body, const att_pa
         if ((st = attach_nl(c, o.get(), inner->nx, inner->ny, inner->nz, inner->ox, inner->oy,
                             inner->oz, inner->spacing, plateau, d_desc, d_list)) != ATT_OK)
             return st;
+        if ((st = add_energy_octets(c, o.get())) != ATT_OK) return st;
     }
     *out = store(c, std::move(o));
     return ATT_OK;
