@@ -158,6 +158,15 @@ att_status fail(att_ctx* c, att_status code, const std::string& msg) {
                         std::string(#expr) + ": " + hipGetErrorString(e_));                  \
     } while (0)
 
+size_t energy_octet_bytes(const DGrid& g) {
+    return sizeof(float4) * 2 * (size_t)(g.nx - 1) * (g.ny - 1) * (g.nz - 1) * g.ngrids;
+}
+
+void drop_energy_octets(GridObj* g) {
+    g->energy.reset();
+    g->inner.octE = g->outer.octE = nullptr;
+}
+
 // Frees the energy octets of the context's grids, except those that a plan or
 // a captured call may still read; false when there were none.
 bool reclaim(att_ctx* c) {
@@ -168,10 +177,7 @@ bool reclaim(att_ctx* c) {
             if (g->energy && !g->captured && g->energy.use_count() == 1) from.push_back(g);
         }
     if (from.empty() || hipDeviceSynchronize() != hipSuccess) return false;
-    for (GridObj* g : from) {
-        g->energy.reset();
-        g->inner.octE = g->outer.octE = nullptr;
-    }
+    for (GridObj* g : from) drop_energy_octets(g);
     return true;
 }
 
@@ -267,20 +273,18 @@ att_status upload_octets(att_ctx* c, Obj* o, const att_grid_desc& g, float4** ou
 att_status add_energy_octets(att_ctx* c, GridObj* o) {
     if (!c->energyOctets) return ATT_OK;
     DGrid* levels[2] = {&o->inner, &o->outer};
-    size_t cells[2], fr = 0, total = 0;
-    for (int k = 0; k < 2; ++k)
-        cells[k] = (size_t)(levels[k]->nx - 1) * (levels[k]->ny - 1) * (levels[k]->nz - 1) * levels[k]->ngrids;
-    const size_t bytes = sizeof(float4) * 2 * (cells[0] + cells[1]);
+    const size_t bytes[2] = {energy_octet_bytes(o->inner), energy_octet_bytes(o->outer)};
+    size_t fr = 0, total = 0;
     ATT_HIP(c, hipMemGetInfo(&fr, &total));
-    if (fr < bytes || fr - bytes < total / 4) return ATT_OK;
+    if (fr < bytes[0] + bytes[1] || fr - bytes[0] - bytes[1] < total / 4) return ATT_OK;
     auto e = std::make_shared<EnergyOctets>();
     for (int k = 0; k < 2; ++k)
-        if (hipMalloc(reinterpret_cast<void**>(&e->level[k]), sizeof(float4) * 2 * cells[k]) != hipSuccess) {
+        if (hipMalloc(reinterpret_cast<void**>(&e->level[k]), bytes[k]) != hipSuccess) {
             (void)hipGetLastError();
             return ATT_OK;  // done without
         }
     for (int k = 0; k < 2; ++k)
-        ATT_HIP(c, launch_energy_octets(levels[k]->oct, e->level[k], cells[k], c->stream));
+        ATT_HIP(c, launch_energy_octets(levels[k]->oct, e->level[k], bytes[k] / (2 * sizeof(float4)), c->stream));
     ATT_HIP(c, hipStreamSynchronize(c->stream));
     o->energy = std::move(e);
     for (int k = 0; k < 2; ++k) levels[k]->octE = o->energy->level[k];
@@ -652,6 +656,25 @@ att_status att_release(att_ctx* c, att_handle h) {
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     c->objs.erase(it);
+    return ATT_OK;
+}
+
+size_t att_grid_energy_bytes(const att_ctx* c, att_handle h) {
+    const auto it = c ? c->objs.find(h) : decltype(c->objs.end()){};
+    if (!c || it == c->objs.end() || it->second->kind != Kind::Grid) return 0;
+    const GridObj* g = static_cast<const GridObj*>(it->second.get());
+    return g->energy ? energy_octet_bytes(g->inner) + energy_octet_bytes(g->outer) : 0;
+}
+
+att_status att_grid_drop_energy_octets(att_ctx* c, att_handle h) {
+    if (!c) return ATT_ERR_INVALID;
+    GridObj* g = lookup<GridObj>(c, h, Kind::Grid);
+    if (!g) return fail(c, ATT_ERR_HANDLE, "unknown grid handle");
+    if (!g->energy) return ATT_OK;
+    if (g->captured) return fail(c, ATT_ERR_INVALID, "a captured call reads the energy octets");
+    ATT_HIP(c, hipSetDevice(c->device));
+    ATT_HIP(c, hipDeviceSynchronize());
+    drop_energy_octets(g);
     return ATT_OK;
 }
 
@@ -1829,6 +1852,12 @@ int att_minjob_round_limit(const att_minjob* j) { return j ? j->R.ivmax + 2 : 0;
 
 void att_minjob_set_running(att_minjob* j, unsigned running) {
     if (j) j->running = running;
+}
+
+void att_minjob_drop_energy_octets(att_minjob* j) {
+    if (!j) return;
+    j->P.inner.octE = j->P.outer.octE = nullptr;
+    j->energy.reset();  // the grid's own share lasts until att_grid_drop_energy_octets
 }
 
 att_status att_minjob_running(att_ctx* c, att_minjob* j, unsigned* h_count, void* stream) {

@@ -58,8 +58,8 @@ struct Receptor {
     att_grid_geom inner{}, outer{};
     float plateau = 0.f, nd = 0.f;
     size_t bytes = 0;
-    size_t energyBytes = 0;  // of the grids' energy octets: held when memory allows
-    bool energy = false;     // and held now
+    size_t energyBytes = 0;  // of the grids' energy octets: held while memory allows
+    bool energy = false;     // and held (counted in `used`) now
     att_handle hProt = 0, hGrid = 0;
     bool resident = false;
     int refs = 0;
@@ -202,6 +202,7 @@ struct att_server {
     bool admit(Job* j);
     void finish(Job* j, const std::string& error);
     void release(Job* j);
+    bool drop_energy_octets();
     bool evict_for(size_t need, const Job* j);
     bool step(Job* j);
     std::string libErr() const { return att_last_error(ctx); }
@@ -243,10 +244,36 @@ void att_server::finish(Job* j, const std::string& error) {
     cvDone.notify_all();
 }
 
-// Evicts resident receptors and ligands that no running job uses, least
-// recently used first, until `need` more bytes fit (lock held by the caller).
+// Frees the energy octets of one resident receptor, idle ones first, least
+// recently used first; false when none holds any (lock held by the caller).
+// The rounds that running jobs have issued are waited for, their later ones
+// read the full octets.
+bool att_server::drop_energy_octets() {
+    Receptor* r = nullptr;
+    uint64_t id = 0;
+    for (auto& kv : receptors) {
+        Receptor* q = kv.second.get();
+        if (!q->energy) continue;
+        if (!r || std::make_pair(q->refs > 0, q->lastUse) < std::make_pair(r->refs > 0, r->lastUse)) {
+            r = q;
+            id = kv.first;
+        }
+    }
+    if (!r) return false;
+    for (Job* j : running)
+        if (j->rec == id) att_minjob_drop_energy_octets(j->mj);
+    if (att_grid_drop_energy_octets(ctx, r->hGrid) != ATT_OK) return false;
+    r->energy = false;
+    used -= r->energyBytes;
+    return true;
+}
+
+// Makes room for `need` more bytes (lock held by the caller): first the energy
+// octets, then the resident receptors and ligands that no running job uses,
+// least recently used first.
 bool att_server::evict_for(size_t need, const Job* j) {
     while (used + need > budget) {
+        if (drop_energy_octets()) continue;
         uint64_t best = 0, stamp = ~0ull;
         int kind = -1;
         for (auto& kv : receptors)
@@ -266,7 +293,7 @@ bool att_server::evict_for(size_t need, const Job* j) {
             att_release(ctx, r.hProt);
             r.hGrid = r.hProt = 0;
             r.resident = false;
-            used -= r.bytes + (r.energy ? r.energyBytes : 0);
+            used -= r.bytes;  // its energy octets are gone by now
         } else {
             Ligand& l = *ligands[best];
             att_release(ctx, l.h);
@@ -286,6 +313,7 @@ bool att_server::admit(Job* j) {
     Receptor* r;
     Ligand* l;
     Params* p;
+    bool wantEnergy = false;
     {
         std::lock_guard<std::mutex> g(m);
         r = receptors[j->rec].get();
@@ -308,9 +336,10 @@ bool att_server::admit(Job* j) {
         }
         queue.erase(std::find(queue.begin(), queue.end(), j));
         j->admitSeq = ++admitted;
-        // The energy octets only make the scoring faster: no job waits, and
-        // nothing is evicted, for their memory.
-        if (!r->resident) r->energy = used + need + r->energyBytes <= budget;
+        // The energy octets only make the scoring faster: they are taken while
+        // there is room for them, and go first when another job needs it
+        // (evict_for), so no job waits, and nothing is evicted, for their memory.
+        wantEnergy = used + need + r->energyBytes <= budget;
         used += j->bytes;  // receptor and ligand bytes are added on upload
         r->refs++;
         l->refs++;
@@ -327,7 +356,7 @@ bool att_server::admit(Job* j) {
         const att_protein_desc pd = r->prot.desc();
         if (att_upload_protein(ctx, &pd, &r->hProt) != ATT_OK) return bad("receptor upload");
         att_status gs;
-        att_set_energy_octets(ctx, r->energy ? 1 : 0);
+        att_set_energy_octets(ctx, wantEnergy ? 1 : 0);
         if (r->fromBody) {
             gs = att_build_grid(ctx, &pd, p->table.data(), p->T, p->shape, p->dielec, p->ffelec,
                                 r->plateau, 0, &r->inner, &r->outer, r->nd, &r->hGrid);
@@ -343,6 +372,7 @@ bool att_server::admit(Job* j) {
         }
         r->resident = true;
         std::lock_guard<std::mutex> g(m);
+        r->energy = att_grid_energy_bytes(ctx, r->hGrid) > 0;
         used += r->bytes + (r->energy ? r->energyBytes : 0);
     }
     if (!l->resident) {

@@ -122,6 +122,11 @@ def lib():
         L.att_ctx_create.argtypes = [C.c_int, C.POINTER(P)]
         L.att_set_pose_order.argtypes = [P, C.c_int]
         L.att_set_energy_octets.argtypes = [P, C.c_int]
+        L.att_grid_energy_bytes.argtypes = [P, H]
+        L.att_grid_energy_bytes.restype = C.c_size_t
+        L.att_grid_drop_energy_octets.argtypes = [P, H]
+        L.att_minjob_drop_energy_octets.argtypes = [P]
+        L.att_minjob_drop_energy_octets.restype = None
         L.att_set_modes_waves.argtypes = [P, C.c_int]
         L.att_debug_pair_counts.argtypes = [P, P, C.c_size_t]
         L.att_ctx_destroy.argtypes = [P]
@@ -289,6 +294,13 @@ class Context:
     def set_energy_octets(self, enabled):
         """Energy octets for the grids uploaded or built from now on (default on)."""
         self._chk(self.L.att_set_energy_octets(self.h, 1 if enabled else 0))
+
+    def grid_energy_bytes(self, grid):
+        """Bytes of a grid's energy octets, 0 where it has none."""
+        return self.L.att_grid_energy_bytes(self.h, grid)
+
+    def drop_energy_octets(self, grid):
+        self._chk(self.L.att_grid_drop_energy_octets(self.h, grid))
 
     def pair_counts(self, fn, n):
         """Per-pose {listed neighbours walked, pairs inside the plateau} of the

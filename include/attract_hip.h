@@ -109,6 +109,12 @@ att_status att_set_pose_order(att_ctx* ctx, int enabled);
  * those of grids that a batch, a minimizer job or a captured call uses.
  * Without them the adjoint reads the full octets.  Results do not depend on it. */
 att_status att_set_energy_octets(att_ctx* ctx, int enabled);
+/* The bytes that a grid's energy octets hold now (0: none), and giving them
+ * back early.  Dropping waits for the device's work.  Batches and minimizer
+ * jobs made before keep them until they are destroyed (a job until
+ * att_minjob_drop_energy_octets); refused while a captured call may read them. */
+size_t att_grid_energy_bytes(const att_ctx* ctx, att_handle grid);
+att_status att_grid_drop_energy_octets(att_ctx* ctx, att_handle grid);
 /* Waves per pose of the flexible forward kernel (att_score_modes[_dev]):
  * 1, 2, 4 or 8, or 0 (default: 1 below 384 ligand beads, else 4).  Energy, forces,
  * torques and ligand mode gradients do not depend on it (bead-order sums);
@@ -410,6 +416,10 @@ att_status att_minjob_running(att_ctx* ctx, att_minjob* job, unsigned* h_count, 
  * att_minjob_running copied): rounds of few poses then get more waves per
  * pose.  Results do not depend on it. */
 void att_minjob_set_running(att_minjob* job, unsigned running);
+/* The job's later rounds read the full octets, with the same results; call
+ * att_grid_drop_energy_octets after it (rounds issued before still read the
+ * energy octets). */
+void att_minjob_drop_energy_octets(att_minjob* job);
 att_status att_minjob_destroy(att_ctx* ctx, att_minjob* job);
 
 /* Library build identification (arch, flags). */

@@ -10,7 +10,8 @@
  * - Receptors (protein + grids), ligands and parameter tables are registered
  *   once and uploaded on first use; receptor grids stay cached across jobs
  *   and are evicted least recently used when their memory is needed and no
- *   running job uses them.
+ *   running job uses them.  Their energy octets (att_set_energy_octets) use what
+ *   the budget has left and are given back first.
  * - A job is a set of starting poses of one receptor-ligand pair, each
  *   minimized by VA13 (at most maxFunEval line-search evaluations) on the
  *   adjoint (att_minimize semantics).  Jobs are admitted in arrival order as

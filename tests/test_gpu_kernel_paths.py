@@ -31,6 +31,19 @@ def test_energy_octets_same_bits(ctx, W, nl, mr, ml, n):
     assert np.array_equal(got.view(np.uint32), full.view(np.uint32))
 
 
+def test_energy_octets_dropped(ctx, W):
+    """32 B per cell and grid of both levels; dropped, the same bits."""
+    wl = W.make_workload("octets dropped", 310, 300, 65, 40, 2, 3, with_lig_grid=False)
+    hs = ctx.upload_workload(wl)
+    cells = sum((g.geom.nx - 1) * (g.geom.ny - 1) * (g.geom.nz - 1) for g in (wl.rec_inner, wl.rec_outer))
+    assert ctx.grid_energy_bytes(hs["grid"]) == 32 * 13 * cells
+    ref = ctx.adjoint(hs, wl.dofs)
+    ctx.drop_energy_octets(hs["grid"])
+    ctx.drop_energy_octets(hs["grid"])
+    assert ctx.grid_energy_bytes(hs["grid"]) == 0
+    assert np.array_equal(ctx.adjoint(hs, wl.dofs).view(np.uint32), ref.view(np.uint32))
+
+
 @pytest.mark.parametrize("nl, mr, ml", [(1, 0, 0), (64, 0, 0), (257, 0, 0), (384, 0, 0), (67, 0, 7),
                                         (130, 1, 0), (300, 5, 5), (383, 10, 4), (513, 4, 9),
                                         (520, 10, 10)])

@@ -185,3 +185,61 @@ def test_serve_device_built_grids(ctx, S, pairs):
         other = srv.add_params(wl.params)
         with pytest.raises(hip.AttError, match="another table"):
             srv.submit(dict(ids, params=other), wl.dofs, 10)
+
+
+def energy_bytes(wl):
+    """The energy octets of a receptor's grids: 32 B per cell and grid."""
+    cells = sum((g.geom.nx - 1) * (g.geom.ny - 1) * (g.geom.nz - 1) for g in (wl.rec_inner, wl.rec_outer))
+    return 32 * (wl.params.T + 1) * cells
+
+
+@pytest.mark.parametrize("first_runs_on", [False, True])
+def test_serve_energy_octets_give_way_to_a_job(ctx, S, W, first_runs_on):
+    """A small job brings its receptor's energy octets; a large job on the same
+    receptor then fits the budget only without them.  It is admitted as if
+    they were not there, beside the first job where that one still runs, and
+    both give the results of their poses alone."""
+    wl = W.make_workload("serve octets", 96, 200, 60, 8000, 10, 10, spacing=1.75, with_lig_grid=False)
+    octets = energy_bytes(wl)
+    jobs = [(wl.dofs[:200], 400 if first_runs_on else 5), (wl.dofs, 5)]
+    with S.Server(0) as srv:
+        ids = srv.add_workload(wl)
+        held = [srv.wait(srv.submit(ids, d, 1))[4]["bytes"] for d, _ in jobs]
+        bodies = srv.stats()["peak_bytes"] - octets - held[1]  # receptor and ligand
+    need = bodies + held[1] + (held[0] if first_runs_on else 0)
+    budget = need + octets // 4
+    assert bodies + held[0] + octets <= budget
+    hs = ctx.upload_workload(wl)
+    ref = [ctx.minimize(hs, d, e) for d, e in jobs]
+    with S.Server(0, budget) as srv:
+        ids = srv.add_workload(wl)
+        if first_runs_on:
+            got = [srv.wait(j) for j in [srv.submit(ids, d, e) for d, e in jobs]]
+            assert srv.stats()["max_running"] == 2
+        else:
+            got = [srv.wait(srv.submit(ids, d, e)) for d, e in jobs]
+        assert all(same(g, r) for g, r in zip(got, ref))
+        st = srv.stats()
+        assert st["peak_bytes"] <= budget and st["evictions"] == 0 and st["grid_hits"] == 1
+
+
+def test_serve_energy_octets_give_way_to_a_receptor(S, W):
+    """Two receptors that fit the budget together without their energy octets
+    both stay resident."""
+    wls = [W.make_workload(f"serve octets {k}", 97 + k, 200, 60, 50, spacing=1.75, with_lig_grid=False)
+           for k in range(2)]
+    octets = [energy_bytes(wl) for wl in wls]
+    with S.Server(0) as srv:
+        ids = [srv.add_workload(wl) for wl in wls]
+        held, peaks = [], []
+        for i, wl in zip(ids, wls):
+            held.append(srv.wait(srv.submit(i, wl.dofs, 3))[4]["bytes"])
+            peaks.append(srv.stats()["peak_bytes"])
+    budget = peaks[1] - sum(octets) + octets[1] // 4
+    assert peaks[0] <= budget  # the first receptor's come with it
+    with S.Server(0, budget) as srv:
+        ids = [srv.add_workload(wl) for wl in wls]
+        for k in (0, 1, 0):
+            srv.wait(srv.submit(ids[k], wls[k].dofs, 3))
+        st = srv.stats()
+        assert st["evictions"] == 0 and st["grid_hits"] == 1 and st["peak_bytes"] <= budget
