@@ -56,9 +56,11 @@ struct AdjWidth {
     int order, work;
 };
 // Static LDS of the adjoint kernels of a width (mm: the pair's modes), and how
-// many of their workgroups one CU holds with `lds` bytes of dynamic LDS.
+// many of their workgroups one CU with ldsPerCu bytes of LDS holds, `lds` of them
+// dynamic.
 size_t adjoint_static_lds(unsigned mm, AdjWidth w);
-unsigned adjoint_blocks_per_cu(unsigned mm, AdjWidth w, bool batch, size_t lds, int pg = 0);
+unsigned adjoint_blocks_per_cu(unsigned mm, AdjWidth w, bool batch, size_t lds, size_t ldsPerCu,
+                               int pg = 0);
 
 // How k_adjoint takes the grid part of the parameter gradient: not at all (no
 // parameter gradient), from the basis grids at every bead (kPgFused), or as

@@ -86,7 +86,7 @@ struct att_ctx {
     size_t d_in_cap = 0;
     void* d_out = nullptr;
     size_t d_out_cap = 0;
-    size_t maxLdsPerBlock = 65536;
+    size_t maxLdsPerBlock = 65536;  // all of a CU's
     unsigned numCU = 256;
     void* d_pg = nullptr;  // per-workgroup parameter-gradient rows of the adjoint
     size_t d_pg_cap = 0;
@@ -913,7 +913,7 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
                         sizeof(float) * cols <= c->maxLdsPerBlock;
     const int pgMode = !pgrad ? kPgNone : useRec ? kPgRecords : kPgFused;
     // persistent grid: as many workgroups as the device holds at once
-    const size_t resident = (size_t)c->numCU * adjoint_blocks_per_cu(mm, width, false, dyn, pgMode);
+    const size_t resident = (size_t)c->numCU * adjoint_blocks_per_cu(mm, width, false, dyn, c->maxLdsPerBlock, pgMode);
     const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(n, resident));
     const unsigned cellBlocks = useRec ? pg_cells_blocks(p->d.T, c->numCU) : 0;
     // per-workgroup rows (the adjoint's, then the cell pass's), then the
@@ -996,7 +996,7 @@ att_status att_score_adjoint_dev_noalloc(att_ctx* c, att_handle hr, att_handle h
         return fail(c, ATT_ERR_UNSUPPORTED, "pair table too large for the LDS of the adjoint kernel");
     hipStream_t s = stream ? (hipStream_t)stream : c->stream;
     const size_t resident =
-        (size_t)c->numCU * adjoint_blocks_per_cu(mm, width, false, dyn, pgrad ? kPgFused : kPgNone);
+        (size_t)c->numCU * adjoint_blocks_per_cu(mm, width, false, dyn, c->maxLdsPerBlock, pgrad ? kPgFused : kPgNone);
     const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(n, resident));
     if (pgrad && blocks > kNoAllocBlocks)
         return fail(c, ATT_ERR_UNSUPPORTED, "more resident workgroups than the no-allocation scratch holds");
@@ -1426,7 +1426,7 @@ att_status batch_tiles(att_ctx* c, att_batch* b, att_batch::Bucket& k) {
 hipError_t batch_launch(att_ctx* c, att_batch* b, size_t i, hipStream_t s) {
     att_batch::Bucket& k = b->buckets[i];
     const size_t resident =
-        (size_t)c->numCU * adjoint_blocks_per_cu(k.mm, AdjWidth{k.waves, k.waves}, true, k.lds);
+        (size_t)c->numCU * adjoint_blocks_per_cu(k.mm, AdjWidth{k.waves, k.waves}, true, k.lds, c->maxLdsPerBlock);
     const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(k.tiles.size(), resident));
     const unsigned* qs = reinterpret_cast<const unsigned*>(k.d_tiles + k.tiles.size());
     return launch_adjoint_batch(k.mm, AdjWidth{k.waves, k.waves}, b->d_pairs, k.d_tiles, qs, (unsigned)k.tiles.size(),
@@ -1803,7 +1803,7 @@ att_status att_minjob_create(att_ctx* c, att_handle hr, att_handle hl, att_handl
     P.n = (unsigned)n; P.tabSlots = slots;
     j->modes = modes != 0;
     for (int k = 0; k < 2; ++k) {
-        const size_t resident = (size_t)c->numCU * adjoint_blocks_per_cu(mm, j->width[k], false, j->dyn);
+        const size_t resident = (size_t)c->numCU * adjoint_blocks_per_cu(mm, j->width[k], false, j->dyn, c->maxLdsPerBlock);
         j->blocks[k] = (unsigned)std::max<size_t>(1, std::min<size_t>(n, resident));
     }
     if (j->width[1].work > j->width[0].work) j->few = 16 * c->numCU / (unsigned)j->width[1].work;
