@@ -239,3 +239,64 @@ def test_parameter_gradient_of_the_widest_tables(ctx, W, O, nl, mr):
     assert np.array_equal(out.view(np.uint32), plain.view(np.uint32))
     ref = O.adjoint(wl, pgrad=True)[1].reshape(-1)
     assert np.abs(pg.reshape(-1) - ref).max() <= 1e-4 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("types, n, places, weights", [(12, 8192, 0, True), (12, 8192, 1, False),
+                                                       (16, 8200, 3, True), (32, 8192, 0, False),
+                                                       (32, 8300, 2, True)])
+def test_parameter_gradient_cell_pass_over_many_steps(ctx, W, O, types, n, places, weights):
+    """Several steps of 64 records per workgroup, buckets that go on from one
+    to the next, and poses at a few places only (whole steps of one cell and
+    type): FP64 oracle to 1e-4 of the largest entry, the per-bead basis path
+    (16 types at most) to FP32 rounding, and the same bits in a second call."""
+    wl = W.make_workload("cell steps", 560 + types + places, 300, 130, n, 0, 0, num_types=types,
+                         with_basis=True, shell=(8.0, 45.0), type0_frac=0.05)
+    if places:
+        wl.dofs = np.ascontiguousarray(wl.dofs[np.arange(n) % places])
+    hs = ctx.upload_workload(wl)
+    ctx.upload_basis(hs["grid"], wl)
+    w = np.linspace(-1.0, 2.0, n).astype(np.float32) if weights else None
+    T = wl.params.T
+    _, pg = ctx.adjoint(hs, wl.dofs, w=w, pgrad=True, T=T)
+    _, again = ctx.adjoint(hs, wl.dofs, w=w, pgrad=True, T=T)
+    assert np.array_equal(pg.view(np.uint32), again.view(np.uint32))
+    ref = O.adjoint(wl, w=None if w is None else w.astype(np.float64), pgrad=True)[1].reshape(-1)
+    assert np.abs(pg.reshape(-1) - ref).max() <= 1e-4 * np.abs(ref).max()
+    if T > 16:
+        return
+    d_in, d_w = ctx.to_device(wl.dofs), None if w is None else ctx.to_device(w)
+    d_out, d_pg = ctx.dev_alloc(n * 7 * 4), ctx.dev_alloc(3 * T * T * 4)
+    ctx.adjoint_dev_noalloc(hs, d_in.ptr, False, n, d_w and d_w.ptr, d_out.ptr, d_pg.ptr)
+    ctx.sync()
+    beads = ctx.to_host(d_pg, (3 * T * T,))
+    assert np.abs(pg.reshape(-1) - beads).max() <= 1e-5 * np.abs(ref).max()
+
+
+def test_parameter_gradient_of_equal_poses_is_their_number_of_one(ctx, W):
+    """400,000 equal poses out of reach of the receptor's beads (the grid part
+    alone): 2000 records of one cell and type per workgroup.  A sum of at most
+    32 steps' trees (6 levels), the 8 corners and the products: 50 roundings of
+    2^-24 against one pose's gradient, times the number."""
+    n = 400000
+    wl = W.make_workload("equal poses", 590, 300, 20, 400, 0, 0, with_basis=True, shell=(8.0, 45.0))
+    hs = ctx.upload_workload(wl)
+    ctx.upload_basis(hs["grid"], wl)
+    far = wl.dofs[np.argmax(np.linalg.norm(wl.dofs[:, :3], axis=1))][None]
+    assert ctx.pair_counts(lambda: ctx.adjoint(hs, far), 1)[0, 1] == 0
+    one = ctx.adjoint(hs, far, pgrad=True, T=12)[1].astype(np.float64) * n
+    assert (one[:, 2] == 0).all() and one[:, :2].any()
+    many = ctx.adjoint(hs, np.repeat(far, n, axis=0), pgrad=True, T=12)[1].astype(np.float64)
+    assert np.all(np.abs(many - one) <= 50 * 2.0 ** -24 * np.abs(one))
+
+
+def test_parameter_gradient_buckets_of_64_cells(ctx, W, O):
+    """2.4 million cells: 64 to a bucket, with 16 types the largest LDS."""
+    wl = W.make_workload("fine grid", 701, 30, 20, 3000, 0, 0, num_types=16, with_basis=True,
+                         shell=(8.0, 20.0), outer_spacing=0.42, with_lig_grid=False)
+    g = wl.rec_outer.geom
+    assert (g.nx - 1) * (g.ny - 1) * (g.nz - 1) > 32 * 65536
+    hs = ctx.upload_workload(wl)
+    ctx.upload_basis(hs["grid"], wl)
+    pg = ctx.adjoint(hs, wl.dofs, pgrad=True, T=16)[1].reshape(-1)
+    ref = O.adjoint(wl, pgrad=True)[1].reshape(-1)
+    assert np.abs(pg - ref).max() <= 1e-4 * np.abs(ref).max()
