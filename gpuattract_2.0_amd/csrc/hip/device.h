@@ -694,7 +694,8 @@ __host__ __device__ constexpr size_t adjoint_pg_offset(unsigned tabSlots) {
 }
 
 // Key of a grid-cell record: cells (inner grid first) in buckets of 2^cellBits,
-// key = bucket << lowBits | (type - 1) << cellBits | cell in its bucket.
+// key = bucket << lowBits | (type - 1) << cellBits | cell in its bucket.  A
+// bucket is one cell (cellBits 0) for the run pass.
 struct PgKeys {
     unsigned cellsIn, cellBits, lowBits;
     unsigned invalid;  // number of buckets << lowBits: no grid term

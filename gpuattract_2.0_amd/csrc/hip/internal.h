@@ -69,10 +69,9 @@ unsigned adjoint_blocks_per_cu(unsigned mm, AdjWidth w, bool batch, size_t lds, 
 // (cell, type) after sorting (kPgRecords; PairDesc.recKey set).
 constexpr int kPgNone = 0, kPgFused = 1, kPgRecords = 2;
 
-// The keys of a call's records (false: they do not fit 32 bits).
-bool pg_keys(size_t cellsIn, size_t cellsOut, unsigned T, PgKeys* keys);
-// Tables up to this many types take the bucket pass, larger ones the run pass.
-constexpr unsigned kPgBucketTypes = 32;
+// The keys of a call's records, and with them its pass (false: they do not fit
+// 32 bits).
+bool pg_keys(size_t cellsIn, size_t cellsOut, unsigned T, size_t records, PgKeys* keys);
 
 // Scratch of the cell pass for `records` records: the adjoint's records
 // (keys, then positions) at the front, sort and reduction buffers after.
@@ -90,9 +89,9 @@ struct PgCellBufs {
     void* temp;
     size_t tempBytes;
 };
-size_t pg_cells_bytes(size_t records, const PgKeys& keys, unsigned T, bool weights);
-PgCellBufs pg_cells_layout(void* scratch, size_t records, const PgKeys& keys, unsigned T, bool weights);
-unsigned pg_cells_blocks(unsigned T, unsigned numCU);
+size_t pg_cells_bytes(size_t records, const PgKeys& keys, bool weights);
+PgCellBufs pg_cells_layout(void* scratch, size_t records, const PgKeys& keys, bool weights);
+unsigned pg_cells_blocks(size_t records, const PgKeys& keys, unsigned numCU);
 // Cell pass over the records of P's k_adjoint launch: the records sorted (by
 // bucket, or by key), the corner weights of each (cell, type) summed in a fixed
 // order and contracted with the cell's basis values by `blocks` one-wave

@@ -8,23 +8,24 @@
 // that cell.  k_adjoint writes one record per bead (key = cell and type, packed
 // by PgKeys; {x, y, z, w}, or {x, y, z} when the call has no pose weights).
 //
-// Bucket pass (up to kPgBucketTypes types): the records are sorted by bucket of
+// Bucket pass (calls of many records, pg_keys): the records are sorted by bucket of
 // cells only (stable radix sort: 16 key bits, two passes over the records
 // instead of three over 24); one wave adds a bucket's corner weights into
 // D[corner][type][cell] in LDS, then multiplies D of every touched cell,
 // [types x corners], with the cell's basis, [corners x 2 T channels], on the
 // matrix cores in FP32, accumulating over all of its cells.
 //
-// Run pass (more types, whose D and products would not fit): the records are
-// sorted by the whole key, the corner weights of each run of equal keys within
-// a group of 64 sorted records summed by a segmented scan across the wave, the
-// run sums compacted (integer scan of the per-group run counts), and each run
-// sum contracted with its cell's basis octets.
+// Run pass (few records, few types, or more types than D and the products fit):
+// the records are sorted by the whole key, the corner weights of each run of
+// equal keys within a group of 64 sorted records summed by a segmented scan
+// across the wave, the run sums compacted (integer scan of the per-group run
+// counts), and each run sum contracted with its cell's basis octets.
 //
 // Either way the basis grids are read about once per distinct cell instead of
 // once per bead, and every step has a fixed order: calls repeat their bits.
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
+#include <algorithm>
 #include <type_traits>
 
 #include "device.h"
@@ -93,14 +94,14 @@ __host__ __device__ inline size_t groups_of(size_t records) { return (records + 
 struct SortBits {
     unsigned begin, end;
 };
-SortBits sort_bits(const PgKeys& keys, unsigned T) {
+SortBits sort_bits(const PgKeys& keys) {
     unsigned end = 0;
     while (end < 32 && (keys.invalid >> end) != 0) ++end;
-    return SortBits{T <= kPgBucketTypes ? keys.lowBits : 0u, end};
+    return SortBits{keys.cellBits ? keys.lowBits : 0u, end};
 }
 
-size_t temp_bytes(size_t records, const PgKeys& keys, unsigned T, bool weights) {
-    const SortBits b = sort_bits(keys, T);
+size_t temp_bytes(size_t records, const PgKeys& keys, bool weights) {
+    const SortBits b = sort_bits(keys);
     size_t sortB = 0, scanB = 0;
     if (weights)
         (void)rocprim::radix_sort_pairs(nullptr, sortB, (unsigned*)nullptr, (unsigned*)nullptr,
@@ -110,7 +111,7 @@ size_t temp_bytes(size_t records, const PgKeys& keys, unsigned T, bool weights) 
         (void)rocprim::radix_sort_pairs(nullptr, sortB, (unsigned*)nullptr, (unsigned*)nullptr,
                                         (float3*)nullptr, (float3*)nullptr, (unsigned)records, b.begin,
                                         b.end);
-    if (T > kPgBucketTypes)
+    if (!keys.cellBits)
         (void)rocprim::exclusive_scan(nullptr, scanB, (const unsigned*)nullptr, (unsigned*)nullptr, 0u,
                                       groups_of(records), rocprim::plus<unsigned>());
     return align256(sortB > scanB ? sortB : scanB);
@@ -459,14 +460,22 @@ __global__ __launch_bounds__(64) void k_pg_buckets(const unsigned* __restrict__ 
             }
 }
 
-bool pg_keys(size_t cellsIn, size_t cellsOut, unsigned T, PgKeys* keys) {
+// The bucket pass works per cell (all types of a touched cell at once, and one
+// wave reads its basis), the run pass per cell and type that is there.  Bucket
+// pass from two records per cell and six types on, us of a call on the bucket
+// and on the run pass: 2.1-2.3 records per cell 455, 446 (8 types, 1000/300) and
+// 1023, 1011 (3000/800); 522, 547 and 1105, 1178 (12); 1172, 1328 (32, 1500/1000);
+// with 1.0-1.2 478, 434 (12) and 1719, 1494 (32); with 0.3 381, 281 (20); with 16
+// and 12 records per cell 1560, 1615 and 3214, 3356 (6 types) but 1564, 1540 and
+// 3142, 3120 (4).  Up to 32 types for the LDS of D.
+bool pg_keys(size_t cellsIn, size_t cellsOut, unsigned T, size_t records, PgKeys* keys) {
     const size_t cells = cellsIn + cellsOut;
     unsigned typeBits = 0;
     while ((1u << typeBits) < T) ++typeBits;
     // Buckets of the fewest cells, 16 or more, for which 16 key bits number them
     // (a third pass of the sort costs a third of its time); 64 at most, for the LDS.
     unsigned cellBits = 0;
-    if (T <= kPgBucketTypes) {
+    if (T >= 6 && T <= 32 && records >= 2 * cells) {
         cellBits = 4;
         while (cellBits < (T <= 16 ? 6u : 5u) && (cells >> cellBits) + 1 >= 65536) ++cellBits;
     }
@@ -477,17 +486,17 @@ bool pg_keys(size_t cellsIn, size_t cellsOut, unsigned T, PgKeys* keys) {
     return true;
 }
 
-unsigned pg_cells_blocks(unsigned T, unsigned numCU) {
-    return T <= kPgBucketTypes ? 16 * numCU : 2048;
+unsigned pg_cells_blocks(size_t records, const PgKeys& keys, unsigned numCU) {
+    return keys.cellBits ? (unsigned)std::min<size_t>(16 * numCU, groups_of(records)) : 2048;
 }
 
-size_t pg_cells_bytes(size_t records, const PgKeys& keys, unsigned T, bool weights) {
+size_t pg_cells_bytes(size_t records, const PgKeys& keys, bool weights) {
     const size_t R = records, G = groups_of(records), pb = weights ? 16 : 12;
-    const size_t runs = T <= kPgBucketTypes ? 0 : align256(4 * R) + align256(sizeof(CellW) * R) + 2 * align256(4 * G);
-    return 2 * align256(4 * R) + 2 * align256(pb * R) + runs + temp_bytes(records, keys, T, weights);
+    const size_t runs = keys.cellBits ? 0 : align256(4 * R) + align256(sizeof(CellW) * R) + 2 * align256(4 * G);
+    return 2 * align256(4 * R) + 2 * align256(pb * R) + runs + temp_bytes(records, keys, weights);
 }
 
-PgCellBufs pg_cells_layout(void* scratch, size_t records, const PgKeys& keys, unsigned T, bool weights) {
+PgCellBufs pg_cells_layout(void* scratch, size_t records, const PgKeys& keys, bool weights) {
     const size_t R = records, pb = weights ? 16 : 12;
     char* p = static_cast<char*>(scratch);
     PgCellBufs B{};
@@ -496,14 +505,14 @@ PgCellBufs pg_cells_layout(void* scratch, size_t records, const PgKeys& keys, un
     B.pos = p; p += align256(pb * R);
     B.keySorted = reinterpret_cast<unsigned*>(p); p += align256(4 * R);
     B.posSorted = p; p += align256(pb * R);
-    if (T > kPgBucketTypes) {
+    if (!keys.cellBits) {
         B.cellKey = reinterpret_cast<unsigned*>(p); p += align256(4 * R);
         B.cellW = reinterpret_cast<float*>(p); p += align256(sizeof(CellW) * R);
         B.groupRuns = reinterpret_cast<unsigned*>(p); p += align256(4 * groups_of(R));
         B.groupOffset = reinterpret_cast<unsigned*>(p); p += align256(4 * groups_of(R));
     }
     B.temp = p;
-    B.tempBytes = temp_bytes(records, keys, T, weights);
+    B.tempBytes = temp_bytes(records, keys, weights);
     return B;
 }
 
@@ -512,7 +521,7 @@ template <class Pos>
 hipError_t pg_cells(const PairDesc& P, const PgCellBufs& B, size_t records, float* rows,
                     unsigned blocks, hipStream_t s) {
     const unsigned T = P.par.T;
-    const SortBits bits = sort_bits(P.recKeys, T);
+    const SortBits bits = sort_bits(P.recKeys);
     size_t tb = B.tempBytes;
     Pos* pos = static_cast<Pos*>(B.pos);
     Pos* posSorted = static_cast<Pos*>(B.posSorted);
@@ -520,7 +529,7 @@ hipError_t pg_cells(const PairDesc& P, const PgCellBufs& B, size_t records, floa
                                              (unsigned)records, bits.begin, bits.end, s);
     if (e != hipSuccess) return e;
     const CellGeom in = cell_geom(P.inner), out = cell_geom(P.outer);
-    if (T <= kPgBucketTypes) {
+    if (P.recKeys.cellBits) {
         const size_t lds = bucket_lds(T, P.recKeys.cellBits);
         auto* kernel = T <= 16 ? k_pg_buckets<1, Pos> : k_pg_buckets<2, Pos>;
         hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64), lds, s, B.keySorted, (const Pos*)posSorted,

@@ -384,8 +384,7 @@ AdjWidth adjoint_width(const att_ctx* c, const DProt& rec, const DProt& lig, con
 }
 // Parameter-gradient records per call up to which the cell pass takes the
 // grid part (32 B of scratch per record, 40 with pose weights, and the sort's
-// own: 4-5 GB and that at the cap; 36 B more for tables of over kPgBucketTypes
-// types).
+// own: 4-5 GB and that at the cap; 36 B more for the run pass).
 constexpr size_t kPgRecordCap = (size_t)1 << 27;
 // Waves per pose of the flexible forward kernel (k_modes): with 384 ligand
 // beads or more, four (3000/800 beads, 5 + 5 modes: 100,000 poses 3% slower
@@ -909,13 +908,13 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
     const size_t cellsOut = (size_t)(g->outer.nx - 1) * (g->outer.ny - 1) * (g->outer.nz - 1);
     PgKeys keys{};
     const bool useRec = records > 0 && records <= kPgRecordCap &&
-                        pg_keys(cellsIn, cellsOut, p->d.T, &keys) &&
+                        pg_keys(cellsIn, cellsOut, p->d.T, records, &keys) &&
                         sizeof(float) * cols <= c->maxLdsPerBlock;
     const int pgMode = !pgrad ? kPgNone : useRec ? kPgRecords : kPgFused;
     // persistent grid: as many workgroups as the device holds at once
     const size_t resident = (size_t)c->numCU * adjoint_blocks_per_cu(mm, width, false, dyn, c->maxLdsPerBlock, pgMode);
     const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(n, resident));
-    const unsigned cellBlocks = useRec ? pg_cells_blocks(p->d.T, c->numCU) : 0;
+    const unsigned cellBlocks = useRec ? pg_cells_blocks(records, keys, c->numCU) : 0;
     // per-workgroup rows (the adjoint's, then the cell pass's), then the
     // reduction's group sums (8-byte aligned)
     const size_t rowBytes = (sizeof(float) * ((size_t)blocks + cellBlocks) * cols + 255) & ~(size_t)255;
@@ -923,7 +922,7 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
         return st;
     const bool recW = d_w != nullptr;
     if (useRec &&
-        (st = grow(c, &c->d_rec, &c->d_rec_cap, pg_cells_bytes(records, keys, p->d.T, recW))) != ATT_OK)
+        (st = grow(c, &c->d_rec, &c->d_rec_cap, pg_cells_bytes(records, keys, recW))) != ATT_OK)
         return st;
     if (n == 0) {
         if (pgrad) ATT_HIP(c, launch_fill_zero(d_pgrad, cols, s));
@@ -940,7 +939,7 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
     if ((st = pair_counts(c, n, &P.counts)) != ATT_OK) return st;
     PgCellBufs B{};
     if (useRec) {
-        B = pg_cells_layout(c->d_rec, records, keys, p->d.T, recW);
+        B = pg_cells_layout(c->d_rec, records, keys, recW);
         P.recKey = B.key;
         if (recW)
             P.recPos4 = static_cast<float4*>(B.pos);

@@ -290,13 +290,74 @@ def test_parameter_gradient_of_equal_poses_is_their_number_of_one(ctx, W):
 
 
 def test_parameter_gradient_buckets_of_64_cells(ctx, W, O):
-    """2.4 million cells: 64 to a bucket, with 16 types the largest LDS."""
+    """2.4 million cells: 64 to a bucket, with 16 types the largest LDS.  3000
+    poses 90 times over are two records per cell."""
     wl = W.make_workload("fine grid", 701, 30, 20, 3000, 0, 0, num_types=16, with_basis=True,
                          shell=(8.0, 20.0), outer_spacing=0.42, with_lig_grid=False)
     g = wl.rec_outer.geom
     assert (g.nx - 1) * (g.ny - 1) * (g.nz - 1) > 32 * 65536
     hs = ctx.upload_workload(wl)
     ctx.upload_basis(hs["grid"], wl)
-    pg = ctx.adjoint(hs, wl.dofs, pgrad=True, T=16)[1].reshape(-1)
-    ref = O.adjoint(wl, pgrad=True)[1].reshape(-1)
+    pg = ctx.adjoint(hs, np.tile(wl.dofs, (90, 1)), pgrad=True, T=16)[1].reshape(-1)
+    ref = 90 * O.adjoint(wl, pgrad=True)[1].reshape(-1)
     assert np.abs(pg - ref).max() <= 1e-4 * np.abs(ref).max()
+
+
+def coarse(W, name, seed, types, n, **kw):
+    """A pair on grids of some 30,000 cells: calls of a few hundred poses have
+    more than two records per cell (the bucket pass)."""
+    wl = W.make_workload(name, seed, 300, 130, n, 0, 0, num_types=types, with_basis=True, spacing=2.0,
+                         outer_spacing=6.0, with_lig_grid=False, **kw)
+    cells = sum((g.geom.nx - 1) * (g.geom.ny - 1) * (g.geom.nz - 1) for g in (wl.rec_inner, wl.rec_outer))
+    return wl, cells
+
+
+@pytest.mark.parametrize("types, weights", [(5, False), (6, True), (12, False), (16, True), (17, False),
+                                            (31, True), (32, False), (33, False)])
+@pytest.mark.parametrize("side", [-1, 0])
+def test_parameter_gradient_passes_on_either_side_of_their_line(ctx, W, O, types, weights, side):
+    """One pose under two records per cell, and the first number of poses from
+    there on, by tables around the bucket pass's limits: FP64 oracle to 1e-4 of
+    the largest entry, the per-bead basis path (16 types at most) to 1e-5."""
+    _, cells = coarse(W, "line", 800 + types, types, 1)
+    n = -(-2 * cells // 130) + side
+    wl, _ = coarse(W, "line", 800 + types, types, n, shell=(8.0, 45.0), type0_frac=0.05)
+    hs = ctx.upload_workload(wl)
+    ctx.upload_basis(hs["grid"], wl)
+    w = np.linspace(-1.0, 2.0, n).astype(np.float32) if weights else None
+    T = wl.params.T
+    pg = ctx.adjoint(hs, wl.dofs, w=w, pgrad=True, T=T)[1].reshape(-1)
+    ref = O.adjoint(wl, w=None if w is None else w.astype(np.float64), pgrad=True)[1].reshape(-1)
+    assert np.abs(pg - ref).max() <= 1e-4 * np.abs(ref).max()
+    if T > 16:
+        return
+    d_in, d_w = ctx.to_device(wl.dofs), None if w is None else ctx.to_device(w)
+    d_out, d_pg = ctx.dev_alloc(n * 7 * 4), ctx.dev_alloc(3 * T * T * 4)
+    ctx.adjoint_dev_noalloc(hs, d_in.ptr, False, n, d_w and d_w.ptr, d_out.ptr, d_pg.ptr)
+    ctx.sync()
+    beads = ctx.to_host(d_pg, (3 * T * T,))
+    assert np.abs(pg - beads).max() <= 1e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("types", [12, 20])
+def test_parameter_gradient_bucket_basis_value_not_finite(ctx, W, types):
+    """As test_parameter_gradient_basis_value_not_finite, with records enough
+    for the bucket pass: the values reach the types of the beads beside them
+    and no others."""
+    wl, cells = coarse(W, "buckets inf", 840 + types, types, 600, shell=(8.0, 30.0))
+    n, T = wl.dofs.shape[0], wl.params.T
+    assert n * 130 >= 2 * cells
+    hs = ctx.upload_workload(wl)
+    ctx.upload_basis(hs["grid"], wl)
+    clean = ctx.adjoint(hs, wl.dofs, pgrad=True, T=T)[1]
+    # receptor type 1: some points of both grids; infinite in the inner, NaN in the outer
+    nv = wl.rec_inner_basis.size // (2 * types)
+    wl.rec_inner_basis[0:nv:997] = np.inf
+    nv = wl.rec_outer_basis.size // (2 * types)
+    wl.rec_outer_basis[nv:2 * nv:499] = np.nan
+    hs = ctx.upload_workload(wl)
+    ctx.upload_basis(hs["grid"], wl)
+    pg = ctx.adjoint(hs, wl.dofs, pgrad=True, T=T)[1]
+    ok = np.isfinite(pg)
+    assert ok[T:].all() and ok[:, 2].all() and not ok[:T, :2].all()
+    assert np.abs(pg - clean)[ok].max() <= 1e-5 * np.abs(clean).max()
