@@ -361,26 +361,35 @@ namespace {
 // same bits.
 int pair_waves(unsigned ligN) { return ligN < 384 ? 1 : 2; }
 // Waves per pose of an adjoint call of n poses: pair_waves order the sums; a
-// call whose poses would leave wave slots empty (16 per CU) gets four times as
-// many to share a pose's work, with modes; without, the order decides no bit and
-// four waves do.  The same bits either way, so the line lies where the CUs are
-// full: 512 poses 3000/800 with 5 + 5 modes 184 -> 100 us, 1024 poses 1000/300
-// rigid 100 -> 47 us, but 2048 and 4096 of them 277 -> 382 and 142 -> 170 us.
+// call of at most 16 waves per CU gets four times as many to share a pose's
+// work, with modes; without, the order decides no bit and four waves do.  The
+// same bits either way, so the line is a matter of time.  While the CUs hold all
+// poses at once: 512 poses 3000/800 with 5 + 5 modes 184 -> 100 us, 1024 poses
+// 1000/300 rigid 100 -> 47 us.  Where they take two rounds (10 modes hold 12 waves per
+// CU, large tables with parameter sums fewer) and the narrow form one, still: 512
+// poses 3989/997 255 us against 321 for 513, 1024 poses 1000/300 167 against 192
+// for 1025.  Not where they take four (rigid, 32 types with parameter sums:
+// one workgroup per CU against four).  Beyond: 2048 and 4096 of the first 277 ->
+// 382 and 142 -> 170 us.
 AdjWidth adjoint_width(const att_ctx* c, const DProt& rec, const DProt& lig, const DPar& par,
-                       unsigned mm, size_t n, bool pgrad) {
+                       unsigned mm, size_t n, int pg) {
+    const bool pgrad = pg != kPgNone;
     const int order = pair_waves(lig.n);
     const AdjWidth few = mm == 0 ? AdjWidth{4, 4} : AdjWidth{order, 4 * order};
-    auto fits = [&](unsigned m, AdjWidth w) {
-        return adjoint_lds_bytes(rec, lig, par, pgrad, w.work, nullptr) + adjoint_static_lds(m, w) <=
-               c->maxLdsPerBlock;
-    };
-    if (n * (size_t)few.work <= 16 * (size_t)c->numCU && fits(mm, few)) return few;
+    AdjWidth own{order, order};
+    auto lds = [&](AdjWidth w) { return adjoint_lds_bytes(rec, lig, par, pgrad, w.work, nullptr); };
+    auto fits = [&](unsigned m, AdjWidth w) { return lds(w) + adjoint_static_lds(m, w) <= c->maxLdsPerBlock; };
     // The super-chunk of two waves is 1 KB larger without modes than with.  A
     // rigid call whose parameter sums leave room for the smaller one only (79
     // types) takes one wave.
-    const AdjWidth own{order, order};
-    if (mm == 0 && order == 2 && !fits(0, own) && fits(ATT_MODES_MAX, own)) return AdjWidth{1, 1};
-    return own;
+    if (mm == 0 && order == 2 && !fits(0, own) && fits(ATT_MODES_MAX, own)) own = AdjWidth{1, 1};
+    if (n * (size_t)few.work > 16 * (size_t)c->numCU || !fits(mm, few)) return own;
+    if (n <= c->numCU || !fits(mm, own)) return few;
+    auto rounds = [&](AdjWidth w) {
+        const size_t r = (size_t)c->numCU * adjoint_blocks_per_cu(mm, w, false, lds(w), c->maxLdsPerBlock, pg);
+        return (n + r - 1) / r;
+    };
+    return rounds(few) <= 2 * rounds(own) ? few : own;
 }
 // Parameter-gradient records per call up to which the cell pass takes the
 // grid part (32 B of scratch per record, 40 with pose weights, and the sort's
@@ -894,7 +903,7 @@ att_status att_score_adjoint_dev(att_ctx* c, att_handle hr, att_handle hl, att_h
         return fail(c, ATT_ERR_INVALID, "parameter gradients need basis grids for this table (att_upload_basis)");
     unsigned slots = 0;
     const unsigned mm = modes ? std::max(rec->d.M, lig->d.M) : 0;
-    const AdjWidth width = adjoint_width(c, rec->d, lig->d, p->d, mm, n, pgrad);
+    const AdjWidth width = adjoint_width(c, rec->d, lig->d, p->d, mm, n, pgrad ? kPgRecords : kPgNone);
     const size_t dyn = adjoint_lds_bytes(rec->d, lig->d, p->d, pgrad, width.work, &slots);
     if (dyn + adjoint_static_lds(mm, width) > c->maxLdsPerBlock)
         return fail(c, ATT_ERR_UNSUPPORTED, "ligand too large for the LDS of the adjoint kernel");
@@ -989,7 +998,7 @@ att_status att_score_adjoint_dev_noalloc(att_ctx* c, att_handle hr, att_handle h
         return fail(c, ATT_ERR_UNSUPPORTED, "parameter gradients without allocation: at most 16 pair types");
     unsigned slots = 0;
     const unsigned mm = modes ? std::max(rec->d.M, lig->d.M) : 0;
-    const AdjWidth width = adjoint_width(c, rec->d, lig->d, p->d, mm, n, pgrad);
+    const AdjWidth width = adjoint_width(c, rec->d, lig->d, p->d, mm, n, pgrad ? kPgFused : kPgNone);
     const size_t dyn = adjoint_lds_bytes(rec->d, lig->d, p->d, pgrad, width.work, &slots);
     if (dyn + adjoint_static_lds(mm, width) > c->maxLdsPerBlock)
         return fail(c, ATT_ERR_UNSUPPORTED, "pair table too large for the LDS of the adjoint kernel");
@@ -1760,7 +1769,7 @@ att_status att_minjob_create(att_ctx* c, att_handle hr, att_handle hl, att_handl
     const unsigned mm = modes ? std::max(rec->d.M, lig->d.M) : 0;
     // the single-pair adjoint's shapes: same results
     j->width[0] = AdjWidth{pair_waves(lig->d.n), pair_waves(lig->d.n)};
-    j->width[1] = adjoint_width(c, rec->d, lig->d, p->d, mm, 1, false);
+    j->width[1] = adjoint_width(c, rec->d, lig->d, p->d, mm, 1, kPgNone);
     if (j->dyn + adjoint_static_lds(mm, j->width[0]) > c->maxLdsPerBlock)
         return fail(c, ATT_ERR_UNSUPPORTED, "ligand too large for the LDS of the adjoint kernel");
     MinRun& R = j->R;
