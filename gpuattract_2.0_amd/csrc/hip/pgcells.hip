@@ -462,12 +462,13 @@ __global__ __launch_bounds__(64) void k_pg_buckets(const unsigned* __restrict__ 
 
 // The bucket pass works per cell (all types of a touched cell at once, and one
 // wave reads its basis), the run pass per cell and type that is there.  Bucket
-// pass from two records per cell and six types on, us of a call on the bucket
-// and on the run pass: 2.1-2.3 records per cell 455, 446 (8 types, 1000/300) and
-// 1023, 1011 (3000/800); 522, 547 and 1105, 1178 (12); 1172, 1328 (32, 1500/1000);
-// with 1.0-1.2 478, 434 (12) and 1719, 1494 (32); with 0.3 381, 281 (20); with 16
-// and 12 records per cell 1560, 1615 and 3214, 3356 (6 types) but 1564, 1540 and
-// 3142, 3120 (4).  Up to 32 types for the LDS of D.
+// pass from two records per cell and six types on, from 1.1 where the types fill
+// a matrix tile (10 to 16).  us of a call on the bucket and on the run pass:
+// 2.1-2.3 records per cell 455, 446 (8 types, 1000/300) and 1023, 1011 (3000/800),
+// 1172, 1328 (32, 1500/1000); 1.1-1.2 679, 712 (12) and 863, 912 (16, 3000/800) but
+// 1719, 1494 (32); 1.0 478, 434 (12, 1000/300); 0.3 381, 281 (20); 16 and 12
+// records per cell 1560, 1615 and 3214, 3356 (6 types) but 1564, 1540 and 3142,
+// 3120 (4).  Up to 32 types for the LDS of D.
 bool pg_keys(size_t cellsIn, size_t cellsOut, unsigned T, size_t records, PgKeys* keys) {
     const size_t cells = cellsIn + cellsOut;
     unsigned typeBits = 0;
@@ -475,7 +476,7 @@ bool pg_keys(size_t cellsIn, size_t cellsOut, unsigned T, size_t records, PgKeys
     // Buckets of the fewest cells, 16 or more, for which 16 key bits number them
     // (a third pass of the sort costs a third of its time); 64 at most, for the LDS.
     unsigned cellBits = 0;
-    if (T >= 6 && T <= 32 && records >= 2 * cells) {
+    if (T >= 6 && T <= 32 && records >= (T >= 10 && T <= 16 ? cells + cells / 10 : 2 * cells)) {
         cellBits = 4;
         while (cellBits < (T <= 16 ? 6u : 5u) && (cells >> cellBits) + 1 >= 65536) ++cellBits;
     }

@@ -316,11 +316,12 @@ def coarse(W, name, seed, types, n, **kw):
                                             (31, True), (32, False), (33, False)])
 @pytest.mark.parametrize("side", [-1, 0])
 def test_parameter_gradient_passes_on_either_side_of_their_line(ctx, W, O, types, weights, side):
-    """One pose under two records per cell, and the first number of poses from
-    there on, by tables around the bucket pass's limits: FP64 oracle to 1e-4 of
+    """One pose under the bucket pass's records per cell (1.1 or 2), and the first
+    number of poses from there on, by tables around its limits: FP64 oracle to 1e-4 of
     the largest entry, the per-bead basis path (16 types at most) to 1e-5."""
     _, cells = coarse(W, "line", 800 + types, types, 1)
-    n = -(-2 * cells // 130) + side
+    line = cells + cells // 10 if 10 <= types <= 16 else 2 * cells
+    n = -(-line // 130) + side
     wl, _ = coarse(W, "line", 800 + types, types, n, shell=(8.0, 45.0), type0_frac=0.05)
     hs = ctx.upload_workload(wl)
     ctx.upload_basis(hs["grid"], wl)
