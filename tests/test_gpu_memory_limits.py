@@ -14,13 +14,6 @@ MB = 1 << 20
 CHUNK = 64 * MB
 
 
-def hip_runtime():
-    """The HIP runtime that the library is bound to."""
-    with open("/proc/self/maps") as f:
-        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
-    return C.CDLL(path)
-
-
 class Card:
     """A context with one pair on it and the rest of the device's memory taken."""
 
@@ -44,7 +37,7 @@ class Card:
         """A graph of one call on a grid of its own."""
         c, n = self.ctx, self.wl.dofs.shape[0]
         hs = dict(self.hs, grid=c.build_grid(self.wl.rec, self.wl.params, *self.geoms))
-        self.rt, self.stream = hip_runtime(), C.c_void_p(c.new_stream())
+        self.rt, self.stream = c.L, C.c_void_p(c.new_stream())  # the runtime the library is bound to
         self.d_in, self.d_out = c.to_device(self.wl.dofs), c.dev_alloc(n * 28)
         graph, self.graph = C.c_void_p(), C.c_void_p()
         assert self.rt.hipStreamBeginCapture(self.stream, 2) == 0  # relaxed
