@@ -405,125 +405,6 @@ __device__ __forceinline__ float plateau_ratio_fast(unsigned n, float P2, double
     return lo == hi ? lo : plateau_ratio(n, P2);  // NaN takes the exact path too
 }
 
-// The pair loop of NLPotForce for one ligand bead (model/neighborlist.h:66-158
-// and the receptor reaction of model/neighborlist_modes.h:68-194) over the
-// list d = {numEl, idx}: every pair in list order, each term added to or
-// subtracted from the bead's accumulators in the reference's order, so the
-// bead's sums are the reference's bits.  Accessors:
-//   recPos(j)    -> float3 receptor position used for the distance
-//   recType(j)   -> receptor type
-//   recCharge(j) -> receptor charge (only read when the ligand bead is charged)
-//   reaction(j, fx, fy, fz) receives the pair's reaction force (no-op for rigid)
-// List entries are fetched NB at a time ahead of use (NB = 1 where recPos
-// itself loads much, as a receptor deformed from its mode row).
-template <int NB = 4, class RecPos, class RecType, class RecCharge, class Reaction>
-__device__ __forceinline__ float4 nl_walk(const DNL& nl, const DPar& par,
-                                          const PairTab& tab, RecPos recPos,
-                                          RecType recType, RecCharge recCharge,
-                                          Reaction reaction, float px, float py, float pz,
-                                          unsigned ligType, float ligCharge, uint2 d,
-                                          unsigned* npairs) {
-    float fx = 0.f, fy = 0.f, fz = 0.f, e = 0.f;
-    unsigned pairs = 0;
-    const unsigned lt1 = ligType - 1;
-    const bool ligCharged = ligCharge != 0.f;  // else q_lig*q_rec*ffelec = 0: no Coulomb term
-    const uint32_t* lst = nl.list + d.y;
-    // Indices of the next batch are loaded while the current batch computes.
-    unsigned nidx[NB];
-    if (d.x != 0) {
-#pragma unroll
-        for (int k = 0; k < NB; ++k) nidx[k] = lst[(unsigned)k < d.x ? k : 0];
-    }
-    for (unsigned j0 = 0; j0 < d.x; j0 += NB) {
-        unsigned idx[NB];
-        float3 rp[NB];
-        unsigned rt[NB];
-#pragma unroll
-        for (int k = 0; k < NB; ++k) idx[k] = nidx[k];
-        if (j0 + NB < d.x) {
-#pragma unroll
-            for (int k = 0; k < NB; ++k) nidx[k] = lst[j0 + NB + k < d.x ? j0 + NB + k : j0 + NB];
-        }
-#pragma unroll
-        for (int k = 0; k < NB; ++k) { rp[k] = recPos(idx[k]); rt[k] = recType(idx[k]); }
-        // Distances of the batch's pairs first, then their plateau ratios, so
-        // the table loads are in flight together.
-        float ddx[NB], ddy[NB], ddz[NB], dr2s[NB], ratios[NB];
-#pragma unroll
-        for (int k = 0; k < NB; ++k) {
-            ddx[k] = px - rp[k].x;
-            ddy[k] = py - rp[k].y;
-            ddz[k] = pz - rp[k].z;
-            dr2s[k] = ddx[k] * ddx[k] + ddy[k] * ddy[k] + ddz[k] * ddz[k];
-        }
-#pragma unroll
-        for (int k = 0; k < NB; ++k)
-            ratios[k] = (j0 + k < d.x && dr2s[k] <= nl.P2)
-                            ? plateau_ratio((unsigned)(int)(dr2s[k] * 10000.f), nl.P2)
-                            : 0.f;
-#pragma unroll
-        for (int k = 0; k < NB; ++k) {
-            if (j0 + k >= d.x) break;
-            const unsigned nIdx = idx[k];
-            float dx = ddx[k], dy = ddy[k], dz = ddz[k];
-            const float dr2 = dr2s[k];
-            if (!(dr2 <= nl.P2)) continue;  // outOfPlateau (model/NLGrid.h:133-135); NaN skipped
-            // A listed bead without a valid type would index outside the table
-            // (the reference reads out of bounds there); such pairs are skipped.
-            if (rt[k] - 1u >= par.T) continue;
-            ++pairs;
-            const float dr2_inv = (float)(1.0 / (double)dr2);
-            dx *= dr2_inv; dy *= dr2_inv; dz *= dr2_inv;
-            const att_pair_params p = tab[par.T * (rt[k] - 1) + lt1];
-            float vx, vy, vz, ve;
-            float rfx = 0.f, rfy = 0.f, rfz = 0.f;
-            lj(dr2, dr2_inv, dx, dy, dz, p, par.shape, vx, vy, vz, ve);
-            fx += vx; fy += vy; fz += vz; e += ve;
-            rfx -= vx; rfy -= vy; rfz -= vz;
-            const float ratio = ratios[k];
-            const float rdx = ratio * dx, rdy = ratio * dy, rdz = ratio * dz;
-            lj(nl.P2, nl.P2_inv, rdx, rdy, rdz, p, par.shape, vx, vy, vz, ve);
-            fx -= vx; fy -= vy; fz -= vz; e -= ve;
-            rfx += vx; rfy += vy; rfz += vz;
-            if (ligCharged) {
-                const float qlr = ligCharge * recCharge(nIdx) * par.ffelec;
-                if (fabsf(qlr) > 0.001f) {
-                    coulomb(dr2_inv, dx, dy, dz, qlr, par.dielec, vx, vy, vz, ve);
-                    fx += vx; fy += vy; fz += vz; e += ve;
-                    rfx -= vx; rfy -= vy; rfz -= vz;
-                    coulomb(nl.P2_inv, rdx, rdy, rdz, qlr, par.dielec, vx, vy, vz, ve);
-                    fx -= vx; fy -= vy; fz -= vz; e -= ve;
-                    rfx += vx; rfy += vy; rfz += vz;
-                }
-            }
-            reaction(nIdx, rfx, rfy, rfz);
-        }
-    }
-    if (npairs) *npairs = pairs;
-    return make_float4(fx, fy, fz, e);
-}
-
-// Neighbour-list term of one ligand bead: cell, then the pair loop.  Returns
-// false when the bead has no neighbour-list term.
-template <class RecPos, class RecType, class RecCharge, class Reaction>
-__device__ __forceinline__ bool nl_bead(const DNL& nl, const DPar& par,
-                                        const PairTab& tab, RecPos recPos,
-                                        RecType recType, RecCharge recCharge, Reaction reaction,
-                                        float px, float py, float pz, unsigned ligType,
-                                        float ligCharge, float4& acc, int* cell,
-                                        unsigned* npairs) {
-    acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (npairs) *npairs = 0;
-    if (ligType == 0) return false;
-    if (!((px >= nl.lox && px <= nl.hix) && (py >= nl.loy && py <= nl.hiy) &&
-          (pz >= nl.loz && pz <= nl.hiz)))
-        return false;
-    const uint2 d = nl_cell(nl, px, py, pz, ligType, cell);
-    acc = nl_walk(nl, par, tab, recPos, recType, recCharge, reaction, px, py, pz, ligType,
-                  ligCharge, d, npairs);
-    return true;
-}
-
 // Beads whose neighbour lists are walked one per quad are ordered by list
 // length, longest first, bead order inside a class, so that the quads of a
 // wave walk lists of similar length.  Nine classes (>= 64, 48, 36, 28, 22, 16,
@@ -757,23 +638,6 @@ struct NoReaction {
     __device__ void operator()(const Rec&, float, float, float) const {}
 };
 
-// Receptor accessors reading the protein arrays in global memory.
-struct RecPosG {
-    const float4* pos;
-    __device__ float3 operator()(unsigned j) const {
-        const float4 v = pos[j];
-        return make_float3(v.x, v.y, v.z);
-    }
-};
-struct RecTypeG {
-    const unsigned* type;
-    __device__ unsigned operator()(unsigned j) const { return type[j]; }
-};
-struct RecChargeG {
-    const float4* pos;
-    __device__ float operator()(unsigned j) const { return pos[j].w; }
-};
-
 // Mode vectors of bead i (modes stored [c][m][n], coalesced over beads); MM
 // is the compile-time capacity (>= the body's number of modes).
 template <int MM>
@@ -819,6 +683,7 @@ template <int MM>
 struct RecBead {
     float x, y, z, q;
     unsigned type;
+    unsigned index;  // with modes only
     float row[MM > 0 ? 4 * ((3 * MM + 4) / 4) : 1];
 
     __device__ __forceinline__ void load(const DProt& rec, unsigned j, const float* amp) {
@@ -863,16 +728,19 @@ struct RecStream {
             idx = lst[min(at + 8, last)];
         } else {
             idx = lst[min(at + 4, last)];
+            rb.index = j;
             rb.load(rec, j, amp);
         }
     }
 };
 
-// The pair loop of NLPotForce for one ligand bead as nl_walk below, by the four
+// The pair loop of NLPotForce for one ligand bead (model/neighborlist.h:66-158
+// and the receptor reaction of model/neighborlist_modes.h:68-194), by the four
 // lanes of a quad (s = lane in the quad) over the list d = {numEl, idx}
 // (numEl > 0): each step takes four consecutive list entries, one per lane, and
-// the four pairs' terms are then added in list order on every lane, so every
-// lane returns the reference's bits.  A pair outside the plateau, or past the
+// the four pairs' terms are then added to and subtracted from the bead's
+// accumulators in list order on every lane, so every lane returns the
+// reference's bits.  A pair outside the plateau, or past the
 // list's end, adds zeros (an accumulator that starts at +0 never becomes -0,
 // so that changes no bit).  reaction(rec, fx, fy, fz) receives each lane's
 // pair's reaction force (zero for those).  Bound like the adjoint's adj_walk;

@@ -34,7 +34,7 @@ hipError_t launch_debug_modes(const DProt& rec, const DProt& lig, const DGrid& r
                               const DGrid& rOuter, const DNL& nl, const DGrid& lInner,
                               const DGrid& lOuter, const DPar& par, const float* dof, float* xyz,
                               float* pot, int* cell, unsigned* npairs, float* rpot, float* rxyz,
-                              float* rdefo, hipStream_t s);
+                              hipStream_t s);
 
 hipError_t launch_debug_rotmats(const float* ang, unsigned n, float* R, hipStream_t s);
 hipError_t launch_debug_sincosf(const float* x, unsigned n, float* sn, float* cs, hipStream_t s);

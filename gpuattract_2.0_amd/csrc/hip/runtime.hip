@@ -1132,7 +1132,7 @@ att_status att_debug_beads_modes(att_ctx* c, att_handle hr, att_handle hl, att_h
         return fail(c, ATT_ERR_INVALID, "receptor mapped type has no ligand grid");
     const unsigned n = lig->d.n, nr = rec->d.n;
     Tmp t(c);
-    float *ddof, *dxyz, *dpot, *drpot, *drxyz, *drdefo;
+    float *ddof, *dxyz, *dpot, *drpot, *drxyz;
     int* dcell;
     unsigned* dnp;
     ATT_HIP(c, t.alloc(&ddof, 26));
@@ -1142,10 +1142,9 @@ att_status att_debug_beads_modes(att_ctx* c, att_handle hr, att_handle hl, att_h
     ATT_HIP(c, t.alloc(&dnp, n));
     ATT_HIP(c, t.alloc(&drpot, 3 * (size_t)nr));
     ATT_HIP(c, t.alloc(&drxyz, 3 * (size_t)nr));
-    ATT_HIP(c, t.alloc(&drdefo, 3 * (size_t)nr));
     ATT_HIP(c, hipMemcpy(ddof, dof, sizeof(att_dof6m), hipMemcpyHostToDevice));
     ATT_HIP(c, launch_debug_modes(rec->d, lig->d, gr->inner, gr->outer, gr->nl, gl->inner, gl->outer,
-                                  p->d, ddof, dxyz, dpot, dcell, dnp, drpot, drxyz, drdefo, c->stream));
+                                  p->d, ddof, dxyz, dpot, dcell, dnp, drpot, drxyz, c->stream));
     ATT_HIP(c, hipStreamSynchronize(c->stream));
     ATT_HIP(c, hipMemcpy(xyz, dxyz, sizeof(float) * 3 * n, hipMemcpyDeviceToHost));
     ATT_HIP(c, hipMemcpy(pot, dpot, sizeof(float) * 4 * n, hipMemcpyDeviceToHost));

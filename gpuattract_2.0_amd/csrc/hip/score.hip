@@ -363,42 +363,59 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(MM >= 10
 
 // ---------------------------------------------------------------- diagnostics
 
+// One wave; the beads' lists are walked as the scoring kernels walk them, one
+// bead per quad of lanes, with the pair table in LDS where theirs is.
 __global__ void k_debug_rigid(DProt rec, DProt lig, DGrid inner, DGrid outer, DNL nl, DPar par,
                               const float* dof, float* xyz, float* pot, int* cell,
                               unsigned* npairs) {
-    const int lane = threadIdx.x;
+    extern __shared__ __align__(16) att_pair_params s_tab[];
+    const PairTab tab = stage_table(par, s_tab);
+    __syncthreads();
+    const unsigned lane = threadIdx.x;
     float t[6];
     pose_trig(dof[3], dof[4], dof[5], lane, t);
     float R[9];
     rotmat_from_trig(t[0], t[1], t[2], t[3], t[4], t[5], R);
     const unsigned n = lig.n;
-    for (unsigned i = lane; i < n; i += kWave) {
+    for (unsigned i = lane >> 2; i < n; i += kWave / 4) {
         const float4 x = lig.pos[i];
         V3 p = matvec(R, x.x, x.y, x.z);
         p.x = p.x + dof[0]; p.y = p.y + dof[1]; p.z = p.z + dof[2];
-        int* c = cell + 9 * i;
+        int c[9];
         for (int k = 0; k < 9; ++k) c[k] = -1;
         float4 pp = pot_bead(inner, outer, p.x, p.y, p.z, lig.mtype[i], x.w, c);
-        float4 a;
+        const uint2 d = nl_cell(nl, p.x, p.y, p.z, lig.type[i], c + 6);
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
         unsigned np = 0;
-        if (nl_bead(nl, par, PairTab{par.tab, false}, RecPosG{rec.pos}, RecTypeG{rec.type},
-                    RecChargeG{rec.pos}, NoReaction{}, p.x, p.y, p.z, lig.type[i], x.w, a, c + 6,
-                    &np)) {
+        if (d.x)
+            a = nl_walk_quad<0>(nl, par, tab, rec, nullptr, NoReaction{}, p.x, p.y, p.z, lig.type[i],
+                                x.w, d, lane & 3u, np);
+        if (c[6] >= 0) {  // inside the lists' box
             pp.x = pp.x + a.x; pp.y = pp.y + a.y; pp.z = pp.z + a.z; pp.w = pp.w + a.w;
         }
+        np += __shfl_xor(np, 1);
+        np += __shfl_xor(np, 2);
+        if ((lane & 3u) != 0) continue;
+        for (int k = 0; k < 9; ++k) cell[9 * i + k] = c[k];
         xyz[i] = p.x; xyz[n + i] = p.y; xyz[2 * n + i] = p.z;
         pot[i] = pp.x; pot[n + i] = pp.y; pot[2 * n + i] = pp.z; pot[3 * n + i] = pp.w;
         npairs[i] = np;
     }
 }
 
-// One wave; the neighbour-list phase runs on lane 0 over the ligand beads in
+// One wave; the neighbour-list phase runs on lanes 0..3 over the ligand beads in
 // order so that receptor reaction forces accumulate in the CPU's order.
 __global__ void k_debug_modes(DProt rec, DProt lig, DGrid rInner, DGrid rOuter, DNL nl,
                               DGrid lInner, DGrid lOuter, DPar par, const float* d, float* xyz,
-                              float* pot, int* cell, unsigned* npairs, float* rpot, float* rxyz,
-                              float* rdefo) {
-    const int lane = threadIdx.x;
+                              float* pot, int* cell, unsigned* npairs, float* rpot, float* rxyz) {
+    extern __shared__ __align__(16) att_pair_params s_tab[];
+    const PairTab tab = stage_table(par, s_tab);
+    const unsigned lane = threadIdx.x;
+    float ampR[ATT_MODES_MAX], ampL[ATT_MODES_MAX];
+    for (unsigned m = 0; m < ATT_MODES_MAX; ++m) {
+        ampR[m] = m < rec.M ? d[6 + m] : 0.f;
+        ampL[m] = m < lig.M ? d[16 + m] : 0.f;
+    }
     float t[6];
     pose_trig(d[3], d[4], d[5], lane, t);
     float R[9], RT[9], Rinv[9];
@@ -414,7 +431,6 @@ __global__ void k_debug_modes(DProt rec, DProt lig, DGrid rInner, DGrid rOuter, 
         BeadModes<ATT_MODES_MAX> md;
         load_modes(rec, j, md);
         const V3 df = deform(md, rec.M, x.x, x.y, x.z, d + 6);
-        rdefo[j] = df.x; rdefo[nr + j] = df.y; rdefo[2 * nr + j] = df.z;
         V3 p = matvec(Rinv, df.x, df.y, df.z);
         p.x = p.x + pinv.x; p.y = p.y + pinv.y; p.z = p.z + pinv.z;
         rxyz[j] = p.x; rxyz[nr + j] = p.y; rxyz[2 * nr + j] = p.z;
@@ -437,18 +453,32 @@ __global__ void k_debug_modes(DProt rec, DProt lig, DGrid rInner, DGrid rOuter, 
         pot[i] = pp.x; pot[nL + i] = pp.y; pot[2 * nL + i] = pp.z; pot[3 * nL + i] = pp.w;
     }
     __syncthreads();
-    if (lane != 0) return;
-    auto recPos = [&](unsigned j) { return make_float3(rdefo[j], rdefo[nr + j], rdefo[2 * nr + j]); };
-    auto reaction = [&](unsigned j, float fx, float fy, float fz) {
+    if (lane >= 4u) return;
+    // A pair's lane adds its reaction; a list names a receptor bead once, and the
+    // next ligand bead's pairs, on any lane, come after the fence.  Pairs that do
+    // not count have none.
+    auto reaction = [&](const RecBead<ATT_MODES_MAX>& rb, float fx, float fy, float fz) {
+        if (fx == 0.f && fy == 0.f && fz == 0.f) return;
+        const unsigned j = rb.index;
         rpot[j] += fx; rpot[nr + j] += fy; rpot[2 * nr + j] += fz;
     };
     for (unsigned i = 0; i < nL; ++i) {
-        const float4 x = lig.pos[i];
-        float4 a;
+        float4 x;
+        unsigned lt;
+        const V3 p = place_from_row<ATT_MODES_MAX>(lig, i, ampL, R, d[0], d[1], d[2], x, lt);
+        int c[3] = {-1, -1, -1};
+        const uint2 list = nl_cell(nl, p.x, p.y, p.z, lt, c);
+        float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
         unsigned np = 0;
-        if (nl_bead(nl, par, PairTab{par.tab, false}, recPos, RecTypeG{rec.type},
-                    RecChargeG{rec.pos}, reaction, xyz[i], xyz[nL + i], xyz[2 * nL + i],
-                    lig.type[i], x.w, a, cell + 9 * i + 6, &np)) {
+        if (list.x)
+            a = nl_walk_quad<ATT_MODES_MAX>(nl, par, tab, rec, ampR, reaction, p.x, p.y, p.z, lt, x.w,
+                                            list, lane, np);
+        __threadfence_block();
+        np += __shfl_xor(np, 1);
+        np += __shfl_xor(np, 2);
+        if (lane != 0) continue;
+        for (int k = 0; k < 3; ++k) cell[9 * i + 6 + k] = c[k];
+        if (c[0] >= 0) {  // inside the lists' box
             pot[i] += a.x; pot[nL + i] += a.y; pot[2 * nL + i] += a.z; pot[3 * nL + i] += a.w;
         }
         npairs[i] = np;
@@ -629,8 +659,8 @@ hipError_t launch_debug_rigid(const DProt& rec, const DProt& lig, const DGrid& i
                               const DGrid& outer, const DNL& nl, const DPar& par,
                               const float* dof, float* xyz, float* pot, int* cell,
                               unsigned* npairs, hipStream_t s) {
-    hipLaunchKernelGGL(k_debug_rigid, dim3(1), dim3(kWave), 0, s, rec, lig, inner, outer, nl, par,
-                       dof, xyz, pot, cell, npairs);
+    hipLaunchKernelGGL(k_debug_rigid, dim3(1), dim3(kWave), modes_lds_bytes(rec, lig, par, nullptr), s,
+                       rec, lig, inner, outer, nl, par, dof, xyz, pot, cell, npairs);
     return hipGetLastError();
 }
 
@@ -638,9 +668,10 @@ hipError_t launch_debug_modes(const DProt& rec, const DProt& lig, const DGrid& r
                               const DGrid& rOuter, const DNL& nl, const DGrid& lInner,
                               const DGrid& lOuter, const DPar& par, const float* dof, float* xyz,
                               float* pot, int* cell, unsigned* npairs, float* rpot, float* rxyz,
-                              float* rdefo, hipStream_t s) {
-    hipLaunchKernelGGL(k_debug_modes, dim3(1), dim3(kWave), 0, s, rec, lig, rInner, rOuter, nl,
-                       lInner, lOuter, par, dof, xyz, pot, cell, npairs, rpot, rxyz, rdefo);
+                              hipStream_t s) {
+    hipLaunchKernelGGL(k_debug_modes, dim3(1), dim3(kWave), modes_lds_bytes(rec, lig, par, nullptr), s,
+                       rec, lig, rInner, rOuter, nl, lInner, lOuter, par, dof, xyz, pot, cell, npairs,
+                       rpot, rxyz);
     return hipGetLastError();
 }
 
