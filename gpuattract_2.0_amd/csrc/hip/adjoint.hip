@@ -780,11 +780,10 @@ const void* adjoint_kernel(AdjWidth w) {
     if constexpr (MM > 0)
         if (w.work != w.order)
             return w.order == 1 ? (const void*)k_adjoint<MM, 1, 4, PG> : (const void*)k_adjoint<MM, 2, 8, PG>;
-    switch (w.order) {
-        case 1: return (const void*)k_adjoint<MM, 1, 1, PG>;
-        case 2: return (const void*)k_adjoint<MM, 2, 2, PG>;
-        default: return (const void*)k_adjoint<MM, 4, 4, PG>;
-    }
+    if (w.order == 1) return (const void*)k_adjoint<MM, 1, 1, PG>;
+    if constexpr (MM == 0)  // four waves' order: rigid calls of few poses only (adjoint_width)
+        if (w.order == 4) return (const void*)k_adjoint<MM, 4, 4, PG>;
+    return (const void*)k_adjoint<MM, 2, 2, PG>;
 }
 template <int MM>
 const void* adjoint_batch_kernel(AdjWidth w) {
