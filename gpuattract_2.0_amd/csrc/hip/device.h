@@ -149,8 +149,9 @@ __device__ __forceinline__ void torque_reduce(float cSSI, float cPHI, float sSSI
 
 // A value that is the same on every lane, in a scalar register: a pose's
 // rotation, translation and amplitudes would otherwise hold some 30 vector
-// registers through the walks (the 10-mode adjoint spilled 84 B per lane with
-// them there and spills none now).
+// registers through the walks (the 10-mode adjoint without parameter gradients
+// spilled 84 B per lane with them there and spills none now; with them 28-44 B are
+// left).
 __device__ __forceinline__ float uniform(float v) {
     return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }

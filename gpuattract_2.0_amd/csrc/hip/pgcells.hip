@@ -248,10 +248,12 @@ __global__ __launch_bounds__(64) void k_pgrad_cells(const unsigned* __restrict__
 // step's lanes of one cell and type add one after the other, four 16-byte LDS
 // operations each) and their latency: 80 million records of 12 types 1.46 ms
 // with 16 workgroups per CU, 1.71 with 12, 1.78 with 8; LDS float atomics in
-// their place 3.7 (a wave's takes about 400 cycles).  The contraction, 2 MT NT
-// products and one read of 64 T bytes of basis per cell, kFlight cells in
-// flight, is 0.2 of it.  Scans and contraction of the run pass: 2.8 ms on the
-// same records, and its third sort pass 0.7.
+// their place 3.7 (a wave's takes about 400 cycles).  16 also where the LDS holds
+// fewer at a time (12 of 12 types, 7 of 20: smaller shares even the work out):
+// calls of 20,000 poses 3000/800 3.29 ms, 3.37 with 12 per CU; 20 types 4.76, 5.06
+// with 7.  The contraction, 2 MT NT products and one read of 64 T bytes of basis per
+// cell, kFlight cells in flight, is 0.2 of it.  Scans and contraction of the run
+// pass: 2.8 ms on the same records, and its third sort pass 0.7.
 template <unsigned MT, class Pos>
 __global__ __launch_bounds__(64) void k_pg_buckets(const unsigned* __restrict__ key,
                                                    const Pos* __restrict__ pos, size_t records,
