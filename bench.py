@@ -267,8 +267,9 @@ def main():
     copy_calibration(args, ctx, sh)
     # roofline numerator: the scoring path's algorithmic bytes per pose (bead
     # attributes, grid corners, neighbour-list descriptors and entries, mode
-    # vectors, DOFs in and results out); the adjoint's own reads (it skips the
-    # receptor-on-ligand-grid lookups) are reported beside it, and the
+    # vectors, DOFs in and results out); the adjoint's own reads (the energy
+    # channel of its lookups, no receptor-on-ligand-grid ones) are reported
+    # beside it, and the
     # parameter gradient's grid-cell records (16 bytes per ligand bead without
     # pose weights: key and position, written, sorted and reduced by the cell
     # pass)
@@ -703,10 +704,7 @@ def batched_leg(args, np, hip, traffic, W, check=0):
             wl.lig_inner = W.IGrid(gli, T + 1, ctx.generate_grid(wl.lig, wl.params, gli, src_is_ligand=True))
             wl.lig_outer = W.IGrid(glo, T + 1, ctx.generate_grid(wl.lig, wl.params, glo, src_is_ligand=True))
         algo += traffic.bytes_per_pose(wl, sample=64, adjoint=True)[0] * s["n"]
-        if wl.modes:
-            algo_fwd += traffic.bytes_per_pose(wl, sample=64)[0] * s["n"]
-        else:
-            algo_fwd += traffic.bytes_per_pose(wl, sample=64, adjoint=True)[0] * s["n"]
+        algo_fwd += traffic.bytes_per_pose(wl, sample=64)[0] * s["n"]
         if not args.no_server and secs is not None:
             sec = server_pass_seconds(np, hip, wl, wl.dofs, 2, reps=1)
             secs = None if sec is None else secs + sec
@@ -731,7 +729,7 @@ def batched_leg(args, np, hip, traffic, W, check=0):
         log(f"batched: drop-in Server path (2 workers, items of 100), pair after pair: {server:.4g} poses/s")
     # the scoring path's bytes per pose as for the single pair (the forward
     # formula: receptor beads on the ligand grids too); the adjoint's own
-    # reads (it builds and reads no ligand grids) reported beside them
+    # reads (the energy channel only, and no ligand grids) reported beside them
     roofline = dict(bound="hbm", achieved=algo_fwd / launch / 1e9, peak=HBM_PEAK / 1e9,
                     unit="GB/s", frac=algo_fwd / launch / HBM_PEAK, kernel="k_adjoint_batch",
                     bytes_per_pose=algo_fwd / total, adjoint_read_bytes_per_pose=algo / total,

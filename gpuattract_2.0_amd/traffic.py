@@ -1,10 +1,15 @@
-"""Algorithmic bytes per pose of the scoring path (the roofline numerator).
+"""Algorithmic bytes per pose of the scoring path.
+
+Every lookup counts in full, also where it is served from L1 or L2: bytes per
+pose times poses per second is a rate of work, which caches let exceed what
+HBM delivers, and no share of the memory's rate.
 
 Per bead touched by a pose:
     20                      bead attributes (x, y, z, type, charge)
   + 128 * (g + e)           8 float4 grid corners for the bead's type (g) and,
                             for charged beads, for the electrostatic grid (e),
-                            when the bead lies in the inner or outer grid
+                            when the bead lies in the inner or outer grid; 32
+                            where the adjoint reads their energy channel only
   + 8 * n + 4 * K           neighbour-list descriptor when the bead is in the
                             neighbour-list box, plus 4 bytes per listed neighbour
   + 12 * M                  mode vectors of the bead (flexible scoring)
@@ -53,12 +58,12 @@ def _deformed(body, amps):
     return x[None] + np.einsum("pm,nmc->pnc", amps.astype(np.float64), modes)
 
 
-def _grid_bytes(inner, outer, p, mtype, charge, basis_T=0):
+def _grid_bytes(inner, outer, p, mtype, charge, basis_T=0, lookup=128.0):
     ing = _inside(inner, p)
     inany = ing | _inside(outer, p)
     g = inany & (mtype[None, :] != 0)
     e = g & (np.abs(charge)[None, :] > 0.001)
-    return 128.0 * (g.sum(axis=1) + e.sum(axis=1)) + 64.0 * basis_T * g.sum(axis=1)
+    return lookup * (g.sum(axis=1) + e.sum(axis=1)) + 64.0 * basis_T * g.sum(axis=1)
 
 
 def _nl_bytes(nl, p, typ):
@@ -74,9 +79,9 @@ def _nl_bytes(nl, p, typ):
 
 def bytes_per_pose(wl, sample=256, seed=0, adjoint=False, pgrad=False):
     """Mean algorithmic bytes per pose over a sample of the workload's poses.
-    adjoint=True counts the adjoint's reads: the receptor beads are deformed
-    for the neighbour list but not interpolated on the ligand grid (that term
-    is not part of the energy); pgrad=True adds the basis-grid reads of the
+    adjoint=True counts the adjoint's reads: the energy channel of a lookup (the
+    energy octets), the receptor beads deformed for the neighbour list but not
+    interpolated on the ligand grid (that term is not part of the energy); pgrad=True adds the basis-grid reads of the
     pair-parameter gradient."""
     rng = np.random.default_rng(seed)
     n = wl.dofs.shape[0]
@@ -94,7 +99,7 @@ def bytes_per_pose(wl, sample=256, seed=0, adjoint=False, pgrad=False):
     pl = np.einsum("pij,pnj->pni", R, xl) + t[:, None, :]
     B = 20.0 * lig.n + 12.0 * lig.n * lig.M
     B = B + _grid_bytes(wl.rec_inner, wl.rec_outer, pl, lig.mtype, lig.charge,
-                        wl.params.T if pgrad else 0)
+                        wl.params.T if pgrad else 0, 32.0 if adjoint else 128.0)
     B = B + _nl_bytes(wl.rec_nl, pl, lig.type)
     per_pose_io = 24.0 + 28.0
     if wl.modes:
