@@ -42,10 +42,9 @@ hipError_t launch_debug_plateau_ratio(float P2, unsigned n, float* ratio, hipStr
 
 hipError_t launch_copy(void* dst, const void* src, size_t n16, hipStream_t s);
 
-hipError_t launch_octets(const float4* grid, float4* oct, unsigned nx, unsigned ny, unsigned nz,
-                         unsigned ngrids, hipStream_t s);
-// The energy octets of `cells` voxels (all grids of a level).
-hipError_t launch_energy_octets(const float4* oct, float4* octE, size_t cells, hipStream_t s);
+// octE (or null): the energy octets.
+hipError_t launch_octets(const float4* grid, float4* oct, float4* octE, unsigned nx, unsigned ny,
+                         unsigned nz, unsigned ngrids, hipStream_t s);
 
 size_t adjoint_lds_bytes(const DProt& rec, const DProt& lig, const DPar& par, bool pgrad,
                          int waves, unsigned* tabSlots);

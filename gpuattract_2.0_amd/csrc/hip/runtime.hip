@@ -100,6 +100,7 @@ struct att_ctx {
     size_t d_ord_cap = 0;
     bool poseOrder = true;
     bool energyOctets = true;
+    GridObj* building = nullptr;  // the grid of an upload or build in progress
     int modesWaves = 0;  // waves per pose of the flexible forward kernel, 0: by ligand size
     uint2* pairCounts = nullptr;  // att_debug_pair_counts: per-pose counts, capacity in poses
     size_t pairCountsCap = 0;
@@ -167,10 +168,12 @@ void drop_energy_octets(GridObj* g) {
     g->inner.octE = g->outer.octE = nullptr;
 }
 
-// Frees the energy octets of the context's grids, except those that a plan or
-// a captured call may still read; false when there were none.
+// Frees the energy octets of the context's grids (and of the one that is being
+// made), except those that a plan or a captured call may still read; false when
+// there were none.
 bool reclaim(att_ctx* c) {
     std::vector<GridObj*> from;
+    if (c->building && c->building->energy) from.push_back(c->building);
     for (auto& kv : c->objs)
         if (kv.second->kind == Kind::Grid) {
             GridObj* g = static_cast<GridObj*>(kv.second.get());
@@ -234,61 +237,69 @@ DGrid make_dgrid(const att_grid_desc& g, const float4* oct) {
     return d;
 }
 
-// Expands a device-resident point grid into voxel octets (owned by o) on the
-// context's stream.
-att_status expand_octets(att_ctx* c, Obj* o, const att_grid_desc& g, const float4* d_points,
+// A grid being made: its energy octets, where it is to have them, until they are
+// found to fit for both levels.  Required buffers take their memory back at
+// any time (dev_malloc).
+struct Building {
+    Building(att_ctx* ctx, GridObj* grid, bool energy) : c(ctx), o(grid) {
+        if (energy && c->energyOctets) o->energy = std::make_shared<EnergyOctets>();
+        c->building = o;
+    }
+    ~Building() { c->building = nullptr; }
+    // Both levels, or neither.
+    void finish() {
+        if (!o->energy) return;
+        o->inner.octE = o->energy->level[0];
+        o->outer.octE = o->energy->level[1];
+    }
+    att_ctx* c;
+    GridObj* o;
+};
+
+// Expands a device-resident point grid into voxel octets of level k (owned by
+// o) on the context's stream, and into energy octets while those of the levels
+// so far are there, fit, and leave a quarter of the device's memory free.
+att_status expand_octets(att_ctx* c, GridObj* o, int k, const att_grid_desc& g, const float4* d_points,
                          float4** out) {
     const size_t cells = (size_t)(g.nx - 1) * (g.ny - 1) * (g.nz - 1) * g.numGrids;
     void* oct = nullptr;
     ATT_HIP(c, dev_malloc(c, &oct, sizeof(float4) * 8 * cells));
     o->allocs.push_back(oct);
-    ATT_HIP(c, launch_octets(d_points, static_cast<float4*>(oct), g.nx, g.ny, g.nz, g.numGrids,
-                             c->stream));
+    if (o->energy) {
+        const size_t bytes = sizeof(float4) * 2 * cells;
+        size_t fr = 0, total = 0;
+        ATT_HIP(c, hipMemGetInfo(&fr, &total));
+        void* e = nullptr;
+        if (fr < bytes || fr - bytes < total / 4 || hipMalloc(&e, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            ATT_HIP(c, hipStreamSynchronize(c->stream));
+            o->energy.reset();  // done without
+        } else {
+            o->energy->level[k] = static_cast<float4*>(e);
+        }
+    }
+    ATT_HIP(c, launch_octets(d_points, static_cast<float4*>(oct), o->energy ? o->energy->level[k] : nullptr,
+                             g.nx, g.ny, g.nz, g.numGrids, c->stream));
     *out = static_cast<float4*>(oct);
     return ATT_OK;
 }
 
 // Upload a [grid][z][y][x] float4 grid and expand it on the device into voxel
-// octets (8x the memory, one 128-byte line per lookup); the compact copy is
-// freed once expanded.
-att_status upload_octets(att_ctx* c, Obj* o, const att_grid_desc& g, float4** out) {
+// octets (8x the memory, one 128-byte line per lookup; 10x with the energy
+// octets); the compact copy is freed once expanded.
+att_status upload_octets(att_ctx* c, GridObj* o, int k, const att_grid_desc& g, float4** out) {
     const size_t n = (size_t)g.nx * g.ny * g.nz * g.numGrids;
     void* tmp = nullptr;
     ATT_HIP(c, dev_malloc(c, &tmp, sizeof(float4) * n));
     hipError_t e = hipMemcpy(tmp, g.data, sizeof(float4) * n, hipMemcpyHostToDevice);
     att_status st = ATT_OK;
-    if (e == hipSuccess) st = expand_octets(c, o, g, static_cast<const float4*>(tmp), out);
+    if (e == hipSuccess) st = expand_octets(c, o, k, g, static_cast<const float4*>(tmp), out);
     if (e == hipSuccess && st == ATT_OK) e = hipStreamSynchronize(c->stream);
     (void)hipFree(tmp);
     if (e != hipSuccess)
         return fail(c, e == hipErrorOutOfMemory ? ATT_ERR_NOMEM : ATT_ERR_HIP,
                     std::string("grid upload: ") + hipGetErrorString(e));
     return st;
-}
-
-// The energy octets of a grid that is complete otherwise: both levels, or
-// neither.  A quarter of the device's memory stays free after them, and the
-// context's later buffers take them back (dev_malloc), so they cost no call
-// its memory.
-att_status add_energy_octets(att_ctx* c, GridObj* o) {
-    if (!c->energyOctets) return ATT_OK;
-    DGrid* levels[2] = {&o->inner, &o->outer};
-    const size_t bytes[2] = {energy_octet_bytes(o->inner), energy_octet_bytes(o->outer)};
-    size_t fr = 0, total = 0;
-    ATT_HIP(c, hipMemGetInfo(&fr, &total));
-    if (fr < bytes[0] + bytes[1] || fr - bytes[0] - bytes[1] < total / 4) return ATT_OK;
-    auto e = std::make_shared<EnergyOctets>();
-    for (int k = 0; k < 2; ++k)
-        if (hipMalloc(reinterpret_cast<void**>(&e->level[k]), bytes[k]) != hipSuccess) {
-            (void)hipGetLastError();
-            return ATT_OK;  // done without
-        }
-    for (int k = 0; k < 2; ++k)
-        ATT_HIP(c, launch_energy_octets(levels[k]->oct, e->level[k], bytes[k] / (2 * sizeof(float4)), c->stream));
-    ATT_HIP(c, hipStreamSynchronize(c->stream));
-    o->energy = std::move(e);
-    for (int k = 0; k < 2; ++k) levels[k]->octE = o->energy->level[k];
-    return ATT_OK;
 }
 
 // Marks a grid whose pointers a captured call on stream s keeps.
@@ -598,9 +609,10 @@ att_status att_upload_grid(att_ctx* c, const att_grid_desc* inner, const att_gri
     if (inner->numGrids != outer->numGrids)
         return fail(c, ATT_ERR_INVALID, "inner and outer grids differ in the number of types");
     auto o = std::make_unique<GridObj>();
+    Building making(c, o.get(), nl != nullptr);
     float4 *din, *dout;
-    if ((st = upload_octets(c, o.get(), *inner, &din)) != ATT_OK) return st;
-    if ((st = upload_octets(c, o.get(), *outer, &dout)) != ATT_OK) return st;
+    if ((st = upload_octets(c, o.get(), 0, *inner, &din)) != ATT_OK) return st;
+    if ((st = upload_octets(c, o.get(), 1, *outer, &dout)) != ATT_OK) return st;
     o->inner = make_dgrid(*inner, din);
     o->outer = make_dgrid(*outer, dout);
     if (nl) {
@@ -629,8 +641,8 @@ att_status att_upload_grid(att_ctx* c, const att_grid_desc* inner, const att_gri
         if ((st = attach_nl(c, o.get(), nl->nx, nl->ny, nl->nz, nl->ox, nl->oy, nl->oz, nl->spacing,
                             nl->plateau, ddesc, dlist)) != ATT_OK)
             return st;
-        if ((st = add_energy_octets(c, o.get())) != ATT_OK) return st;
     }
+    making.finish();
     *out = store(c, std::move(o));
     return ATT_OK;
 }
@@ -2194,6 +2206,7 @@ att_status att_build_grid(att_ctx* c, const att_protein_desc* body, const att_pa
     GenInputs in(c);
     if ((st = gen_prepare(c, body, table, numTypes, srcIsLigand, plateau, in)) != ATT_OK) return st;
     auto o = std::make_unique<GridObj>();
+    Building making(c, o.get(), neighbourdis > 0.f);
     const att_grid_geom* geoms[2] = {inner, outer};
     float4* oct[2];
     for (int k = 0; k < 2; ++k) {
@@ -2202,7 +2215,7 @@ att_status att_build_grid(att_ctx* c, const att_protein_desc* body, const att_pa
         float4* d;
         ATT_HIP(c, tmp.alloc(&d, (size_t)gd.nx * gd.ny * gd.nz * gd.numGrids));
         if ((st = gen_grid(c, in, *geoms[k], numTypes, potShape, dielec, ffelec, d)) != ATT_OK) return st;
-        if ((st = expand_octets(c, o.get(), gd, d, &oct[k])) != ATT_OK) return st;
+        if ((st = expand_octets(c, o.get(), k, gd, d, &oct[k])) != ATT_OK) return st;
         ATT_HIP(c, hipStreamSynchronize(c->stream));
     }
     o->inner = make_dgrid(grid_of(*inner, numTypes + 1), oct[0]);
@@ -2223,8 +2236,8 @@ att_status att_build_grid(att_ctx* c, const att_protein_desc* body, const att_pa
         if ((st = attach_nl(c, o.get(), inner->nx, inner->ny, inner->nz, inner->ox, inner->oy,
                             inner->oz, inner->spacing, plateau, d_desc, d_list)) != ATT_OK)
             return st;
-        if ((st = add_energy_octets(c, o.get())) != ATT_OK) return st;
     }
+    making.finish();
     *out = store(c, std::move(o));
     return ATT_OK;
 }

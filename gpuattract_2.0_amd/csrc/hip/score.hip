@@ -508,9 +508,11 @@ __global__ void k_debug_plateau_ratio(float P2, double c, unsigned n, float* rat
     if (i < n) ratio[i] = plateau_ratio_fast(i, P2, c);
 }
 
-// Expands a [grid][z][y][x] float4 grid into voxel octets (see DGrid).
+// Expands a [grid][z][y][x] float4 grid into voxel octets and, with octE, their
+// energy channel (see DGrid).
 __global__ __launch_bounds__(256) void k_octets(const float4* __restrict__ g,
-                                                float4* __restrict__ oct, unsigned nx,
+                                                float4* __restrict__ oct,
+                                                float4* __restrict__ octE, unsigned nx,
                                                 unsigned ny, unsigned nz, unsigned ngrids) {
     const size_t nvo = (size_t)(nx - 1) * (ny - 1) * (nz - 1);
     const size_t total = nvo * ngrids;
@@ -532,16 +534,11 @@ __global__ __launch_bounds__(256) void k_octets(const float4* __restrict__ g,
         d[5] = b[nxy + nx];
         d[6] = b[nx + 1];
         d[7] = b[nxy + nx + 1];
+        if (octE) {
+            octE[2 * o] = make_float4(b[0].w, b[1].w, b[nx].w, b[nxy].w);
+            octE[2 * o + 1] = make_float4(b[nxy + 1].w, b[nxy + nx].w, b[nx + 1].w, b[nxy + nx + 1].w);
+        }
     }
-}
-
-// The energy channel of the voxel octets: one value per thread.  Bound by HBM:
-// the full octets are read for a quarter of their bytes.
-__global__ __launch_bounds__(256) void k_energy_octets(const float4* __restrict__ oct,
-                                                       float* __restrict__ octE, size_t n) {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x)
-        octE[i] = oct[i].w;
 }
 
 __global__ __launch_bounds__(256) void k_copy(float4* __restrict__ dst,
@@ -553,19 +550,12 @@ __global__ __launch_bounds__(256) void k_copy(float4* __restrict__ dst,
 
 // ------------------------------------------------------------------ launchers
 
-hipError_t launch_octets(const float4* grid, float4* oct, unsigned nx, unsigned ny, unsigned nz,
-                         unsigned ngrids, hipStream_t s) {
+hipError_t launch_octets(const float4* grid, float4* oct, float4* octE, unsigned nx, unsigned ny,
+                         unsigned nz, unsigned ngrids, hipStream_t s) {
     const size_t total = (size_t)(nx - 1) * (ny - 1) * (nz - 1) * ngrids;
     const size_t blocks = std::min<size_t>((total + 255) / 256, 256 * 256);
-    hipLaunchKernelGGL(k_octets, dim3((unsigned)blocks), dim3(256), 0, s, grid, oct, nx, ny, nz,
-                       ngrids);
-    return hipGetLastError();
-}
-
-hipError_t launch_energy_octets(const float4* oct, float4* octE, size_t cells, hipStream_t s) {
-    const size_t n = 8 * cells, blocks = std::min<size_t>((n + 255) / 256, 256 * 256);
-    hipLaunchKernelGGL(k_energy_octets, dim3((unsigned)blocks), dim3(256), 0, s, oct,
-                       reinterpret_cast<float*>(octE), n);
+    hipLaunchKernelGGL(k_octets, dim3((unsigned)blocks), dim3(256), 0, s, grid, oct, octE, nx, ny,
+                       nz, ngrids);
     return hipGetLastError();
 }
 

@@ -104,8 +104,8 @@ att_status att_set_pose_order(att_ctx* ctx, int enabled);
 /* Energy octets (default on) of the grids with a neighbour list uploaded or
  * built from now on: a second copy of their energy channel (a quarter more
  * memory) that the adjoint reads 1.04 to 1.09 times as fast.  They are made
- * last, while a quarter of the device's memory stays free after them, and the
- * context frees them again when a later buffer of its own does not fit, except
+ * while a quarter of the device's memory stays free after them, and the
+ * context frees them again when another buffer of its own does not fit, except
  * those of grids that a batch, a minimizer job or a captured call uses.
  * Without them the adjoint reads the full octets.  Results do not depend on it. */
 att_status att_set_energy_octets(att_ctx* ctx, int enabled);
