@@ -408,7 +408,8 @@ __global__ __launch_bounds__(64) void k_pg_buckets(const unsigned* __restrict__ 
             // ms, 0.12 so).  A tree costs about as much as ten turns; 8 lanes as the line
             // were as fast, and 2 % slower for 4096 places.  The sum of a cell is
             // also at most a quarter as long a chain.
-            unsigned long long crowd = __ballot(mine && __popcll(same) >= kCrowd);
+            unsigned long long crowd = 0;
+            if (__ballot(mine && turn + 1u >= (unsigned)kCrowd)) crowd = __ballot(mine && __popcll(same) >= kCrowd);
             while (crowd) {  // uniform
                 const int lead = __builtin_ctzll(crowd);
                 const unsigned long long members =
